@@ -23,6 +23,8 @@ uint32_t bits_for(uint32_t max_value)
 }
 
 bool finite_f(float x) { return isfinite(x) != 0; }
+
+constexpr uint32_t kNbrWords = 64;  // neighbour-row words per particle
 }  // namespace
 
 float sqrt_threshold(float h)
@@ -343,7 +345,8 @@ int Engine::alloc(uint32_t cap, uint32_t tcap, std::string *err)
         if (!rc) rc = dm((void **)&d_.wvals[b], u4, "work order");
     }
     if (!rc) rc = dm((void **)&d_.rank, u4, "rank");
-    if (!rc) rc = dm((void **)&d_.nbr, u4 * 64, "neighbour rows");
+    if (!rc) rc = dm((void **)&d_.nbr, (u4 + sizeof(uint32_t)) * kNbrWords, "neighbour rows");  // one row spare
+    d_.nbr_words = kNbrWords;
     if (!rc) rc = dm((void **)&d_.ncnt, u4, "neighbour counts");
     if (!rc) rc = dm((void **)&d_.sflags, sizeof(uint32_t) * scene_cap_, "scene flags");
     if (!rc) rc = dm((void **)&d_.scan_err, sizeof(uint32_t), "scan error flag");
@@ -387,7 +390,7 @@ Engine::~Engine()
 
 void Engine::invalidate_graph()
 {
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kGraphs; ++i) {
         if (graph_exec_[i]) (void)hipGraphExecDestroy(graph_exec_[i]);
         if (graph_[i]) (void)hipGraphDestroy(graph_[i]);
         graph_exec_[i] = nullptr;
@@ -694,10 +697,12 @@ hipError_t Engine::enqueue_update(hipEvent_t *ev, bool rebuild_work, bool fresh,
     // fresh: the previous update did not record this one's buckets (its
     // viscosity pass does otherwise)
     hipError_t e;
+    LaunchCfg cfg = cfg_;
+    cfg.coop_n = coop_slots_now();
 #define LK(x)                              \
     if ((e = (x)) != hipSuccess) return e;
     if (ev && mark_predict) LK(hipEventRecord(ev[0], stream_));
-    if (fresh) LK(launch_predict(d_, cfg_, stream_));
+    if (fresh) LK(launch_predict(d_, cfg, stream_));
     if (ev) LK(hipEventRecord(ev[1], stream_));
     if (rebuild_work) {
         int wb = 0;
@@ -710,13 +715,13 @@ hipError_t Engine::enqueue_update(hipEvent_t *ev, bool rebuild_work, bool fresh,
         LK(launch_fused_update(d_, stream_));
         return hipSuccess;
     }
-    LK(launch_bucket_sort(d_, cfg_, stream_));
+    LK(launch_bucket_sort(d_, cfg, stream_));
     if (ev) LK(hipEventRecord(ev[2], stream_));
-    LK(launch_density(d_, cfg_, stream_));
+    LK(launch_density(d_, cfg, stream_));
     if (ev) LK(hipEventRecord(ev[3], stream_));
-    LK(launch_pressure(d_, cfg_, stream_));
+    LK(launch_pressure(d_, cfg, stream_));
     if (ev) LK(hipEventRecord(ev[4], stream_));
-    LK(launch_viscosity_integrate(d_, cfg_, stream_));
+    LK(launch_viscosity_integrate(d_, cfg, stream_));
     if (ev) LK(hipEventRecord(ev[5], stream_));
 #undef LK
     return hipSuccess;
@@ -748,7 +753,7 @@ int Engine::update(float dt, std::string *err)
         }
         stage_ms_[5] = 0.0;  // position + collision runs inside the viscosity kernel
     } else if (use_graph_) {
-        const int gi = (rebuild ? 1 : 0) + (fresh ? 2 : 0);
+        const int gi = (rebuild ? 1 : 0) + (fresh ? 2 : 0) + (coop_slots_now() ? 4 : 0);
         if (!graph_exec_[gi]) {
             CK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
             hipError_t le = enqueue_update(nullptr, rebuild, fresh);
@@ -812,6 +817,7 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
     struct Cand {
         GatherVariant v;
         bool nbr;
+        bool by_size = false;
     };
     std::vector<Cand> cands;
     // (the cell-grid key has no work order; its row mode uses neighbour masks)
@@ -819,6 +825,9 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
         for (int l = 0; l < 2; ++l)
             for (int b : {64, 128, 256}) cands.push_back({GatherVariant{w != 0, l != 0, b, false}, false});
     for (int b : {64, 128, 256}) cands.push_back({GatherVariant{!grid_, false, b, true}, true});
+    // the form that the defaults take at this size, if it is another one
+    if (coop_slots(grid_, n, d_.capacity)) cands.push_back({GatherVariant{}, false, true});
+    double size_ms[3] = {1e30, 1e30, 1e30};
     double walk_ms[3] = {1e30, 1e30, 1e30}, row_ms[3] = {1e30, 1e30, 1e30};
     GatherVariant walk_v[3] = {keep.density, keep.pressure, keep.viscosity}, row_v[3];
     int rc = check(save(), "autotune snapshot", err);
@@ -830,6 +839,9 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
         LaunchCfg c = keep;
         c.density = c.pressure = c.viscosity = cands[ci].v;
         c.nbr = cands[ci].nbr;
+        c.fused = false;
+        c.by_size = cands[ci].by_size;
+        if (c.by_size) c = default_launch_cfg(grid_);
         cfg_ = c;
         invalidate_graph();
         work_valid_ = false;
@@ -844,6 +856,10 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
         for (uint32_t q = 0; q < n_scenes() && !rc; ++q)
             rc = check(refresh_render(q), "autotune restore", err);
         if (rc) break;
+        if (cands[ci].by_size) {  // one form: its three kernels go together
+            for (int q = 0; q < 3; ++q) size_ms[q] = std::min(size_ms[q], ms[2 + q]);
+            continue;
+        }
         double *best = cands[ci].nbr ? row_ms : walk_ms;
         GatherVariant *pick = cands[ci].nbr ? row_v : walk_v;
         for (int q = 0; q < 3; ++q)
@@ -880,13 +896,18 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
         chosen.viscosity = pick[2];
         chosen.nbr = use_nbr;
         chosen.fused = false;
+        chosen.by_size = false;
+        if (size_ms[0] + size_ms[1] + size_ms[2] < best[0] + best[1] + best[2]) {
+            chosen = default_launch_cfg(grid_);
+            for (int q = 0; q < 3; ++q) best[q] = size_ms[q];
+        }
     }
     // The fused update (one persistent launch per steady update) against the
     // separate launches of the chosen variants: `updates` steady updates
     // each, timed whole, two runs of each interleaved, the faster kept.
     cfg_ = chosen;
     cfg_.fused = true;
-    const bool try_fused = !rc && fused_ok(false, false);
+    const bool try_fused = !rc && !chosen.by_size && fused_ok(false, false);
     cfg_ = chosen;
     if (try_fused) {
         hipEvent_t t0 = nullptr, t1 = nullptr;
@@ -998,7 +1019,7 @@ int Engine::step(float dt, int substeps, bool sync_after, std::string *err)
         // all, which saves the gaps between separate graph launches.  While
         // profiling, the first update of the step is the profiled one.
         if (left > 1 && use_graph_ && !timing_ && (!prof_active_ || i > 0) && recorded_ &&
-            sub == dt_cached_ && (grid_ || !cfg_.needs_work())) {
+            sub == dt_cached_ && (grid_ || coop_slots_now() || !cfg_.needs_work())) {
             const int rc = run_steady(left, err);
             if (rc) return rc;
             break;
@@ -1011,7 +1032,8 @@ int Engine::step(float dt, int substeps, bool sync_after, std::string *err)
 
 int Engine::run_steady(int n, std::string *err)
 {
-    if (!run_exec_ || run_len_ != n) {
+    const bool coop = coop_slots_now() != 0;
+    if (!run_exec_ || run_len_ != n || run_coop_ != coop) {
         if (run_exec_) (void)hipGraphExecDestroy(run_exec_);
         if (run_graph_) (void)hipGraphDestroy(run_graph_);
         run_exec_ = nullptr;
@@ -1025,6 +1047,7 @@ int Engine::run_steady(int n, std::string *err)
         CK(ce, "end capture");
         CK(hipGraphInstantiate(&run_exec_, run_graph_, nullptr, nullptr, 0), "instantiate graph");
         run_len_ = n;
+        run_coop_ = coop;
     }
     CK(hipGraphLaunch(run_exec_, stream_), "graph launch");
     work_updates_ += (uint64_t)n;
@@ -1080,15 +1103,17 @@ int Engine::prime(std::string *err)
         sd_h_[q].lookahead = 0.0f;
     }
     rc = push_descs(err);
-    hipError_t e = rc ? hipSuccess : launch_predict(d_, cfg_, stream_);
-    if (!rc && e == hipSuccess && !grid_ && cfg_.needs_work()) {
+    LaunchCfg cfg = cfg_;
+    cfg.coop_n = coop_slots_now();
+    hipError_t e = rc ? hipSuccess : launch_predict(d_, cfg, stream_);
+    if (!rc && e == hipSuccess && !grid_ && !cfg.coop_n && cfg.needs_work()) {
         int wb = 0;
         e = launch_radix_sort(d_, d_.wkeys, d_.wvals, d_.ids, 32, stream_, &wb);
         d_.work = d_.wvals[wb];
         work_valid_ = e == hipSuccess;
     }
-    if (!rc && e == hipSuccess) e = launch_bucket_sort(d_, cfg_, stream_);
-    if (!rc && e == hipSuccess) e = launch_density(d_, cfg_, stream_);
+    if (!rc && e == hipSuccess) e = launch_bucket_sort(d_, cfg, stream_);
+    if (!rc && e == hipSuccess) e = launch_density(d_, cfg, stream_);
     if (!rc && e == hipSuccess) e = hipStreamSynchronize(stream_);
     // the settings' lookahead again for the updates
     for (size_t q = 0; q < sd_h_.size(); ++q) sd_h_[q].lookahead = lookahead[q];

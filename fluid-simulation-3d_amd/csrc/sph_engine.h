@@ -114,6 +114,7 @@ class Engine {
     void set_launch_cfg(const LaunchCfg &c)
     {
         cfg_ = sanitize_launch_cfg(c, grid_);
+        cfg_.by_size = same_variants(cfg_, default_launch_cfg(grid_));
         invalidate_graph();
     }
     bool grid() const { return grid_; }
@@ -129,8 +130,14 @@ class Engine {
     // three kernels, a steady update, and a launch the device holds resident
     bool fused_ok(bool rebuild_work, bool fresh) const
     {
-        return cfg_.fused && grid_ && cfg_.nbr && cfg_.density.rows && cfg_.pressure.rows &&
+        return cfg_.fused && coop_slots_now() == 0 && grid_ && cfg_.nbr && cfg_.density.rows && cfg_.pressure.rows &&
                cfg_.viscosity.rows && !rebuild_work && !fresh && d_.fused_grid != 0;
+    }
+    // Slots of the sixteen-work-item gathers' grid for the present layout (0:
+    // the one-work-item forms run).
+    uint32_t coop_slots_now() const
+    {
+        return cfg_.by_size ? coop_slots(grid_, ed_h_->n_total, d_.capacity) : 0u;
     }
     int set_use_graph(bool on) { use_graph_ = on; invalidate_graph(); return 0; }
     // Mean duration (ms) of each gather kernel over the last timed update.
@@ -151,7 +158,7 @@ class Engine {
     int run_steady(int n, std::string *err);  // n steady updates as one graph launch
     bool rebuild_due() const
     {
-        return !grid_ && cfg_.needs_work() && (!work_valid_ || work_updates_ % work_period_ == 0);
+        return !grid_ && coop_slots_now() == 0 && cfg_.needs_work() && (!work_valid_ || work_updates_ % work_period_ == 0);
     }
     int check(hipError_t e, const char *what, std::string *err);
     // After a stream synchronisation: a device-side failure of the updates
@@ -184,14 +191,16 @@ class Engine {
     bool have_tables_ = false;
     bool grid_ = false;  // cell-grid bucket key (else the reference's hash % table)
     bool use_graph_ = true;
-    // [rebuild work order? + 2 * fresh predict?]
-    hipGraph_t graph_[4] = {nullptr, nullptr, nullptr, nullptr};
-    hipGraphExec_t graph_exec_[4] = {nullptr, nullptr, nullptr, nullptr};
+    // [rebuild work order? + 2 * fresh predict? + 4 * sixteen-work-item gathers?]
+    static constexpr int kGraphs = 8;
+    hipGraph_t graph_[kGraphs] = {};
+    hipGraphExec_t graph_exec_[kGraphs] = {};
     // run_len_ consecutive steady updates (buckets recorded, no work-order
     // rebuild) captured as one graph, for the substeps of a step
     hipGraph_t run_graph_ = nullptr;
     hipGraphExec_t run_exec_ = nullptr;
     int run_len_ = 0;
+    bool run_coop_ = false;
     // The last update's viscosity pass recorded the next update's buckets
     // (keys, tickets, counts) and nothing has changed since: state, settings,
     // layout and dt.  Otherwise the next update starts with predict.

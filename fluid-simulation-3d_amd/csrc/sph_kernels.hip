@@ -36,8 +36,7 @@
 // particle index) whatever order its input is in.
 #include <hip/hip_runtime.h>
 
-#include "sph_device.h"
-#include "sph_launch.h"
+#include "sph_kernel_common.h"
 
 namespace sph {
 
@@ -48,128 +47,10 @@ constexpr int kRadix = 1 << kRadixBits;
 constexpr int kSortBlock = 256;  // 4 waves
 constexpr int kSortWaves = kSortBlock / 64;
 
-__device__ __forceinline__ uint32_t grid_stride() { return gridDim.x * blockDim.x; }
-__device__ __forceinline__ uint32_t global_id() { return blockIdx.x * blockDim.x + threadIdx.x; }
-
-// Scene q's descriptor for a wave-uniform q, read through the constant
-// address space: the table does not change while a kernel runs, so the reads
-// are scalar loads into scalar registers wherever they are placed.
-__device__ __forceinline__ SceneDesc scene_uniform(const SceneDesc *sd, uint32_t q)
-{
-#if __HIP_DEVICE_COMPILE__
-    typedef const __attribute__((address_space(4))) uint32_t ConstWord;
-    const ConstWord *w = (const ConstWord *)(sd + q);
-    SceneDesc d;
-    uint32_t *o = reinterpret_cast<uint32_t *>(&d);
-#pragma unroll
-    for (uint32_t j = 0; j < sizeof(SceneDesc) / 4; ++j) o[j] = w[j];
-    return d;
-#else
-    return sd[q];  // (host pass: never called)
-#endif
-}
-
-// Runs body(S) with slot k's scene.  MULTI: the wave takes its scenes one at
-// a time (one pass unless it spans a scene boundary), the lanes of that scene
-// active and its descriptor read with scalar loads into scalar registers.
-// The loop runs on a wave-uniform mask, and a lane's membership is read back
-// from a ballot, so the compiler keeps the body inside the loop with the
-// uniform scene index (rather than substituting the per-lane one).
-template <bool MULTI, typename Body>
-__device__ __forceinline__ void run_scene(const SceneDesc *sd, const uint32_t *scene_of, uint32_t k,
-                                          Body &body)
-{
-    if (!MULTI) {
-        body(sd[0]);
-        return;
-    }
-    const uint32_t q = scene_of[k], lane = threadIdx.x & 63u;
-    uint64_t pending = __ballot(1);
-    while (pending) {
-        const uint32_t qq = (uint32_t)__builtin_amdgcn_readlane((int)q, (int)__builtin_ctzll(pending));
-        const uint64_t mine = __ballot(q == qq);
-        if ((mine >> lane) & 1u) body(scene_uniform(sd, qq));
-        pending &= ~mine;
-    }
-}
-
-template <bool MULTI>
-__device__ __forceinline__ const SceneDesc &scene_of_slot(const SceneDesc *sd,
-                                                          const uint32_t *scene_of, uint32_t k)
-{
-    return MULTI ? sd[scene_of[k]] : sd[0];
-}
-
-// PositionToCellCoord (cc:499-503): floor(pos / r) with IEEE division, then (int).
-__device__ __forceinline__ int cell_coord(float x, float h) { return (int)floorf(x / h); }
-
-// ---------------------------------------------------------------------------
-// Stage A + B1
-// ---------------------------------------------------------------------------
-// 10-bit Morton spread: bit i of x moves to bit 3i.
-__device__ __forceinline__ uint32_t spread3(uint32_t x)
-{
-    x &= 0x3ffu;
-    x = (x | (x << 16)) & 0x030000ffu;
-    x = (x | (x << 8)) & 0x0300f00fu;
-    x = (x | (x << 4)) & 0x030c30c3u;
-    x = (x | (x << 2)) & 0x09249249u;
-    return x;
-}
-
-// Ordering key of the gather kernels' work order: scene index in the top
-// bits, then the Morton code of the cell (relative to the scene's box,
-// clamped to 10 bits per axis).  It only decides WHICH work-item handles a
-// particle, never a result, so clamping and truncation are harmless.
-__device__ __forceinline__ uint32_t work_key(const EngineDesc &E, const SceneDesc &S, uint32_t s,
-                                             int cx, int cy, int cz)
-{
-    const uint32_t ux = (uint32_t)min(max(cx - S.cell_lo[0], 0), 1023);
-    const uint32_t uy = (uint32_t)min(max(cy - S.cell_lo[1], 0), 1023);
-    const uint32_t uz = (uint32_t)min(max(cz - S.cell_lo[2], 0), 1023);
-    const uint32_t m = spread3(ux) | (spread3(uy) << 1) | (spread3(uz) << 2);
-    return E.scene_shift >= 32 ? m : ((s << E.scene_shift) | (m >> E.morton_drop));
-}
-
-// ---------------------------------------------------------------------------
-// Stage A + B1
-// ---------------------------------------------------------------------------
-// Stage A of one particle (cc:42-48) and its cell (cc:499-503) and hash
-// (cc:505-511).  Every kernel that needs them recomputes them from the same
-// inputs with the same operations, so the values agree to the bit.
-struct Predicted {
-    float vx, vy, vz;  // velocity += CalculateExternalFoce(...) * deltatime (cc:45)
-    float px, py, pz;  // predictedPositions = positions + velocity * (1/120) (cc:47)
-    int cx, cy, cz;
-    uint32_t hash;
-};
-
-__device__ __forceinline__ Predicted predict_particle(const SceneDesc &S, const float4 &x,
-                                                      const float4 &v)
-{
-    Predicted P;
-    const float dt = S.dt;
-    P.vx = v.x + S.g[0] * dt;
-    P.vy = v.y + S.g[1] * dt;
-    P.vz = v.z + S.g[2] * dt;
-    P.px = x.x + P.vx * S.lookahead;
-    P.py = x.y + P.vy * S.lookahead;
-    P.pz = x.z + P.vz * S.lookahead;
-    P.cx = cell_coord(P.px, S.h);
-    P.cy = cell_coord(P.py, S.h);
-    P.cz = cell_coord(P.pz, S.h);
-    P.hash = hash_cell(P.cx, P.cy, P.cz);
-    return P;
-}
-
-// Where the next sort puts a particle: its bucket (GetKeyFromHash, cc:513-516,
-// or the cell-grid key) and a ticket, a distinct place in the bucket in
-// arbitrary order, from count ([table_total] records per bucket, zero before
-// the first record; then [n_scenes] flags raised when a particle's cell lies
-// outside the grid's box).  One atomic per run of equal keys in consecutive
-// lanes: in the resident order, nearly sorted, a wave's 64 records fall in a
-// few runs.  Every lane of the wave that has not exited calls this, the
-// active lanes a prefix of the wave; S is read only when `valid`.
+// Where the next sort puts a particle: its bucket and a ticket in it, from
+// count ([table_total] records per bucket, zero before the first record; then
+// [n_scenes] flags raised when a particle's cell lies outside the grid's box).
+// S is read only when `valid`; see bucket_ticket for the lanes that call this.
 __device__ __forceinline__ void record_bucket(const EngineDesc &E, const SceneDesc &S,
                                               const Predicted &P, bool valid, uint32_t g,
                                               uint32_t *__restrict__ keys,
@@ -177,31 +58,14 @@ __device__ __forceinline__ void record_bucket(const EngineDesc &E, const SceneDe
                                               uint32_t *__restrict__ count,
                                               uint32_t *__restrict__ wkeys)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t upto = (2ull << lane) - 1ull;  // lanes 0..lane
     uint32_t key = 0xffffffffu;
     if (valid) {
-        key = S.key_off + (S.grid ? grid_key(P.cx, P.cy, P.cz, S.cell_lo, S.gdim, S.gmod)
-                                  : fastmod(P.hash, S.mod_m, S.table));
+        key = bucket_key(E, S, P, count);
         keys[g] = key;
-        // grid key: a cell outside the grid's box wraps onto another cell's bucket
-        if (S.grid && ((uint32_t)P.cx - (uint32_t)S.cell_lo[0] >= S.gdim[0] ||
-                       (uint32_t)P.cy - (uint32_t)S.cell_lo[1] >= S.gdim[1] ||
-                       (uint32_t)P.cz - (uint32_t)S.cell_lo[2] >= S.gdim[2]))
-            count[E.table_total + S.index] = 1u;
         if (wkeys) wkeys[g] = work_key(E, S, S.index, P.cx, P.cy, P.cz);
     }
-    // runs of equal keys: a run starts at lane 0, after a different key, and
-    // after a lane without a record (those come after every lane with one)
-    const uint32_t prev = __shfl_up(key, 1u, 64);
-    const uint64_t heads = __ballot(valid && (lane == 0u || prev != key)) | ~__ballot(valid);
-    const uint32_t first = 63u - (uint32_t)__builtin_clzll(heads & upto);  // this run's head
-    const uint64_t later = heads & ~upto;
-    const uint32_t len = (later ? (uint32_t)__builtin_ctzll(later) : 64u) - lane;
-    uint32_t base = 0;
-    if (valid && first == lane) base = atomicAdd(&count[key], len);
-    base = __shfl(base, (int)first, 64);
-    if (valid) ticks[g] = base + (lane - first);
+    const uint32_t ticket = bucket_ticket(valid, key, count);
+    if (valid) ticks[g] = ticket;
 }
 
 // Stage A + B1 over resident slots g, for an update whose buckets the previous
@@ -1628,10 +1492,10 @@ __device__ __forceinline__ void density_vblock(uint32_t vblock_, SPH_GATHER_PARA
     uint32_t *row = ROWS ? nbr + (size_t)i * kNbrMax : nullptr;
     uint32_t c = 0;
     auto body = [&](uint32_t m, float, float, float, float d2, const float4 &) {
-        const float d = sqrtf(d2);
-        const float v = h - d;
-        rho += v * v * w2c;       // SmoothingPow2, kernels.h:31
-        rhon += v * v * v * w3c;  // SmoothingPow3, kernels.h:43
+        float a, b;
+        density_pair(h, w2c, w3c, d2, a, b);
+        rho += a;
+        rhon += b;
         if (ROWS && m != k) {
             if (c < kNbrMax) row[c] = m;
             ++c;
@@ -1703,10 +1567,10 @@ __global__ __launch_bounds__(256) void k_density_rows(SPH_GATHER_PARAMS, float4 
         float rho = 0.0f, rhon = 0.0f;
         walk<false, false, false>(S, xps, nullptr, start, endt, k, pi, nullptr, false,
                            [&](uint32_t m, float, float, float, float d2, const float4 &) {
-            const float d = sqrtf(d2);
-            const float v = h - d;
-            rho += v * v * w2c;       // SmoothingPow2, kernels.h:31
-            rhon += v * v * v * w3c;  // SmoothingPow3, kernels.h:43
+            float a, b;
+            density_pair(h, w2c, w3c, d2, a, b);
+            rho += a;
+            rhon += b;
             if (m != k) {
                 if (c < kNbrMax) my[c] = m;
                 ++c;
@@ -1735,57 +1599,16 @@ __device__ __forceinline__ void pressure_vblock(uint32_t vblock_, SPH_GATHER_PAR
     constexpr bool CONSUMER = NBR && GRID;  // reads the neighbour masks
     SPH_GATHER_PROLOGUE();
     const float4 di = dens[k];
-    const float h = S.h, dw2c = S.dw2c, dw3c = S.dw3c, rho0 = S.rho0, kp = S.k, kn = S.k_near;
-    const float P = (di.x - rho0) * kp, Pn = di.y * kn;  // cc:371-372
-    // the quotients by d need only d's range when the coordinate differences
-    // to every neighbour are either zero or of magnitude >= 2^-84
-    const int near_ok = (int)coords_clear_of_zero(pi.x, pi.y, pi.z);
+    const PressureSelf self = pressure_self(S, pi, di);
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-    // Every division is correctly rounded.  dj = (rho_j, rho_near_j,
-    // RN(1/rho_j), RN(1/rho_near_j)); the six divisions by rho_j / rho_near_j
-    // use those reciprocals and the three by d use RN(1/d), through
-    // quotient() (exact in its stated range), and fall back to IEEE division
-    // outside that range
     auto body = [&](uint32_t, float ox, float oy, float oz, float d2, const float4 &dj) {
-        const float pj = (dj.x - rho0) * kp, pnj = dj.y * kn;  // cc:407-408
-        const float sp = (P + pj) * 0.5f;     // cc:410
-        const float snp = (Pn + pnj) * 0.5f;  // cc:411
-        const float d = sqrtf(d2);
-        float dirx = 0.0f, diry = 1.0f, dirz = 0.0f;  // cc:414
-        if (d > 0.0f) {
-            if ((near_ok & (int)divisor_ok(d)) != 0) {
-                const float yd = recip_rn(d);
-                dirx = quotient(ox, d, yd);
-                diry = quotient(oy, d, yd);
-                dirz = quotient(oz, d, yd);
-            } else {
-                dirx = ox / d;
-                diry = oy / d;
-                dirz = oz / d;
-            }
-        }
-        const float v = h - d;
-        const float a = -v * dw2c;      // SmoothingDerivativePow2, kernels.h:55
-        const float b = -v * v * dw3c;  // SmoothingDerivativePow3, kernels.h:67
-        const float tx = dirx * a * sp, ty = diry * a * sp, tz = dirz * a * sp;
-        const float ux = dirx * b * snp, uy = diry * b * snp, uz = dirz * b * snp;
-        const bool fast = ((int)(dj.z != 0.0f) & (int)(dj.w != 0.0f) &
-                           (int)quotients_ok(tx, ty, tz, ux, uy, uz)) != 0;
-        if (fast) {
-            fx += quotient(tx, dj.x, dj.z);  // cc:416
-            fy += quotient(ty, dj.x, dj.z);
-            fz += quotient(tz, dj.x, dj.z);
-            fx += quotient(ux, dj.y, dj.w);  // cc:417
-            fy += quotient(uy, dj.y, dj.w);
-            fz += quotient(uz, dj.y, dj.w);
-        } else {
-            fx += tx / dj.x;
-            fy += ty / dj.x;
-            fz += tz / dj.x;
-            fx += ux / dj.y;
-            fy += uy / dj.y;
-            fz += uz / dj.y;
-        }
+        const PressureTerms r = pressure_pair(self, ox, oy, oz, d2, dj);
+        fx += r.tx;  // cc:416
+        fy += r.ty;
+        fz += r.tz;
+        fx += r.ux;  // cc:417
+        fy += r.uy;
+        fz += r.uz;
     };
     if (NBR && GRID) {
         const uint2 mt2 = reinterpret_cast<const uint2 *>(nbr)[kMaskMetaAt * (size_t)ed->n_total + k];
@@ -1840,9 +1663,7 @@ __device__ __forceinline__ void viscosity_vblock(uint32_t vblock_, SPH_GATHER_PA
     const float hh = S.hh, c6 = S.poly6c;
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     auto body = [&](uint32_t, float, float, float, float d2, const float4 &vj) {
-        const float d = sqrtf(d2);
-        const float v = hh - d * d;          // kernels.h:78
-        const float w = v * v * v * c6;      // kernels.h:79
+        const float w = viscosity_weight(hh, c6, d2);
         fx += (vj.x - vi.x) * w;             // cc:460
         fy += (vj.y - vi.y) * w;
         fz += (vj.z - vi.z) * w;
@@ -1859,20 +1680,8 @@ __device__ __forceinline__ void viscosity_vblock(uint32_t vblock_, SPH_GATHER_PA
     } else {
         gather<GRID, LIST, true, true>(S, xps, vs2, start, endt, lst, stage, clean, k, pi, body);
     }
-    const float dt = S.dt, mu = S.mu;
-    float4 v = vi;
-    v.x = vi.x + fx * mu * dt;  // cc:463
-    v.y = vi.y + fy * mu * dt;
-    v.z = vi.z + fz * mu * dt;
-    // stage F (cc:84-107), per particle
-    float4 x = x0;
-    x.x += v.x * dt;
-    x.y += v.y * dt;
-    x.z += v.z * dt;
-    if (S.half[0] - fabsf(x.x) <= 0.0f) { x.x = S.half[0] * sign_f(x.x); v.x *= S.damp_neg; }
-    if (S.half[1] - fabsf(x.y) <= 0.0f) { x.y = S.half[1] * sign_f(x.y); v.y *= S.damp_neg; }
-    if (S.half[2] - fabsf(x.z) <= 0.0f) { x.z = S.half[2] * sign_f(x.z); v.z *= S.damp_neg; }
-    x.w = 0.34f;  // OutPositions[i] = vec4(positions[i], 0.34f), cc:107
+    float4 x, v;
+    integrate_particle(S, vi, fx, fy, fz, x0, x, v);
     pos[k] = x;
     vel[k] = v;
     ids[k] = g;
@@ -2252,6 +2061,7 @@ inline uint32_t gather_grid(uint32_t cap, int block)
 
 hipError_t launch_density(const DevState &s, const LaunchCfg &c, hipStream_t st)
 {
+    if (c.coop_n) return launch_coop_density(s, c.coop_n, st);
     if (c.nbr && s.grid) {
         // the density pass records the neighbour masks
         const int b = c.density.block;
@@ -2283,6 +2093,7 @@ hipError_t launch_density(const DevState &s, const LaunchCfg &c, hipStream_t st)
 
 hipError_t launch_pressure(const DevState &s, const LaunchCfg &c, hipStream_t st)
 {
+    if (c.coop_n) return launch_coop_pressure(s, c.coop_n, st);
     SPH_GATHER_LAUNCH(k_pressure, c.pressure, c.pressure.block, st, SPH_GATHER_ARGS, s.dens, s.vs,
                       s.vs2);
     SPH_LAUNCH_CHECK();
@@ -2290,6 +2101,7 @@ hipError_t launch_pressure(const DevState &s, const LaunchCfg &c, hipStream_t st
 
 hipError_t launch_viscosity_integrate(const DevState &s, const LaunchCfg &c, hipStream_t st)
 {
+    if (c.coop_n) return launch_coop_viscosity_integrate(s, c.coop_n, st);
     SPH_GATHER_LAUNCH(k_viscosity_integrate, c.viscosity, c.viscosity.block, st, SPH_GATHER_ARGS,
                       s.vs2, s.ps, s.pos, s.vel, s.ids, s.rpos, s.colors, s.keys[0], s.keys[1],
                       s.count, s.grid ? nullptr : s.wkeys[0]);

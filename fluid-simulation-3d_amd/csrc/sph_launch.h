@@ -60,7 +60,8 @@ struct DevState {
     float4 *rpos;        // [capacity] render positions, particle order (null: not written)
     uint32_t *sflags;    // [scenes] grid key: 1 when a particle's cell lies outside the grid's box
                          // (copied from the count flags by the bucket sort)
-    uint32_t *nbr;       // [capacity * 64] neighbour rows by work index (nbr mode)
+    uint32_t *nbr;       // [(capacity + 1) * nbr_words] neighbour rows by work index (nbr mode); one spare
+    uint32_t nbr_words;  // words per particle of nbr
     uint32_t *ncnt;      // [capacity] neighbour count per row
     uint32_t *scan_err;  // [1] raised when a bounded wait gave up (count scan, grid barrier)
     uint32_t *fbar;      // [kFusedBarWords] grid barrier of the fused update (zero between launches)
@@ -89,6 +90,12 @@ struct LaunchCfg {
     // recorded) is one persistent launch with grid barriers between its
     // stages (launch_fused_update) instead of one launch per stage
     bool fused = false;
+    // the form of the gathers follows the scene's size (coop_slots): set in the
+    // defaults, cleared by any other choice of variants
+    bool by_size = false;
+    // > 0: the gathers run with sixteen work-items per particle, over a grid
+    // of this many slots (by_size, set per update by the engine)
+    uint32_t coop_n = 0;
     int block_stream = 256;  // threads per block of streaming kernels
     bool needs_work() const { return nbr || density.work || pressure.work || viscosity.work; }
 };
@@ -113,7 +120,37 @@ inline LaunchCfg default_launch_cfg(bool grid)
         c.viscosity = GatherVariant{false, false, 128, true};
         c.nbr = true;
     }
+    c.by_size = true;
     return sanitize_launch_cfg(c, grid);
+}
+
+// The same variants (whatever by_size and coop_n say).
+inline bool same_variants(const LaunchCfg &a, const LaunchCfg &b)
+{
+    auto same = [](const GatherVariant &x, const GatherVariant &y) {
+        return x.work == y.work && x.list == y.list && x.block == y.block && x.rows == y.rows;
+    };
+    return same(a.density, b.density) && same(a.pressure, b.pressure) && same(a.viscosity, b.viscosity) &&
+           a.nbr == b.nbr && a.fused == b.fused;
+}
+
+// Largest particle count for which the gathers run with several work-items per
+// particle (sph_coop.hip); above it one work-item per particle fills the chip
+// and tests each candidate cheaper.  Measured, us per steady update (all
+// kernels) with one / several work-items per particle:
+//   grid key       1,000: 64 / 27   16,384: 77 / 34   65,536: 85 / 60
+//                  131,072: 94 / 94   200,000: 115 / 127
+//   reference key  4,000: 153 / 30   50,000: 195 / 67   200,000: 318 / 184
+//                  1,000,000: 1,018 / 878
+constexpr uint32_t kCoopMaxGrid = 1u << 17;
+constexpr uint32_t kCoopMaxReference = 1u << 20;
+
+// Slots that the sixteen-work-item gathers' grid covers for n particles in a
+// layout of `capacity` slots, or 0 when the one-work-item forms run.
+inline uint32_t coop_slots(bool grid, uint32_t n, uint32_t capacity)
+{
+    const uint32_t most = grid ? kCoopMaxGrid : kCoopMaxReference;
+    return n > most ? 0u : (capacity < most ? capacity : most);
 }
 
 // Stage A + B1 when the previous update did not record the buckets: clears
@@ -140,6 +177,12 @@ hipError_t launch_radix_sort(const DevState &s, uint32_t *const keys[2], uint32_
 hipError_t launch_density(const DevState &s, const LaunchCfg &c, hipStream_t st);
 hipError_t launch_pressure(const DevState &s, const LaunchCfg &c, hipStream_t st);
 hipError_t launch_viscosity_integrate(const DevState &s, const LaunchCfg &c, hipStream_t st);
+
+// The same stages with sixteen work-items per particle (sph_coop.hip), over the
+// first n slots (n >= the live particles).
+hipError_t launch_coop_density(const DevState &s, uint32_t n, hipStream_t st);
+hipError_t launch_coop_pressure(const DevState &s, uint32_t n, hipStream_t st);
+hipError_t launch_coop_viscosity_integrate(const DevState &s, uint32_t n, hipStream_t st);
 
 // Sorted -> particle order densities (rho, rho_near) for download.
 hipError_t launch_unpermute_dens(const DevState &s, float2 *out, hipStream_t st);

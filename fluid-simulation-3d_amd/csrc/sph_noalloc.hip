@@ -34,6 +34,8 @@ constexpr uint32_t kNoAllocMaxParticles = SPH_NOALLOC_MAX_PARTICLES;
 // the cell-grid key sizes a scene of n <= 2^16 particles to at most
 // max(8n, 2^20) = 2^20 buckets (grid_table_size)
 constexpr uint32_t kNoAllocMaxBuckets = 1u << 20;
+// neighbour-row words per particle (neighbour-mask records use up to 18 of them)
+constexpr uint32_t kNoAllocNbrWords = 27;
 constexpr uint32_t kCountChunk = sph::kCountChunkBuckets;  // buckets per workgroup of the count scan
 
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -77,7 +79,7 @@ constexpr Layout make_layout()
     L.sids = take(4 * N);
     L.ncnt = take(4 * N);
     L.order = take(8 * N);
-    L.nbr = take(4 * 27 * N);  // neighbour-mask records: up to 18 words per particle used
+    L.nbr = take(4 * kNoAllocNbrWords * N);
     L.total = o;
     return L;
 }
@@ -198,6 +200,7 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     s.bounds = at<uint32_t>(base, kLayout.bounds);
     s.sflags = at<uint32_t>(base, kLayout.sflags);
     s.nbr = at<uint32_t>(base, kLayout.nbr);
+    s.nbr_words = kNoAllocNbrWords;
     s.ncnt = at<uint32_t>(base, kLayout.ncnt);
     s.scan_err = at<uint32_t>(base, kLayout.scan_err);
     s.capacity = n;
@@ -206,7 +209,8 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     sph::DevState out = s;  // the viscosity pass and the unpermute: state in `scratch`
     out.pos = at<float4>(base, kLayout.pos);
     out.vel = at<float4>(base, kLayout.vel);
-    const sph::LaunchCfg c = sph::default_launch_cfg(true);
+    sph::LaunchCfg c = sph::default_launch_cfg(true);
+    c.coop_n = sph::coop_slots(true, n, n);
 
     hipError_t e = hipSuccess;
 #define NA(x, what)                                  \

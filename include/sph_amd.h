@@ -192,7 +192,10 @@ int sph_profile_end(sph_handle h, double mean_ms[6], uint32_t *updates);
  * variants give bit-identical results.  ms (may be NULL) gets the chosen
  * variants' mean ms (density, pressure, viscosity).  Densities and debug
  * tables are recomputed by the next update.  Without it a handle runs the
- * defaults (under the grid key: neighbour masks for all three kernels). */
+ * defaults (under the grid key: neighbour masks for all three kernels), and
+ * while its variants are the defaults the form of the three kernels follows
+ * the scene's size: small scenes run them with several work-items per
+ * particle. */
 int sph_autotune(sph_handle h, float dt, int updates, double ms[3]);
 /* The variant of each gather kernel, q = 0 density, 1 pressure, 2 viscosity:
  * v[4q+0] work order (reference key only; ignored under the grid key),
