@@ -109,8 +109,11 @@ int sph_device_count(void)
     return n;
 }
 
-int sph_debug_reciprocal_mismatches(uint32_t lo_bits, uint32_t hi_bits, uint64_t *count,
-                                    uint32_t *first)
+namespace {
+using FloatCheck = hipError_t (*)(uint32_t, uint32_t, unsigned long long *, uint32_t *, hipStream_t);
+
+// Runs `check` over the floats with bit patterns in [lo_bits, hi_bits].
+int float_check(FloatCheck check, uint32_t lo_bits, uint32_t hi_bits, uint64_t *count, uint32_t *first)
 {
     SPH_GUARD_BEGIN
     if (!count || lo_bits > hi_bits) return fail(SPH_ERR_INVALID, "null count or empty range");
@@ -125,16 +128,28 @@ int sph_debug_reciprocal_mismatches(uint32_t lo_bits, uint32_t hi_bits, uint64_t
     hipError_t e = hipMalloc((void **)&dev, sizeof(Out));
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMemcpyAsync(dev, &host, sizeof(Out), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = sph::launch_recip_check(lo_bits, hi_bits, &dev->bad, &dev->first, st);
+    if (e == hipSuccess) e = check(lo_bits, hi_bits, &dev->bad, &dev->first, st);
     if (e == hipSuccess) e = hipMemcpyAsync(&host, dev, sizeof(Out), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (st) (void)hipStreamDestroy(st);
     if (dev) (void)hipFree(dev);
-    if (e != hipSuccess) return fail(SPH_ERR_HIP, std::string("reciprocal check: ") + hipGetErrorString(e));
+    if (e != hipSuccess) return fail(SPH_ERR_HIP, std::string("float check: ") + hipGetErrorString(e));
     *count = host.bad;
     if (first) *first = host.first;
     return SPH_OK;
     SPH_GUARD_END
+}
+}  // namespace
+
+int sph_debug_reciprocal_mismatches(uint32_t lo_bits, uint32_t hi_bits, uint64_t *count,
+                                    uint32_t *first)
+{
+    return float_check(sph::launch_recip_check, lo_bits, hi_bits, count, first);
+}
+
+int sph_debug_root_mismatches(uint32_t lo_bits, uint32_t hi_bits, uint64_t *count, uint32_t *first)
+{
+    return float_check(sph::launch_root_check, lo_bits, hi_bits, count, first);
 }
 
 int sph_copy_calibration(uint64_t bytes, int reps, double *ms_per_copy)

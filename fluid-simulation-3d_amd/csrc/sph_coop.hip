@@ -373,7 +373,7 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_density(const CoopArgs A
                     const uint32_t at = have ? t : 0u;
                     const uint2 e = lst[at];
                     float a, b;
-                    density_pair(h, w2c, w3c, __uint_as_float(e.y), a, b);
+                    density_pair<true>(h, w2c, w3c, __uint_as_float(e.y), true, a, b);
                     t0p[r + gl] = have ? a : 0.0f;
                     t1p[r + gl] = have ? b : 0.0f;
                     out.rows[(size_t)(cnt ? k : out.spare) * out.cap + min(total + at, out.cap - 1u)] = (T)e.x;
@@ -435,8 +435,9 @@ __device__ __forceinline__ float coop_sum(const CoopArgs &A, const SceneDesc &S,
                 if (!wave_any(c0 + r * G < cnt)) break;
                 float out[3 * NT];
                 const float ox = x[r].x - pi.x, oy = x[r].y - pi.y, oz = x[r].z - pi.z;
-                pair(ox * ox + oy * oy + oz * oz, ox, oy, oz, a[r], out);
                 const bool have = m[r] != k;  // not the particle itself, nor past the end
+                // (at distance 0 the terms would take their slow path)
+                pair(have ? ox * ox + oy * oy + oz * oz : 0.25f * S.thr, ox, oy, oz, a[r], out);
 #pragma unroll
                 for (int c = 0; c < 3; ++c)
 #pragma unroll
@@ -468,11 +469,11 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_pressure(const CoopArgs 
     float4 v = vs[k];
     auto scene = [&](const SceneDesc &S) __attribute__((always_inline)) {
         const bool clean = GRID && A.sflags[S.index] == 0u;
-        const PressureSelf self = pressure_self(S, pi, di);
+        const PressureSelf self = pressure_self<true>(S, pi, di);
         const float f = coop_sum<G, GRID, 2>(
             A, S, in, dens, k, pi, clean, lists[gq], &terms[gq][0][0],
             [&](float d2, float ox, float oy, float oz, const float4 &dj, float out[6]) {
-                const PressureTerms r = pressure_pair(self, ox, oy, oz, d2, dj);
+                const PressureTerms r = pressure_pair<true>(self, ox, oy, oz, d2, dj);
                 out[0] = r.tx;
                 out[1] = r.ty;
                 out[2] = r.tz;
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_viscosity(const CoopArgs
         const float f = coop_sum<G, GRID, 1>(
             A, S, in, W.vs2, k, pi, clean, lists[gq], &terms[gq][0][0],
             [&](float d2, float, float, float, const float4 &vj, float out[3]) {
-                const float w = viscosity_weight(hh, c6, d2);
+                const float w = viscosity_weight<true>(hh, c6, d2);
                 out[0] = (vj.x - vi.x) * w;  // cc:460
                 out[1] = (vj.y - vi.y) * w;
                 out[2] = (vj.z - vi.z) * w;

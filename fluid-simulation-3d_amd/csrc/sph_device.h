@@ -159,17 +159,36 @@ SPH_HD float recip_rn(float x)
 // y = RN(1/x) for x in [2^-26, 2^26], else 0 (no fast quotient by x).
 SPH_HD float reciprocal_or_zero(float x) { return divisor_ok(x) ? recip_rn(x) : 0.0f; }
 
-// True when |x|, |y|, |z| >= 2^-60.  Then every nonzero difference between
-// this point's coordinates and another float's has magnitude >= 2^-84:
-// floats of magnitude >= 2^-61 are multiples of 2^-84, and a float below
-// 2^-61 lies at least 2^-61 away.  Such differences are valid quotient()
-// numerators whenever the divisor d bounds them (|difference| <= d(1+2^-22)
-// for the components of a distance d <= 2^26).
-SPH_HD bool coords_clear_of_zero(float x, float y, float z)
+// sqrt(x), correctly rounded, for x in [2^-100, 2^100]; for x = 0 it is 0 and
+// for 0 < x < 2^-100 a value in [0, 2^-50] (which is all the same to h - d and
+// h * h - d * d when h >= 2^-16).  On the GPU: g = x * y and h = y / 2 from the
+// hardware estimate y of 1 / sqrt(x) and one residual step g + (x - g * g) * h
+// (Markstein); it equals IEEE sqrt for every float of the range (checked
+// exhaustively on the GPU by sph_debug_root_mismatches).  One transcendental
+// and four fused operations, where the general square root, with its scaling,
+// two neighbours tried and special cases, takes 16 instructions, half of them
+// compares and selects at half rate.  On the host: IEEE sqrt.
+SPH_HD float root_rn(float x)
 {
-    const uint32_t a = mag_bits(x), b = mag_bits(y), c = mag_bits(z);
-    const uint32_t m = a < b ? (a < c ? a : c) : (b < c ? b : c);
-    return m >= 0x21800000u;  // 2^-60
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float y = __builtin_amdgcn_rsqf(fmaxf(x, 0x1p-100f));
+    const float g = x * y, hy = 0.5f * y;
+    return fmaf(fmaf(-g, g, x), hy, g);
+#else
+    return sqrtf(x);
+#endif
+}
+
+// Smoothing radii for which the kernels use root_rn.
+SPH_HD bool radius_fast(float h) { return h >= 0x1p-16f && h <= 0x1p26f; }
+
+// True when |x|, |y|, |z| >= t.  Then every nonzero difference between this
+// point's coordinates and another float's has magnitude >= t * 2^-25: a float
+// of magnitude >= t / 2 is a multiple of an ulp of at least t * 2^-25, and one
+// below t / 2 lies at least t / 2 away.
+SPH_HD bool coords_clear_of_zero(float x, float y, float z, float t)
+{
+    return fminf(fminf(fabsf(x), fabsf(y)), fabsf(z)) >= t;
 }
 
 // glm::sign for float (func_common.inl:144-150): (0 < x) - (x < 0).

@@ -409,6 +409,10 @@ int Engine::push_descs(std::string *err)
         *err = "scene capacity exceeded";
         return SPH_ERR_INVALID;
     }
+    bool fast = true;
+    for (const SceneDesc &d : sd_h_) fast = fast && scene_fast(d);
+    if (fast != all_fast_) invalidate_graph();
+    all_fast_ = fast;
     // the next staging slot, once the copies of its previous use have run
     // (kDescRing uploads ago: normally long done)
     const int q = (int)(desc_no_++ % kDescRing);
@@ -697,8 +701,7 @@ hipError_t Engine::enqueue_update(hipEvent_t *ev, bool rebuild_work, bool fresh,
     // fresh: the previous update did not record this one's buckets (its
     // viscosity pass does otherwise)
     hipError_t e;
-    LaunchCfg cfg = cfg_;
-    cfg.coop_n = coop_slots_now();
+    const LaunchCfg cfg = run_cfg();
 #define LK(x)                              \
     if ((e = (x)) != hipSuccess) return e;
     if (ev && mark_predict) LK(hipEventRecord(ev[0], stream_));
@@ -1103,8 +1106,7 @@ int Engine::prime(std::string *err)
         sd_h_[q].lookahead = 0.0f;
     }
     rc = push_descs(err);
-    LaunchCfg cfg = cfg_;
-    cfg.coop_n = coop_slots_now();
+    const LaunchCfg cfg = run_cfg();
     hipError_t e = rc ? hipSuccess : launch_predict(d_, cfg, stream_);
     if (!rc && e == hipSuccess && !grid_ && !cfg.coop_n && cfg.needs_work()) {
         int wb = 0;

@@ -130,14 +130,21 @@ class Engine {
     // three kernels, a steady update, and a launch the device holds resident
     bool fused_ok(bool rebuild_work, bool fresh) const
     {
-        return cfg_.fused && coop_slots_now() == 0 && grid_ && cfg_.nbr && cfg_.density.rows && cfg_.pressure.rows &&
+        return cfg_.fused && all_fast_ && grid_ && cfg_.nbr && cfg_.density.rows && cfg_.pressure.rows &&
                cfg_.viscosity.rows && !rebuild_work && !fresh && d_.fused_grid != 0;
     }
     // Slots of the sixteen-work-item gathers' grid for the present layout (0:
     // the one-work-item forms run).
     uint32_t coop_slots_now() const
     {
-        return cfg_.by_size ? coop_slots(grid_, ed_h_->n_total, d_.capacity) : 0u;
+        return cfg_.by_size && all_fast_ ? coop_slots(grid_, ed_h_->n_total, d_.capacity) : 0u;
+    }
+    // The variants that an update of the present layout runs.
+    LaunchCfg run_cfg() const
+    {
+        LaunchCfg c = grid_ ? limit_launch_cfg(cfg_, all_fast_) : cfg_;
+        c.coop_n = coop_slots_now();
+        return c;
     }
     int set_use_graph(bool on) { use_graph_ = on; invalidate_graph(); return 0; }
     // Mean duration (ms) of each gather kernel over the last timed update.
@@ -201,6 +208,7 @@ class Engine {
     hipGraphExec_t run_exec_ = nullptr;
     int run_len_ = 0;
     bool run_coop_ = false;
+    bool all_fast_ = true;  // scene_fast of every scene
     // The last update's viscosity pass recorded the next update's buckets
     // (keys, tickets, counts) and nothing has changed since: state, settings,
     // layout and dt.  Otherwise the next update starts with predict.

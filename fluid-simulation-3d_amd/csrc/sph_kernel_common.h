@@ -164,11 +164,20 @@ __device__ __forceinline__ uint32_t bucket_ticket(bool valid, uint32_t key, uint
 // ---------------------------------------------------------------------------
 // Pair terms of stages C to E, and stage F
 // ---------------------------------------------------------------------------
-// Density terms of a neighbour at squared distance d2 (kernels.h:31, 43).
-__device__ __forceinline__ void density_pair(float h, float w2c, float w3c, float d2, float &a, float &b)
+// FAST: the scene's radius lies in radius_fast's range.
+template <bool FAST>
+__device__ __forceinline__ float pair_root(float d2)
 {
-    const float d = sqrtf(d2);
-    const float v = h - d;
+    return FAST ? root_rn(d2) : sqrtf(d2);
+}
+
+// Density terms of a neighbour at squared distance d2 (kernels.h:31, 43); 0
+// when !in.
+template <bool FAST>
+__device__ __forceinline__ void density_pair(float h, float w2c, float w3c, float d2, bool in, float &a, float &b)
+{
+    const float d = pair_root<FAST>(d2);
+    const float v = in ? h - d : 0.0f;
     a = v * v * w2c;      // SmoothingPow2
     b = v * v * v * w3c;  // SmoothingPow3
 }
@@ -177,9 +186,10 @@ __device__ __forceinline__ void density_pair(float h, float w2c, float w3c, floa
 struct PressureSelf {
     float h, dw2c, dw3c, rho0, kp, kn;
     float P, Pn;  // cc:371-372
-    int near_ok;  // the quotients by d need only d's range (coords_clear_of_zero)
+    bool near_ok;
 };
 
+template <bool FAST>
 __device__ __forceinline__ PressureSelf pressure_self(const SceneDesc &S, const float4 &pi, const float4 &di)
 {
     PressureSelf p;
@@ -191,9 +201,7 @@ __device__ __forceinline__ PressureSelf pressure_self(const SceneDesc &S, const 
     p.kn = S.k_near;
     p.P = (di.x - p.rho0) * p.kp;
     p.Pn = di.y * p.kn;
-    // the quotients by d need only d's range when the coordinate differences
-    // to every neighbour are either zero or of magnitude >= 2^-84
-    p.near_ok = (int)coords_clear_of_zero(pi.x, pi.y, pi.z);
+    p.near_ok = FAST && coords_clear_of_zero(pi.x, pi.y, pi.z, S.h * 0x1p-26f);
     return p;
 }
 
@@ -201,39 +209,61 @@ __device__ __forceinline__ PressureSelf pressure_self(const SceneDesc &S, const 
 // Every division is correctly rounded.  dj = (rho_j, rho_near_j,
 // RN(1/rho_j), RN(1/rho_near_j)); the six divisions by rho_j / rho_near_j
 // use those reciprocals and the three by d use RN(1/d), through quotient()
-// (exact in its stated range), and fall back to IEEE division outside that
-// range.
+// (exact for divisors in [2^-26, 2^26] and numerators that are 0 or of
+// magnitude in [2^-91, 2^100]), and fall back to IEEE division outside that
+// range.  FAST proves the range from few values, for h in [2^-16, 2^26]:
+//   - d in [2^-26, 2^26] from d2 >= 2^-52 and d < h, and a nonzero difference
+//     is >= h 2^-51 (near_ok), so a nonzero component of the direction is of
+//     magnitude in [2^-51 (1 - 2^-23), 1 + 2^-22];
+//   - with |sp|, |snp| <= 2^30 and |a sp|, |b snp| >= 2^-38, |a| and |b| are
+//     >= 2^-69, so no product dir * a or dir * b underflows (>= 2^-121), and
+//     every nonzero term is >= 2^-91; |a| <= 15 / (pi h^4) and |b| <= 45 /
+//     (pi h^4) are <= 2^68, so it is <= 2^100.
+// The reciprocals are 0 when unusable and >= 2^-26 else, so one minimum over
+// four values and one maximum over two decide (7 instructions, where testing
+// the six terms takes 26): with root_rn, pressure 120 -> 103 us on 1,048,576
+// uniform particles, where the L1 accesses of the neighbour gathers now take
+// the whole time (41 cycles a load, two loads a neighbour).  Pairs that fail it (weak forces, odd units) are
+// tested term by term before IEEE division is taken.
 struct PressureTerms {
     float tx, ty, tz, ux, uy, uz;
 };
 
+template <bool FAST>
 __device__ __forceinline__ PressureTerms pressure_pair(const PressureSelf &p, float ox, float oy, float oz,
                                                        float d2, const float4 &dj)
 {
     const float pj = (dj.x - p.rho0) * p.kp, pnj = dj.y * p.kn;  // cc:407-408
     const float sp = (p.P + pj) * 0.5f;     // cc:410
     const float snp = (p.Pn + pnj) * 0.5f;  // cc:411
-    const float d = sqrtf(d2);
-    float dirx = 0.0f, diry = 1.0f, dirz = 0.0f;  // cc:414
-    if (d > 0.0f) {
-        if ((p.near_ok & (int)divisor_ok(d)) != 0) {
-            const float yd = recip_rn(d);
-            dirx = quotient(ox, d, yd);
-            diry = quotient(oy, d, yd);
-            dirz = quotient(oz, d, yd);
-        } else {
-            dirx = ox / d;
-            diry = oy / d;
-            dirz = oz / d;
-        }
+    float d = pair_root<FAST>(d2);
+    float dirx, diry, dirz;
+    const bool near_fast = FAST && p.near_ok & (d2 >= 0x1p-52f);
+    if (near_fast) {
+        const float yd = recip_rn(d);
+        dirx = quotient(ox, d, yd);
+        diry = quotient(oy, d, yd);
+        dirz = quotient(oz, d, yd);
+    } else {
+        d = sqrtf(d2);
+        const bool apart = d > 0.0f;  // (0, 1, 0) at d = 0, cc:414
+        dirx = apart ? ox / d : 0.0f;
+        diry = apart ? oy / d : 1.0f;
+        dirz = apart ? oz / d : 0.0f;
     }
     const float v = p.h - d;
     const float a = -v * p.dw2c;      // SmoothingDerivativePow2, kernels.h:55
     const float b = -v * v * p.dw3c;  // SmoothingDerivativePow3, kernels.h:67
     const float tx = dirx * a * sp, ty = diry * a * sp, tz = dirz * a * sp;
     const float ux = dirx * b * snp, uy = diry * b * snp, uz = dirz * b * snp;
-    const bool fast = ((int)(dj.z != 0.0f) & (int)(dj.w != 0.0f) &
-                       (int)quotients_ok(tx, ty, tz, ux, uy, uz)) != 0;
+    bool fast = false;
+    if (FAST) {
+        const float as = fabsf(a * sp), bs = fabsf(b * snp);
+        fast = ((int)near_fast & (int)(fminf(fminf(fminf(as, bs), dj.z), dj.w) >= 0x1p-38f) &
+                (int)(fmaxf(fabsf(sp), fabsf(snp)) <= 0x1p30f)) != 0;
+    }
+    if (!fast)
+        fast = ((int)(dj.z != 0.0f) & (int)(dj.w != 0.0f) & (int)quotients_ok(tx, ty, tz, ux, uy, uz)) != 0;
     PressureTerms r;
     if (fast) {
         r.tx = quotient(tx, dj.x, dj.z);
@@ -254,9 +284,10 @@ __device__ __forceinline__ PressureTerms pressure_pair(const PressureSelf &p, fl
 }
 
 // Viscosity weight of a neighbour at squared distance d2 (kernels.h:78-79).
+template <bool FAST>
 __device__ __forceinline__ float viscosity_weight(float hh, float c6, float d2)
 {
-    const float d = sqrtf(d2);
+    const float d = pair_root<FAST>(d2);
     const float v = hh - d * d;
     return v * v * v * c6;
 }

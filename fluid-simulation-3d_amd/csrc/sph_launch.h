@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "sph_device.h"
 #include "sph_generate.h"
 #include "sph_types.h"
 
@@ -134,6 +135,23 @@ inline bool same_variants(const LaunchCfg &a, const LaunchCfg &b)
            a.nbr == b.nbr && a.fused == b.fused;
 }
 
+// The kernels that read the density pass's records (neighbour masks, or lists
+// with several work-items per particle) take square roots and quotients by
+// methods that are exact for every usual radius; a scene outside that range
+// runs the walking kernels instead, with IEEE operations.
+inline bool scene_fast(const SceneDesc &d) { return radius_fast(d.h) && d.thr >= 0x1p-60f; }
+
+// The variants that run: c, or its walking forms when a scene is not fast.
+inline LaunchCfg limit_launch_cfg(LaunchCfg c, bool all_fast)
+{
+    if (!all_fast) {
+        c.coop_n = 0;
+        c.fused = c.nbr = false;
+        c.density.rows = c.pressure.rows = c.viscosity.rows = false;
+    }
+    return c;
+}
+
 // Largest particle count for which the gathers run with several work-items per
 // particle (sph_coop.hip); above it one work-item per particle fills the chip
 // and tests each candidate cheaper.  Measured, us per steady update (all
@@ -210,6 +228,9 @@ hipError_t launch_generate(const GenPlan &g, float4 *pos, float4 *vel, hipStream
 // min into *first_bad, which the caller sets first).
 hipError_t launch_recip_check(uint32_t lo, uint32_t hi, unsigned long long *bad,
                               uint32_t *first_bad, hipStream_t st);
+// The same for the kernel square root (root_rn) and IEEE sqrt.
+hipError_t launch_root_check(uint32_t lo, uint32_t hi, unsigned long long *bad,
+                             uint32_t *first_bad, hipStream_t st);
 // Plain copy of n float4 (HBM counter calibration).
 hipError_t launch_copy(const float4 *src, float4 *dst, size_t n, hipStream_t st);
 // Count of non-finite position/velocity components (error flag).

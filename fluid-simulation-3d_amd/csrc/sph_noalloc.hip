@@ -211,6 +211,7 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     out.vel = at<float4>(base, kLayout.vel);
     sph::LaunchCfg c = sph::default_launch_cfg(true);
     c.coop_n = sph::coop_slots(true, n, n);
+    c = sph::limit_launch_cfg(c, sph::scene_fast(D));
 
     hipError_t e = hipSuccess;
 #define NA(x, what)                                  \

@@ -187,6 +187,7 @@ def lib():
         "sph_bucket_of": (u32, [u32, u32]),
         "sph_debug_quotients": (i32, [p, p, p, u64]),
         "sph_debug_reciprocal_mismatches": (i32, [u32, u32, p, p]),
+        "sph_debug_root_mismatches": (i32, [u32, u32, p, p]),
     }
     for name, (res, args) in sig.items():
         fn = getattr(L, name)
@@ -250,6 +251,14 @@ def debug_reciprocal_mismatches(lo_bits, hi_bits):
     cnt = np.zeros(1, np.uint64)
     first = np.zeros(1, np.uint32)
     _check(lib().sph_debug_reciprocal_mismatches(int(lo_bits), int(hi_bits), _ptr(cnt), _ptr(first)))
+    return int(cnt[0]), int(first[0])
+
+
+def debug_root_mismatches(lo_bits, hi_bits):
+    """(count, first) of floats in the bit range whose GPU square root differs from IEEE sqrt."""
+    cnt = np.zeros(1, np.uint64)
+    first = np.zeros(1, np.uint32)
+    _check(lib().sph_debug_root_mismatches(int(lo_bits), int(hi_bits), _ptr(cnt), _ptr(first)))
     return int(cnt[0]), int(first[0])
 
 

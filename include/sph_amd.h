@@ -297,6 +297,9 @@ int sph_debug_quotients(const float *a, const float *b, float *out, uint64_t n);
 int sph_debug_reciprocal_mismatches(uint32_t lo_bits, uint32_t hi_bits, uint64_t *count,
                                     uint32_t *first);
 
+/* The same for the kernels' square root and IEEE sqrt. */
+int sph_debug_root_mismatches(uint32_t lo_bits, uint32_t hi_bits, uint64_t *count, uint32_t *first);
+
 /* ---- batching: many independent scenes per launch ----
  * No reference counterpart (the reference simulates one scene per process,
  * physicsWorld.cc:32-37).  A batch owns n_scenes scenes of uneven sizes, each
