@@ -349,8 +349,11 @@ int Engine::alloc(uint32_t cap, uint32_t tcap, std::string *err)
     d_.nbr_words = kNbrWords;
     if (!rc) rc = dm((void **)&d_.ncnt, u4, "neighbour counts");
     if (!rc) rc = dm((void **)&d_.sflags, sizeof(uint32_t) * scene_cap_, "scene flags");
-    if (!rc) rc = dm((void **)&d_.scan_err, sizeof(uint32_t), "scan error flag");
-    if (!rc) rc = check(hipMemset(d_.scan_err, 0, sizeof(uint32_t)), "scan error flag", err);
+    // in host memory that the kernels write: read after a synchronisation without a copy
+    if (!rc) rc = check(hipHostMalloc((void **)&scan_err_h_, sizeof(uint32_t)), "scan error flag", err);
+    if (!rc) *scan_err_h_ = 0;
+    if (!rc)
+        rc = check(hipHostGetDevicePointer((void **)&d_.scan_err, scan_err_h_, 0), "scan error flag", err);
     if (!rc) rc = dm((void **)&d_.fbar, sizeof(uint32_t) * kFusedBarWords, "grid barrier");
     if (!rc) rc = check(hipMemset(d_.fbar, 0, sizeof(uint32_t) * kFusedBarWords), "grid barrier", err);
     // wrapped until a predict pass says otherwise
@@ -371,7 +374,7 @@ Engine::~Engine()
                     d_.ids,      d_.ps,       d_.order,    d_.sids,
                     d_.hist,     d_.bounds,   d_.count,    d_.chain,
                     d_.wkeys[0], d_.wkeys[1], d_.wvals[0], d_.wvals[1], d_.rank,
-                    d_.nbr,      d_.ncnt,     d_.sflags,   d_.scan_err, d_.fbar};
+                    d_.nbr,      d_.ncnt,     d_.sflags,   d_.fbar};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (tmp_pos_) (void)hipFree(tmp_pos_);
@@ -379,6 +382,7 @@ Engine::~Engine()
     if (colors_buf_) (void)hipFree(colors_buf_);
     if (rpos_) (void)hipFree(rpos_);
     if (ed_h_) (void)hipHostFree(ed_h_);
+    if (scan_err_h_) (void)hipHostFree(scan_err_h_);
     for (int q = 0; q < kDescRing; ++q) {
         if (desc_ring_[q]) (void)hipHostFree(desc_ring_[q]);
         if (desc_ev_[q]) (void)hipEventDestroy(desc_ev_[q]);
@@ -1067,11 +1071,9 @@ int Engine::sync(std::string *err)
 
 int Engine::device_status(int s, std::string *err)
 {
-    uint32_t flag = 0;
-    CK(hipMemcpy(&flag, d_.scan_err, sizeof(uint32_t), hipMemcpyDeviceToHost), "read device status");
-    if (flag) {
+    if (*static_cast<volatile uint32_t *>(scan_err_h_)) {
         for (uint8_t &v : invalid_) v = 1;
-        CK(hipMemset(d_.scan_err, 0, sizeof(uint32_t)), "clear device status");
+        *scan_err_h_ = 0;
         // a fused update's barrier that gave up leaves its count behind
         CK(hipMemset(d_.fbar, 0, sizeof(uint32_t) * kFusedBarWords), "clear device status");
     }
@@ -1134,45 +1136,21 @@ int Engine::download(uint32_t s, float *pos4, float *vel4, float *dens2, std::st
         return SPH_ERR_INVALID;
     }
     const SceneDesc &d = sd_h_[s];
+    // Into particle order on the device, in the neighbour rows, which hold
+    // nothing between updates (40 of their 256 bytes per particle), then one
+    // copy per array to the caller.
+    static_assert(sizeof(uint32_t) * kNbrWords >= 2 * sizeof(float4) + sizeof(float2), "download staging");
+    float4 *const pos = reinterpret_cast<float4 *>(d_.nbr), *const vel = pos + d.n;
+    float2 *const dens = reinterpret_cast<float2 *>(vel + d.n);
+    const bool from_tables = dens2 && have_tables_;
+    CK(launch_download(d_, d.p_off, d.n, pos4 ? pos : nullptr, vel4 ? vel : nullptr, from_tables ? dens : nullptr,
+                       stream_), "download order");
     CK(hipStreamSynchronize(stream_), "sync before download");
     if (int rc = device_status((int)s, err)) return rc;
-    if (pos4 || vel4) {
-        // resident order -> particle order on the host
-        std::vector<uint32_t> ids(d.n);
-        std::vector<float4> buf(d.n);
-        CK(hipMemcpy(ids.data(), d_.ids + d.p_off, sizeof(uint32_t) * d.n, hipMemcpyDeviceToHost),
-           "download order");
-        for (uint32_t k = 0; k < d.n; ++k)
-            if (ids[k] - d.p_off >= d.n) {
-                *err = "resident order is corrupt";
-                return SPH_ERR_STATE;
-            }
-        for (int a = 0; a < 2; ++a) {
-            float *out = a ? vel4 : pos4;
-            if (!out) continue;
-            CK(hipMemcpy(buf.data(), (a ? d_.vel : d_.pos) + d.p_off, sizeof(float4) * d.n,
-                         hipMemcpyDeviceToHost), a ? "download velocities" : "download positions");
-            float4 *o4 = reinterpret_cast<float4 *>(out);
-            for (uint32_t k = 0; k < d.n; ++k) o4[ids[k] - d.p_off] = buf[k];
-        }
-    }
-    if (dens2) {
-        if (!have_tables_) {
-            memset(dens2, 0, sizeof(float) * 2 * d.n);
-            return SPH_OK;
-        }
-        // particle order through the repack staging where it exists (its
-        // capacity float4s hold the capacity float2s), else a buffer of its own
-        float2 *tmp = reinterpret_cast<float2 *>(tmp_pos_);
-        if (!tmp) CK(hipMalloc((void **)&tmp, sizeof(float2) * d_.capacity), "density staging");
-        hipError_t e1 = launch_unpermute_dens(d_, tmp, stream_);
-        hipError_t e2 = e1 == hipSuccess ? hipStreamSynchronize(stream_) : e1;
-        hipError_t e3 = e2 == hipSuccess ? hipMemcpy(dens2, tmp + d.p_off, sizeof(float2) * d.n,
-                                                     hipMemcpyDeviceToHost)
-                                         : e2;
-        if (tmp != reinterpret_cast<float2 *>(tmp_pos_)) (void)hipFree(tmp);
-        CK(e3, "download densities");
-    }
+    if (pos4) CK(hipMemcpy(pos4, pos, sizeof(float4) * d.n, hipMemcpyDeviceToHost), "download positions");
+    if (vel4) CK(hipMemcpy(vel4, vel, sizeof(float4) * d.n, hipMemcpyDeviceToHost), "download velocities");
+    if (from_tables) CK(hipMemcpy(dens2, dens, sizeof(float2) * d.n, hipMemcpyDeviceToHost), "download densities");
+    else if (dens2) memset(dens2, 0, sizeof(float) * 2 * d.n);
     return SPH_OK;
 }
 

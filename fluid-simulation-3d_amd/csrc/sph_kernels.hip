@@ -1851,14 +1851,23 @@ static_assert(gather_wave_words(true, true, false) <= kMaskTabWords &&
 // ---------------------------------------------------------------------------
 // Download / parity helpers (not on the step path)
 // ---------------------------------------------------------------------------
-__global__ void k_unpermute_dens(const EngineDesc *__restrict__ ed,
-                                 const uint32_t *__restrict__ svals,
-                                 const float4 *__restrict__ dens, float2 *__restrict__ out)
+__global__ void k_download(const float4 *__restrict__ pos, const float4 *__restrict__ vel,
+                           const uint32_t *__restrict__ ids, const float4 *__restrict__ dens,
+                           const uint32_t *__restrict__ sids, uint32_t off, uint32_t n,
+                           float4 *__restrict__ out_pos, float4 *__restrict__ out_vel,
+                           float2 *__restrict__ out_dens)
 {
-    const uint32_t n = ed->n_total;
-    for (uint32_t k = global_id(); k < n; k += grid_stride()) {
-        const float4 d = dens[k];
-        out[svals[k]] = make_float2(d.x, d.y);
+    for (uint32_t k = off + global_id(); k < off + n; k += grid_stride()) {
+        const uint32_t q = ids[k] - off;  // ids and sids of the scene lie in [off, off + n)
+        if (q < n) {
+            if (out_pos) out_pos[q] = pos[k];
+            if (out_vel) out_vel[q] = vel[k];
+        }
+        if (out_dens) {
+            const uint32_t r = sids[k] - off;
+            const float4 d = dens[k];
+            if (r < n) out_dens[r] = make_float2(d.x, d.y);
+        }
     }
 }
 
@@ -2177,9 +2186,10 @@ uint32_t fused_update_grid(bool multi, int device)
     return (uint32_t)(per_cu * cus) & ~7u;
 }
 
-hipError_t launch_unpermute_dens(const DevState &s, float2 *out, hipStream_t st)
+hipError_t launch_download(const DevState &s, uint32_t off, uint32_t n, float4 *pos, float4 *vel, float2 *dens,
+                           hipStream_t st)
 {
-    k_unpermute_dens<<<grid_for(s.capacity, 256), 256, 0, st>>>(s.ed, s.sids, s.dens, out);
+    k_download<<<grid_for(n, 256), 256, 0, st>>>(s.pos, s.vel, s.ids, s.dens, s.sids, off, n, pos, vel, dens);
     SPH_LAUNCH_CHECK();
 }
 

@@ -64,7 +64,7 @@ struct DevState {
     uint32_t *nbr;       // [(capacity + 1) * nbr_words] neighbour rows by work index (nbr mode); one spare
     uint32_t nbr_words;  // words per particle of nbr
     uint32_t *ncnt;      // [capacity] neighbour count per row
-    uint32_t *scan_err;  // [1] raised when a bounded wait gave up (count scan, grid barrier)
+    uint32_t *scan_err;  // [1] (host memory in an engine) raised when a bounded wait gave up (count scan, grid barrier)
     uint32_t *fbar;      // [kFusedBarWords] grid barrier of the fused update (zero between launches)
     uint32_t fused_grid; // workgroups of the fused update that the device holds resident at once
     uint32_t capacity;       // particle slots allocated
@@ -202,8 +202,11 @@ hipError_t launch_coop_density(const DevState &s, uint32_t n, hipStream_t st);
 hipError_t launch_coop_pressure(const DevState &s, uint32_t n, hipStream_t st);
 hipError_t launch_coop_viscosity_integrate(const DevState &s, uint32_t n, hipStream_t st);
 
-// Sorted -> particle order densities (rho, rho_near) for download.
-hipError_t launch_unpermute_dens(const DevState &s, float2 *out, hipStream_t st);
+// Particles off .. off + n - 1 (one scene) into particle order: positions and
+// velocities from the resident slots [off, off + n), densities (rho, rho_near)
+// from the sorted ones; a null destination is left out.
+hipError_t launch_download(const DevState &s, uint32_t off, uint32_t n, float4 *pos, float4 *vel, float2 *dens,
+                           hipStream_t st);
 // Resident slots [off, off + n) of one scene (particles off .. off + n - 1)
 // into particle order: dst_pos[i] / dst_vel[i] = state of particle off + i.
 hipError_t launch_unpermute_state(const DevState &s, uint32_t off, uint32_t n, float4 *dst_pos,

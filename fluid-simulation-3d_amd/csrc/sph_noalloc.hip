@@ -227,10 +227,9 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     NA(sph::launch_density(s, c, st), "density");
     NA(sph::launch_pressure(s, c, st), "pressure");
     NA(sph::launch_viscosity_integrate(out, c, st), "viscosity + integrate");
-    NA(sph::launch_unpermute_state(out, 0, n, reinterpret_cast<float4 *>(pos4_out),
-                                   reinterpret_cast<float4 *>(vel4_out), st),
-       "unpermute state");
-    if (dens2_out) NA(sph::launch_unpermute_dens(out, reinterpret_cast<float2 *>(dens2_out), st), "densities");
+    NA(sph::launch_download(out, 0, n, reinterpret_cast<float4 *>(pos4_out), reinterpret_cast<float4 *>(vel4_out),
+                            reinterpret_cast<float2 *>(dens2_out), st),
+       "particle order");
     if (!wait) return SPH_OK;
     NA(hipStreamSynchronize(st), "sync");
     uint32_t flag = 0;
