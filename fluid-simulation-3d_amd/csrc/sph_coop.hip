@@ -340,6 +340,7 @@ struct CoopArgs {
     const uint32_t *bounds;
     const uint32_t *sflags;
     uint32_t *ncnt;
+    uint32_t *clear;  // counts to clear for the next update (table_total + n_scenes), or null
 };
 
 template <uint32_t G, bool MULTI, bool GRID, typename T>
@@ -350,6 +351,10 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_density(const CoopArgs A
     __shared__ uint2 lists[Group<G>::kParticles][kList + 1];                // (slot, d2)
     __shared__ __align__(16) float terms[Group<G>::kParticles][2][kChunk];  // the two sums' terms
     const uint32_t n = A.ed->n_total, k = coop_slot<G>(n);
+    if (A.clear) {
+        const uint32_t nc = A.ed->table_total + A.ed->n_scenes;
+        for (uint32_t i = blockIdx.x * kCoopBlock + threadIdx.x; i < nc; i += gridDim.x * kCoopBlock) A.clear[i] = 0u;
+    }
     if (k >= n) return;
     const uint32_t gl = threadIdx.x & (G - 1u), gq = threadIdx.x / G;
     uint2 *const lst = lists[gq];
@@ -497,6 +502,11 @@ struct CoopState {  // what the viscosity stage writes (see k_viscosity_integrat
     uint32_t *ids;
     float4 *rpos, *colors;
     uint32_t *keys, *ticks, *count, *wkeys;
+    // the state in particle order (sph_update_noalloc), or null; with them the
+    // resident state and the next update's buckets (pos .. wkeys) are not written
+    float4 *out_pos, *out_vel;
+    float2 *out_dens;
+    const float4 *dens;
 };
 
 template <uint32_t G, bool MULTI, bool GRID, typename T>
@@ -524,6 +534,15 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_viscosity(const CoopArgs
         float4 x, v;
         integrate_particle(S, vi, group_bcast<G, 0>(f), group_bcast<G, 1>(f), group_bcast<G, 2>(f), x0, x, v);
         if (gl != 0u) return;
+        if (W.out_pos) {
+            W.out_pos[g] = x;
+            W.out_vel[g] = v;
+            if (W.out_dens) {
+                const float4 d = W.dens[k];
+                W.out_dens[g] = make_float2(d.x, d.y);
+            }
+            return;
+        }
         W.pos[k] = x;
         W.vel[k] = v;
         W.ids[k] = g;
@@ -539,6 +558,7 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_viscosity(const CoopArgs
         if (W.wkeys) W.wkeys[k] = work_key(*A.ed, S, S.index, P.cx, P.cy, P.cz);
     };
     if (k < n) run_scene<MULTI>(A.sd, A.scene_of, k, scene);
+    if (W.out_pos) return;
     // the tickets of the workgroup's particles, by one lane each: one atomic
     // per run of equal buckets
     __syncthreads();
@@ -569,7 +589,7 @@ static_assert(kCoopWide <= 65536u, "16-bit rows");
 
 CoopArgs coop_args(const DevState &s)
 {
-    return CoopArgs{s.ed, s.sd, s.scene_of, s.sids, s.xps, s.bounds, s.sflags, s.ncnt};
+    return CoopArgs{s.ed, s.sd, s.scene_of, s.sids, s.xps, s.bounds, s.sflags, s.ncnt, nullptr};
 }
 
 // Rows of nbr_words words per particle: whole groups of entries.
@@ -600,9 +620,10 @@ Rows<T> coop_rows(const DevState &s)
 
 }  // namespace
 
-hipError_t launch_coop_density(const DevState &s, uint32_t n, hipStream_t st)
+hipError_t launch_coop_density(const DevState &s, uint32_t n, bool clear_counts, hipStream_t st)
 {
-    const CoopArgs a = coop_args(s);
+    CoopArgs a = coop_args(s);
+    if (clear_counts) a.clear = s.count;
     SPH_COOP_LAUNCH(k_coop_density, n, st, s.dens);
     return hipGetLastError();
 }
@@ -618,7 +639,23 @@ hipError_t launch_coop_viscosity_integrate(const DevState &s, uint32_t n, hipStr
 {
     const CoopArgs a = coop_args(s);
     const CoopState w{s.vs2, s.ps,     s.pos,     s.vel,     s.ids,   s.rpos,
-                      s.colors, s.keys[0], s.keys[1], s.count, s.grid ? nullptr : s.wkeys[0]};
+                      s.colors, s.keys[0], s.keys[1], s.count, s.grid ? nullptr : s.wkeys[0],
+                      nullptr,  nullptr,   nullptr,   nullptr};
+    SPH_COOP_LAUNCH(k_coop_viscosity, n, st, w);
+    return hipGetLastError();
+}
+
+hipError_t launch_coop_viscosity_out(const DevState &s, uint32_t n, float4 *pos, float4 *vel, float2 *dens,
+                                     hipStream_t st)
+{
+    const CoopArgs a = coop_args(s);
+    CoopState w{};
+    w.vs2 = s.vs2;
+    w.ps = s.ps;
+    w.out_pos = pos;
+    w.out_vel = vel;
+    w.out_dens = dens;
+    w.dens = s.dens;
     SPH_COOP_LAUNCH(k_coop_viscosity, n, st, w);
     return hipGetLastError();
 }

@@ -311,7 +311,16 @@ int Engine::alloc(uint32_t cap, uint32_t tcap, std::string *err)
     d_.capacity = cap;
     d_.table_capacity = tcap;
     int rc = 0;
-    if (!rc) rc = check(hipHostMalloc((void **)&ed_h_, sizeof(EngineDesc)), "pinned desc", err);
+    // the engine descriptor's host copy, and behind it the scan error flag: host
+    // memory that the kernels write, read after a synchronisation without a copy
+    if (!rc) rc = check(hipHostMalloc((void **)&ed_h_, 2 * sizeof(EngineDesc)), "pinned desc", err);
+    if (!rc) {
+        scan_err_h_ = reinterpret_cast<uint32_t *>(ed_h_ + 1);
+        *scan_err_h_ = 0;
+        void *dev = nullptr;
+        rc = check(hipHostGetDevicePointer(&dev, ed_h_, 0), "scan error flag", err);
+        d_.scan_err = reinterpret_cast<uint32_t *>(static_cast<EngineDesc *>(dev) + 1);
+    }
     if (!rc) rc = dm((void **)&d_ed_, sizeof(EngineDesc), "engine desc");
     if (!rc) rc = dm((void **)&d_sd_, sizeof(SceneDesc) * scene_cap_, "scene table");
     for (int q = 0; q < kDescRing && !rc; ++q) {
@@ -349,11 +358,6 @@ int Engine::alloc(uint32_t cap, uint32_t tcap, std::string *err)
     d_.nbr_words = kNbrWords;
     if (!rc) rc = dm((void **)&d_.ncnt, u4, "neighbour counts");
     if (!rc) rc = dm((void **)&d_.sflags, sizeof(uint32_t) * scene_cap_, "scene flags");
-    // in host memory that the kernels write: read after a synchronisation without a copy
-    if (!rc) rc = check(hipHostMalloc((void **)&scan_err_h_, sizeof(uint32_t)), "scan error flag", err);
-    if (!rc) *scan_err_h_ = 0;
-    if (!rc)
-        rc = check(hipHostGetDevicePointer((void **)&d_.scan_err, scan_err_h_, 0), "scan error flag", err);
     if (!rc) rc = dm((void **)&d_.fbar, sizeof(uint32_t) * kFusedBarWords, "grid barrier");
     if (!rc) rc = check(hipMemset(d_.fbar, 0, sizeof(uint32_t) * kFusedBarWords), "grid barrier", err);
     // wrapped until a predict pass says otherwise
@@ -382,7 +386,6 @@ Engine::~Engine()
     if (colors_buf_) (void)hipFree(colors_buf_);
     if (rpos_) (void)hipFree(rpos_);
     if (ed_h_) (void)hipHostFree(ed_h_);
-    if (scan_err_h_) (void)hipHostFree(scan_err_h_);
     for (int q = 0; q < kDescRing; ++q) {
         if (desc_ring_[q]) (void)hipHostFree(desc_ring_[q]);
         if (desc_ev_[q]) (void)hipEventDestroy(desc_ev_[q]);
@@ -1091,6 +1094,7 @@ int Engine::device_status(int s, std::string *err)
 int Engine::set_scan_spin(uint32_t sleeps, std::string *err)
 {
     ed_h_->scan_spin = sleeps;
+    invalidate_graph();
     return push_descs(err);
 }
 

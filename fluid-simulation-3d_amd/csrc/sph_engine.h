@@ -144,6 +144,9 @@ class Engine {
     {
         LaunchCfg c = grid_ ? limit_launch_cfg(cfg_, all_fast_) : cfg_;
         c.coop_n = coop_slots_now();
+        // (set_scan_spin is about the scan's waits, which the one-launch sort has none of)
+        c.small_sort = c.coop_n && small_sort_ok(d_.multi, d_.capacity, d_.table_capacity) &&
+                       ed_h_->scan_spin == kScanSpinDefault;
         return c;
     }
     int set_use_graph(bool on) { use_graph_ = on; invalidate_graph(); return 0; }

@@ -90,6 +90,27 @@ __global__ void k_predict(const EngineDesc *__restrict__ ed, const SceneDesc *__
     }
 }
 
+// The same for one scene in particle order whose descriptors come with the
+// call: they are written to device memory for the kernels that follow.  The
+// counts are zero.
+__global__ void k_predict_first(const EngineDesc E, const SceneDesc S, EngineDesc *__restrict__ ed,
+                                SceneDesc *__restrict__ sd, const float4 *__restrict__ pos,
+                                const float4 *__restrict__ vel, uint32_t *__restrict__ keys,
+                                uint32_t *__restrict__ ticks, uint32_t *__restrict__ count)
+{
+    if (global_id() == 0) {
+        *ed = E;
+        *sd = S;
+    }
+    for (uint32_t g0 = blockIdx.x * blockDim.x; g0 < E.n_total; g0 += grid_stride()) {
+        const uint32_t g = g0 + threadIdx.x;
+        const bool valid = g < E.n_total;
+        Predicted P{};
+        if (valid) P = predict_particle(S, pos[g], vel[g]);
+        record_bucket(E, S, P, valid, g, keys, ticks, count, nullptr);
+    }
+}
+
 // count[0, n) <- 0: the counts and flags of a recorded update that will not run.
 __global__ void k_count_clear(uint32_t *__restrict__ count, uint32_t n)
 {
@@ -454,6 +475,94 @@ __global__ void k_count_scatter(const EngineDesc *__restrict__ ed,
 constexpr uint32_t kRankDirect = 64;
 constexpr uint32_t kReorderBlock = 256;
 
+// Sorted arrays that the reorder writes.
+struct Sorted {
+    uint32_t *sids;
+    float4 *xps, *vs, *ps;
+    uint32_t *rank;
+};
+
+// The records at places t (< end) of `order`, one per work-item of the whole
+// workgroup: bucket_of(key, lo, hi) gives the places [lo, hi) of a bucket.
+template <bool MULTI, typename BucketOf>
+__device__ __forceinline__ void reorder_tile(uint32_t t, uint32_t end, uint32_t n, const SceneDesc *__restrict__ sd,
+                                             const uint32_t *__restrict__ scene_of,
+                                             const uint32_t *__restrict__ keys, const uint2 *order,
+                                             const float4 *__restrict__ vel, const float4 *__restrict__ pos,
+                                             const Sorted &out, BucketOf &&bucket_of)
+{
+    __shared__ uint32_t tile[kReorderBlock];
+    __shared__ uint32_t next_key;
+    const uint32_t B = kReorderBlock, tid = threadIdx.x;
+    uint2 o = make_uint2(n, 0u);  // (resident slot, particle index)
+    if (t < end) o = order[t];
+    const bool have = o.x < n;    // always, while the counts start at zero
+    float4 x0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v0 = x0;
+    uint32_t key = 0, lo = 0, hi = 0;
+    if (have) {
+        x0 = pos[o.x];  // in flight during the bucket count
+        v0 = vel[o.x];
+        key = keys[o.x];
+        bucket_of(key, lo, hi);
+    }
+    const bool big = have && hi > lo && hi - lo > kRankDirect;
+    uint32_t before = 0;
+    if (have && !big) {
+        // the bucket's records four at a time, all four loads issued
+        // before any compare (past hi the load repeats record j and is not
+        // counted)
+        for (uint32_t j = lo; j < hi; j += 4) {
+            uint32_t y[4];
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) y[q] = order[j + q < hi ? j + q : j].y;
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) before += (j + q < hi && y[q] < o.y) ? 1u : 0u;
+        }
+    }
+    if (__syncthreads_or(big)) {
+        bool pending = big;
+        for (;;) {
+            // the next large bucket of this workgroup (the smallest key left)
+            if (tid == 0) next_key = 0xffffffffu;
+            __syncthreads();
+            if (pending) atomicMin(&next_key, key);
+            __syncthreads();
+            const uint32_t bk = next_key;
+            if (bk == 0xffffffffu) break;
+            uint32_t blo, bhi;
+            bucket_of(bk, blo, bhi);
+            const bool mine = pending && key == bk;
+            for (uint32_t j0 = blo; j0 < bhi; j0 += B) {
+                const uint32_t m = min(B, bhi - j0);
+                __syncthreads();  // the previous tile is consumed
+                if (tid < m) tile[tid] = order[j0 + tid].y;
+                __syncthreads();
+                if (mine) {
+                    uint32_t c0 = 0, c1 = 0;
+                    uint32_t q = 0;
+                    for (; q + 1 < m; q += 2) {
+                        c0 += tile[q] < o.y ? 1u : 0u;
+                        c1 += tile[q + 1] < o.y ? 1u : 0u;
+                    }
+                    if (q < m) c0 += tile[q] < o.y ? 1u : 0u;
+                    before += c0 + c1;
+                }
+            }
+            pending = pending && !mine;
+        }
+    }
+    if (!have) return;
+    const uint32_t slot = lo + before;
+    if (slot >= hi) return;  // as above
+    const SceneDesc &S = scene_of_slot<MULTI>(sd, scene_of, o.x);
+    const Predicted P = predict_particle(S, x0, v0);
+    out.sids[slot] = o.y;
+    out.xps[slot] = make_float4(P.px, P.py, P.pz, (float)P.hash);
+    out.vs[slot] = make_float4(P.vx, P.vy, P.vz, v0.w);
+    out.ps[slot] = make_float4(x0.x, x0.y, x0.z, __uint_as_float(P.hash));
+    if (out.rank) out.rank[o.y] = slot;  // only the Morton work order reads it
+}
+
 // Workgroup b of nblk (of kReorderBlock work-items) of the reorder.
 template <bool MULTI>
 __device__ __forceinline__ void reorder_blocks(
@@ -465,80 +574,15 @@ __device__ __forceinline__ void reorder_blocks(
     uint32_t *__restrict__ rank, uint32_t *__restrict__ count, uint64_t *__restrict__ chain,
     uint32_t chain_words)
 {
-    __shared__ uint32_t tile[kReorderBlock];
-    __shared__ uint32_t next_key;
     const uint32_t n = ed->n_total, B = blockDim.x, tid = threadIdx.x;
+    const Sorted out{sids, xps, vs, ps, rank};
     // whole workgroups iterate together (the cooperative rank synchronises)
-    for (uint32_t t0 = b * B; t0 < n; t0 += nblk * B) {
-        const uint32_t t = t0 + tid;
-        uint2 o = make_uint2(n, 0u);  // (resident slot, particle index)
-        if (t < n) o = order[t];
-        const bool have = o.x < n;    // always, while the counts start at zero
-        float4 x0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v0 = x0;
-        uint32_t key = 0, lo = 0, hi = 0;
-        if (have) {
-            x0 = pos[o.x];  // in flight during the bucket count
-            v0 = vel[o.x];
-            key = keys[o.x];
-            lo = bounds[key];
-            hi = min(bounds[key + 1], n);
-        }
-        const bool big = have && hi > lo && hi - lo > kRankDirect;
-        uint32_t before = 0;
-        if (have && !big) {
-            // the bucket's records four at a time, all four loads issued
-            // before any compare (past hi the load repeats record j and is not
-            // counted)
-            for (uint32_t j = lo; j < hi; j += 4) {
-                uint32_t y[4];
-#pragma unroll
-                for (uint32_t q = 0; q < 4; ++q) y[q] = order[j + q < hi ? j + q : j].y;
-#pragma unroll
-                for (uint32_t q = 0; q < 4; ++q) before += (j + q < hi && y[q] < o.y) ? 1u : 0u;
-            }
-        }
-        if (__syncthreads_or(big)) {
-            bool pending = big;
-            for (;;) {
-                // the next large bucket of this workgroup (the smallest key left)
-                if (tid == 0) next_key = 0xffffffffu;
-                __syncthreads();
-                if (pending) atomicMin(&next_key, key);
-                __syncthreads();
-                const uint32_t bk = next_key;
-                if (bk == 0xffffffffu) break;
-                const uint32_t blo = bounds[bk], bhi = min(bounds[bk + 1], n);
-                const bool mine = pending && key == bk;
-                for (uint32_t j0 = blo; j0 < bhi; j0 += B) {
-                    const uint32_t m = min(B, bhi - j0);
-                    __syncthreads();  // the previous tile is consumed
-                    if (tid < m) tile[tid] = order[j0 + tid].y;
-                    __syncthreads();
-                    if (mine) {
-                        uint32_t c0 = 0, c1 = 0;
-                        uint32_t q = 0;
-                        for (; q + 1 < m; q += 2) {
-                            c0 += tile[q] < o.y ? 1u : 0u;
-                            c1 += tile[q + 1] < o.y ? 1u : 0u;
-                        }
-                        if (q < m) c0 += tile[q] < o.y ? 1u : 0u;
-                        before += c0 + c1;
-                    }
-                }
-                pending = pending && !mine;
-            }
-        }
-        if (!have) continue;
-        const uint32_t slot = lo + before;
-        if (slot >= hi) continue;  // as above
-        const SceneDesc &S = scene_of_slot<MULTI>(sd, scene_of, o.x);
-        const Predicted P = predict_particle(S, x0, v0);
-        sids[slot] = o.y;
-        xps[slot] = make_float4(P.px, P.py, P.pz, (float)P.hash);
-        vs[slot] = make_float4(P.vx, P.vy, P.vz, v0.w);
-        ps[slot] = make_float4(x0.x, x0.y, x0.z, __uint_as_float(P.hash));
-        if (rank) rank[o.y] = slot;  // only the Morton work order reads it
-    }
+    for (uint32_t t0 = b * B; t0 < n; t0 += nblk * B)
+        reorder_tile<MULTI>(t0 + tid, n, n, sd, scene_of, keys, order, vel, pos, out,
+                            [&](uint32_t key, uint32_t &lo, uint32_t &hi) {
+                                lo = bounds[key];
+                                hi = min(bounds[key + 1], n);
+                            });
     const uint32_t nc = ed->table_total + ed->n_scenes;
     for (uint32_t i = b * B + tid; i < nc; i += nblk * B) count[i] = 0u;
     for (uint32_t i = b * B + tid; i < chain_words; i += nblk * B) chain[i] = 0u;
@@ -556,6 +600,202 @@ __global__ __launch_bounds__(kReorderBlock) void k_count_reorder(
 {
     reorder_blocks<MULTI>(blockIdx.x, gridDim.x, ed, sd, scene_of, keys, bounds, order, sids, vel, pos, xps,
                           vs, ps, rank, count, chain, chain_words);
+}
+
+// The whole bucket sort of a small scene by one launch: workgroup b owns a
+// contiguous range of buckets, finds its particles -- and how many lie before
+// them, instead of a look-back chain -- by reading every key, and ranks and
+// writes them.  What bounds a sort of this size is the chain of
+// dependent loads, each some 600 ns (the data come from other XCDs): the scan,
+// scatter and reorder launches make about twelve and start three times, this
+// one makes four (12.6 -> 10.3 us of kernel time at 16,384 particles, 9.9 ->
+// 7.1 at 1,000) -- counts and
+// keys together, then ticket, index, position and velocity of the particles found, whose ranks are taken in LDS.  Each workgroup reads all keys, so it
+// is kept to kSmallSortMax particles.  A workgroup with more than kSmallOwn particles
+// (compressed fluid, tiny tables) puts them in ticket order in `order` and
+// runs the reorder over them.  The counts stay as they are (other workgroups
+// read them): the density pass that follows clears them.  ids null: the
+// resident order is particle order.
+constexpr uint32_t kFlight = 8;                                // 16-byte loads in flight per work-item
+constexpr uint32_t kSmallPer = 16;                             // buckets per work-item
+constexpr uint32_t kSmallBuckets = kSmallPer * kReorderBlock;  // most buckets per workgroup
+constexpr uint32_t kSmallWave = 256;                           // particles that a wave lists
+constexpr uint32_t kSmallOwn = kSmallWave * kSortWaves;        // particles ranked in LDS
+static_assert(kReorderBlock == kSortBlock, "one block scan");
+
+__global__ __launch_bounds__(kReorderBlock) void k_small_sort(
+    const EngineDesc *__restrict__ ed, const SceneDesc *__restrict__ sd, const uint32_t *__restrict__ keys,
+    const uint32_t *__restrict__ ticks, const uint32_t *__restrict__ ids, const uint32_t *__restrict__ count,
+    uint32_t *__restrict__ bounds, uint32_t *__restrict__ sflags, uint2 *order, const float4 *__restrict__ vel,
+    const float4 *__restrict__ pos, const Sorted out, uint32_t buckets, uint32_t n, uint32_t T)
+{
+    __shared__ uint32_t lb[kSmallBuckets + 1];  // places of the own buckets
+    __shared__ uint32_t wsum[kSortWaves], wbefore[kSortWaves];
+    __shared__ uint2 own[kSortWaves][kSmallWave + 1];  // (resident slot, bucket - b0) of the own particles; the
+                                                       // last of a wave's: not own
+    __shared__ uint32_t index[kSmallOwn];              // particle index by place
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+    const uint32_t b0 = min(T, blockIdx.x * buckets), b1 = min(T, b0 + buckets);  // b0: a multiple of 4, or T
+    const uint32_t per = (buckets + kReorderBlock - 1) / kReorderBlock;           // <= kSmallPer
+    const uint4 *const k4 = reinterpret_cast<const uint4 *>(keys);
+    const uint32_t nk4 = n / 4;
+    // which 16 bytes of keys a work-item reads: a workgroup's particles are
+    // nearly consecutive in the resident order, and this spreads them over the
+    // waves' lists
+    const uint32_t at4 = lane * kSortWaves + w;
+    // the first keys and the own counts in flight together
+    uint4 k[kFlight];
+#pragma unroll
+    for (uint32_t q = 0; q < kFlight; ++q)
+        k[q] = nk4 ? k4[min(at4 + q * kReorderBlock, nk4 - 1u)] : make_uint4(~0u, ~0u, ~0u, ~0u);
+    uint32_t c[kSmallPer], mine = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kSmallPer; ++j) {
+        if (j >= per) {
+            c[j] = 0;
+            continue;
+        }
+        const uint32_t b = b0 + tid * per + j;
+        c[j] = count[min(b, T)];  // (count[T] exists: the scene flags)
+        c[j] = b < b1 ? c[j] : 0u;
+    }
+    // The own particles are listed in any order, each wave its own list (past
+    // kSmallWave they are only counted); `before` counts the keys of the
+    // buckets before b0.  No lane-dependent branch round the ballots: see
+    // coop_walk.
+    uint32_t before = 0, listed = 0;
+    auto list = [&](uint32_t g, uint32_t d, bool hit) {
+        const uint64_t hits = __ballot(hit);
+        if (hits == 0) return;
+        const uint32_t at = listed + __builtin_amdgcn_mbcnt_hi((uint32_t)(hits >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)hits, 0u));
+        own[w][hit ? min(at, kSmallWave) : kSmallWave] = make_uint2(g, d);
+        listed += (uint32_t)__popcll(hits);
+    };
+    const uint32_t width = b1 - b0;
+    for (uint32_t i0 = 0; i0 < nk4; i0 += kFlight * kReorderBlock) {
+#pragma unroll
+        for (uint32_t q = 0; q < kFlight; ++q) {
+            if (i0 + q * kReorderBlock >= nk4) break;
+            const uint32_t i = i0 + q * kReorderBlock + at4;
+            const bool valid = i < nk4;
+            const uint4 u = k[q];
+            if (valid) before += (u.x < b0) + (u.y < b0) + (u.z < b0) + (u.w < b0);
+            const uint32_t d0 = u.x - b0, d1 = u.y - b0, d2 = u.z - b0, d3 = u.w - b0;
+            if (__ballot(valid & (min(min(d0, d1), min(d2, d3)) < width)) == 0) continue;
+            list(4 * i, d0, valid & (d0 < width));
+            list(4 * i + 1, d1, valid & (d1 < width));
+            list(4 * i + 2, d2, valid & (d2 < width));
+            list(4 * i + 3, d3, valid & (d3 < width));
+        }
+        if (i0 + kFlight * kReorderBlock >= nk4) break;
+#pragma unroll
+        for (uint32_t q = 0; q < kFlight; ++q)
+            k[q] = k4[min(i0 + (kFlight + q) * kReorderBlock + at4, nk4 - 1u)];
+    }
+    if (tid < 64u && 4u * nk4 < n) {  // up to three more
+        const uint32_t g = 4u * nk4 + tid;
+        const uint32_t key = keys[min(g, n - 1u)];
+        before += g < n && key < b0 ? 1u : 0u;
+        list(g, key - b0, g < n && key - b0 < width);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kSmallPer; ++j) mine += c[j];
+    // one scan: exclusive prefix of the own counts, and the sum of those before
+    uint32_t x = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off, 64);
+        if (lane >= (uint32_t)off) x += y;
+        before += __shfl_xor(before, off, 64);
+    }
+    if (lane == 63u) {
+        wsum[w] = x;
+        wbefore[w] = before;
+    }
+    __syncthreads();
+    uint32_t first = 0, total = 0, p = x - mine;
+    for (uint32_t q = 0; q < kSortWaves; ++q) {
+        first += wbefore[q];
+        total += wsum[q];
+        p += q < w ? wsum[q] : 0u;
+    }
+    p += first;
+#pragma unroll
+    for (uint32_t j = 0; j < kSmallPer; ++j) {
+        const uint32_t b = b0 + tid * per + j;
+        if (j < per && b < b1) {
+            const uint32_t at = min(p, n);
+            lb[b - b0] = at;
+            bounds[b] = at;
+        }
+        p += c[j];
+    }
+    first = min(first, n);
+    const uint32_t end = min(first + total, n);
+    if (tid == 0) {
+        lb[b1 - b0] = end;
+        if (b1 == T) bounds[T] = end;
+        if (blockIdx.x == 0)
+            for (uint32_t q = 0; q < ed->n_scenes; ++q) sflags[q] = count[T + q];
+    }
+    if (total == 0) return;  // (the whole workgroup)
+    const bool small = !__syncthreads_or(listed > kSmallWave);
+    if (!small) {
+        for (uint32_t g = tid; g < n; g += kReorderBlock) {
+            const uint32_t d = keys[g] - b0;
+            if (d < width) {
+                const uint32_t slot = lb[d] + ticks[g];
+                if (slot < n) order[slot] = make_uint2(g, ids ? ids[g] : g);
+            }
+        }
+        __syncthreads();  // this workgroup's places are read by itself only
+        for (uint32_t t0 = first; t0 < end; t0 += kReorderBlock) {
+            reorder_tile<false>(t0 + tid, end, n, sd, nullptr, keys, order, vel, pos, out,
+                                [&](uint32_t key, uint32_t &lo, uint32_t &hi) {
+                                    const uint32_t d = min(key - b0, width - 1u);
+                                    lo = lb[d];
+                                    hi = lb[d + 1];
+                                });
+            __syncthreads();  // the cooperative rank's shared values are read
+        }
+        return;
+    }
+    constexpr uint32_t E = kSmallWave / 64u;
+    uint32_t d[E], id[E];
+    float4 x0[E], v0[E];
+#pragma unroll
+    for (uint32_t q = 0; q < E; ++q) {
+        const uint32_t t = lane + 64u * q;
+        d[q] = 0;
+        id[q] = 0;
+        if (t < listed) {
+            const uint2 o = own[w][t];
+            const uint32_t tick = ticks[o.x];
+            id[q] = ids ? ids[o.x] : o.x;
+            x0[q] = pos[o.x];
+            v0[q] = vel[o.x];
+            d[q] = o.y;
+            const uint32_t at = lb[o.y] + tick - first;
+            if (at < kSmallOwn) index[at] = id[q];
+        }
+    }
+    __syncthreads();
+    const SceneDesc &S = sd[0];
+#pragma unroll
+    for (uint32_t q = 0; q < E; ++q) {
+        if (lane + 64u * q >= listed) break;
+        const uint32_t lo = lb[d[q]], hi = lb[d[q] + 1];
+        uint32_t slot = lo;
+        for (uint32_t j = lo; j < hi; ++j) slot += index[j - first] < id[q] ? 1u : 0u;
+        if (slot >= hi) continue;
+        const Predicted P = predict_particle(S, x0[q], v0[q]);
+        out.sids[slot] = id[q];
+        out.xps[slot] = make_float4(P.px, P.py, P.pz, (float)P.hash);
+        out.vs[slot] = make_float4(P.vx, P.vy, P.vz, v0[q].w);
+        out.ps[slot] = make_float4(x0[q].x, x0[q].y, x0[q].z, __uint_as_float(P.hash));
+        if (out.rank) out.rank[id[q]] = slot;  // only the Morton work order reads it
+    }
 }
 
 // Resident slots [0, n) of one scene into particle order:
@@ -2030,6 +2270,14 @@ hipError_t launch_predict(const DevState &s, const LaunchCfg &c, hipStream_t st)
     SPH_LAUNCH_CHECK();
 }
 
+hipError_t launch_predict_first(const DevState &s, const EngineDesc &e, const SceneDesc &d, hipStream_t st)
+{
+    k_predict_first<<<grid_for(e.n_total, 256), 256, 0, st>>>(e, d, const_cast<EngineDesc *>(s.ed),
+                                                              const_cast<SceneDesc *>(s.sd), s.pos, s.vel, s.keys[0],
+                                                              s.keys[1], s.count);
+    SPH_LAUNCH_CHECK();
+}
+
 hipError_t launch_radix_sort(const DevState &s, uint32_t *const keys[2], uint32_t *const vals[2],
                              const uint32_t *first_vals, uint32_t bits, hipStream_t st,
                              int *result_buf)
@@ -2052,6 +2300,18 @@ hipError_t launch_radix_sort(const DevState &s, uint32_t *const keys[2], uint32_
 
 hipError_t launch_bucket_sort(const DevState &s, const LaunchCfg &c, hipStream_t st)
 {
+    if (c.small_sort) {
+        // enough workgroups that each places about one tile of particles
+        const uint32_t want = max(16u, min(512u, s.capacity / 64u));
+        uint32_t buckets = ((s.table_capacity + want - 1) / want + 3u) & ~3u;
+        buckets = min(buckets, kSmallBuckets);
+        const uint32_t g = (s.table_capacity + buckets - 1) / buckets;
+        const Sorted out{s.sids, s.xps, s.vs, s.ps, s.grid ? nullptr : s.rank};
+        k_small_sort<<<g, kReorderBlock, 0, st>>>(s.ed, s.sd, s.keys[0], s.keys[1], s.ids, s.count, s.bounds,
+                                                  s.sflags, s.order, s.vel, s.pos, out, buckets, s.capacity,
+                                                  s.table_capacity);
+        SPH_LAUNCH_CHECK();
+    }
     const uint32_t nb = s.count_blocks, g = grid_for(s.capacity, c.block_stream);
     k_count_scan<<<nb, kSortBlock, 0, st>>>(s.ed, s.count, s.chain, s.bounds, s.sflags,
                                              s.scan_err);
@@ -2118,7 +2378,7 @@ inline uint32_t gather_grid(uint32_t cap, int block)
 
 hipError_t launch_density(const DevState &s, const LaunchCfg &c, hipStream_t st)
 {
-    if (c.coop_n) return launch_coop_density(s, c.coop_n, st);
+    if (c.coop_n) return launch_coop_density(s, c.coop_n, c.small_sort, st);
     if (c.nbr && s.grid) {
         // the density pass records the neighbour masks
         const int b = c.density.block;

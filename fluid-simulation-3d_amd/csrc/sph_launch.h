@@ -97,6 +97,9 @@ struct LaunchCfg {
     // > 0: the gathers run with sixteen work-items per particle, over a grid
     // of this many slots (by_size, set per update by the engine)
     uint32_t coop_n = 0;
+    // the bucket sort is one launch, and the density pass clears its counts
+    // (with coop_n only; small_sort_ok, set per update by the engine)
+    bool small_sort = false;
     int block_stream = 256;  // threads per block of streaming kernels
     bool needs_work() const { return nbr || density.work || pressure.work || viscosity.work; }
 };
@@ -146,6 +149,7 @@ inline LaunchCfg limit_launch_cfg(LaunchCfg c, bool all_fast)
 {
     if (!all_fast) {
         c.coop_n = 0;
+        c.small_sort = false;
         c.fused = c.nbr = false;
         c.density.rows = c.pressure.rows = c.viscosity.rows = false;
     }
@@ -171,9 +175,24 @@ inline uint32_t coop_slots(bool grid, uint32_t n, uint32_t capacity)
     return n > most ? 0u : (capacity < most ? capacity : most);
 }
 
+// The one-launch bucket sort (k_small_sort) for one scene of n particles and
+// `table` buckets.  Every workgroup reads all keys, so above some 20,000
+// particles the three launches are faster.  us per steady update with three
+// launches / with one: 1,000: 25.9 / 21.9, 4,000: 28.1 / 24.9, 10,000: 31.6 /
+// 29.5, 16,384: 33.6 / 32.6, 24,000: 37.7 / 38.4, 50,000: 52.9 / 58.5.  The
+// table's limit is what 16 workgroups' buckets in LDS cover.
+constexpr uint32_t kSmallSortMax = 16384, kSmallSortTable = 65536;
+inline bool small_sort_ok(bool multi, uint32_t n, uint32_t table)
+{
+    return !multi && n <= kSmallSortMax && table <= kSmallSortTable;
+}
+
 // Stage A + B1 when the previous update did not record the buckets: clears
 // the counts, then predict, cell, hash, bucket key and ticket of every particle.
 hipError_t launch_predict(const DevState &s, const LaunchCfg &c, hipStream_t st);
+// The same for one scene in particle order (ids not read), counts at zero, its
+// descriptors written to s.ed and s.sd by the kernel.
+hipError_t launch_predict_first(const DevState &s, const EngineDesc &e, const SceneDesc &d, hipStream_t st);
 // A steady update (buckets recorded by the previous one) as one launch of
 // s.fused_grid persistent workgroups: count scan, scatter, reorder, density,
 // pressure, viscosity+integrate, separated by grid barriers.  Grid key with
@@ -198,9 +217,13 @@ hipError_t launch_viscosity_integrate(const DevState &s, const LaunchCfg &c, hip
 
 // The same stages with sixteen work-items per particle (sph_coop.hip), over the
 // first n slots (n >= the live particles).
-hipError_t launch_coop_density(const DevState &s, uint32_t n, hipStream_t st);
+hipError_t launch_coop_density(const DevState &s, uint32_t n, bool clear_counts, hipStream_t st);
 hipError_t launch_coop_pressure(const DevState &s, uint32_t n, hipStream_t st);
 hipError_t launch_coop_viscosity_integrate(const DevState &s, uint32_t n, hipStream_t st);
+// Its last stage writing the new state (and, unless null, the densities) in
+// particle order only: no resident state, no buckets of a next update.
+hipError_t launch_coop_viscosity_out(const DevState &s, uint32_t n, float4 *pos, float4 *vel, float2 *dens,
+                                     hipStream_t st);
 
 // Particles off .. off + n - 1 (one scene) into particle order: positions and
 // velocities from the resident slots [off, off + n), densities (rho, rho_near)

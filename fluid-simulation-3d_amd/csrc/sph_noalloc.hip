@@ -46,6 +46,7 @@ struct Layout {
     size_t pos, vel, xps, vs, vs2, dens, ps;
     size_t keys0, keys1, ids, sids, ncnt, order, nbr;
     size_t total;
+    size_t chain_words;
 };
 
 constexpr Layout make_layout()
@@ -63,6 +64,7 @@ constexpr Layout make_layout()
     L.sd = take(sizeof(SceneDesc));
     L.scan_err = take(sizeof(uint32_t));
     L.sflags = take(sizeof(uint32_t));
+    L.chain_words = chain_words;
     L.chain = take(sizeof(uint64_t) * chain_words);
     L.bounds = take(sizeof(uint32_t) * (T + 1));
     L.count = take(sizeof(uint32_t) * (T + 1));  // the buckets, then one scene flag
@@ -103,6 +105,20 @@ __global__ void k_write_descs(const EngineDesc e, const SceneDesc d, EngineDesc 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 unsigned char *g_scratch[kMaxDevices] = {};
+bool g_dirty[kMaxDevices] = {};  // the bucket counts may not be zero
+
+// Whether the counts of the array at `base` are zero, and from now on `clean`.
+bool scratch_clean(const unsigned char *base, bool clean)
+{
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    bool was = false;
+    for (int d = 0; d < kMaxDevices; ++d)
+        if (g_scratch[d] == base) {
+            was = !g_dirty[d];
+            g_dirty[d] = !clean;
+        }
+    return was;
+}
 
 // The device address of `scratch` on the current device, looked up once per
 // device (with that device current) and kept.
@@ -216,20 +232,43 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     hipError_t e = hipSuccess;
 #define NA(x, what)                                  \
     if ((e = (x)) != hipSuccess) return hip_fail(e, what)
-    k_write_descs<<<1, 64, 0, st>>>(E, D, at<EngineDesc>(base, kLayout.ed), at<SceneDesc>(base, kLayout.sd));
-    NA(hipGetLastError(), "descriptors");
-    // the scan's chunk status words must start at zero (the reorder of every
-    // call clears them again; this covers a call cut short before it)
-    NA(sph::launch_clear_words(reinterpret_cast<uint32_t *>(s.chain), 2 * (cb + 1), st), "clear chain");
-    NA(sph::launch_iota(s.ids, n, 0, st), "resident order");
-    NA(sph::launch_predict(s, c, st), "predict");  // clears the counts first
-    NA(sph::launch_bucket_sort(s, c, st), "bucket sort");
-    NA(sph::launch_density(s, c, st), "density");
-    NA(sph::launch_pressure(s, c, st), "pressure");
-    NA(sph::launch_viscosity_integrate(out, c, st), "viscosity + integrate");
-    NA(sph::launch_download(out, 0, n, reinterpret_cast<float4 *>(pos4_out), reinterpret_cast<float4 *>(vel4_out),
-                            reinterpret_cast<float2 *>(dens2_out), st),
-       "particle order");
+    // The counts are zero when the previous call on this GPU left them so (it
+    // enqueued all its launches and none of them recorded a next update's buckets).
+    const bool clean = scratch_clean(base, false);
+    if (c.coop_n) {
+        if (!clean) {
+            NA(sph::launch_clear_words(s.count, kNoAllocMaxBuckets + 1, st), "clear counts");
+            NA(sph::launch_clear_words(reinterpret_cast<uint32_t *>(s.chain), 2 * (kLayout.chain_words), st),
+               "clear chain");
+        }
+        // five launches: predict, sort (one to three), density, pressure and
+        // viscosity, which writes the caller's particle order
+        NA(sph::launch_predict_first(s, E, D, st), "predict");
+        c.small_sort = sph::small_sort_ok(false, n, T);
+        if (c.small_sort) s.ids = nullptr;  // particle order
+        else NA(sph::launch_iota(s.ids, n, 0, st), "resident order");
+        NA(sph::launch_bucket_sort(s, c, st), "bucket sort");
+        NA(sph::launch_density(s, c, st), "density");
+        NA(sph::launch_pressure(s, c, st), "pressure");
+        NA(sph::launch_coop_viscosity_out(s, c.coop_n, reinterpret_cast<float4 *>(pos4_out),
+                                          reinterpret_cast<float4 *>(vel4_out),
+                                          reinterpret_cast<float2 *>(dens2_out), st),
+           "viscosity + integrate");
+        scratch_clean(base, true);
+    } else {
+        k_write_descs<<<1, 64, 0, st>>>(E, D, at<EngineDesc>(base, kLayout.ed), at<SceneDesc>(base, kLayout.sd));
+        NA(hipGetLastError(), "descriptors");
+        NA(sph::launch_clear_words(reinterpret_cast<uint32_t *>(s.chain), 2 * (cb + 1), st), "clear chain");
+        NA(sph::launch_iota(s.ids, n, 0, st), "resident order");
+        NA(sph::launch_predict(s, c, st), "predict");  // clears the counts first
+        NA(sph::launch_bucket_sort(s, c, st), "bucket sort");
+        NA(sph::launch_density(s, c, st), "density");
+        NA(sph::launch_pressure(s, c, st), "pressure");
+        NA(sph::launch_viscosity_integrate(out, c, st), "viscosity + integrate");
+        NA(sph::launch_download(out, 0, n, reinterpret_cast<float4 *>(pos4_out),
+                                reinterpret_cast<float4 *>(vel4_out), reinterpret_cast<float2 *>(dens2_out), st),
+           "particle order");
+    }
     if (!wait) return SPH_OK;
     NA(hipStreamSynchronize(st), "sync");
     uint32_t flag = 0;

@@ -63,6 +63,26 @@ def test_dense_bitexact(n, spacing, key):
     _check(W.scene_params(box=(6.0, 6.0, 6.0)), pos, vel, S.TABLE_GRID if key == "grid" else n, updates=1)
 
 
+# the one-launch sort: tables of a few buckets (thousands of records each), not a multiple of the workgroups'
+# ranges, and on both sides of its limit
+@pytest.mark.parametrize("n,table", [(3000, 1), (3000, 7), (9001, 4097), (9001, 65535), (9001, 65536), (9001, 65537),
+                                     (16384, 65536), (16384, 30011), (16385, 65536)])
+def test_sort_tables_bitexact(n, table):
+    announce("small sort", n, table)
+    L = 0.1 * (4 * n) ** (1.0 / 3.0) + 1.0
+    pos, vel = _lattice(n, 0.1, (L, L, L))
+    p = W.scene_params(box=(L, L, L))
+    _check(p, pos, vel, table, updates=4)
+    with S.Sim(p, n, table) as sim:
+        sim.upload(pos, vel)
+        sim.update(_sub_dt())
+        got = sim.debug_spatial()
+    _, xp = O.predict(orc_params(p), _sub_dt(), pos, vel)
+    want = O.spatial(xp, table, p.smoothing_radius)
+    for k in ("hash_id", "key_id", "sorted_idx", "start"):
+        np.testing.assert_array_equal(got[k], getattr(want, k))
+
+
 @pytest.mark.parametrize("counts", [(5, 1, 130, 64, 4000), (9000, 7, 12345, 3)])
 @pytest.mark.parametrize("reference", [False, True])
 def test_scene_boundaries_bitexact(counts, reference):
@@ -101,3 +121,25 @@ def test_variants_changed_between_updates_bitexact(key):
     assert_bitexact(got[0][:, :3], want[0][:, :3], "positions")
     assert_bitexact(got[1][:, :3], want[1][:, :3], "velocities")
     assert_bitexact(got[2], want[2], "densities")
+
+
+def test_noalloc_sizes_and_sparse_boxes_bitexact():
+    """sph_update_noalloc over its forms of the sort (a small table, a table past the one-launch sort's limit) and a
+    radius that takes the walking kernels, in turn: each call leaves the shared scratch as the next one needs it."""
+    import test_zz_no_alloc as N
+    hip = N._Hip()
+    cases = [(1000, 0.2, 4.0), (5000, 0.2, 9.0), (20000, 0.2, 8.0), (5000, 2.0 ** -18, 2.0 ** -12), (5000, 0.2, 12.0),
+             (1, 0.2, 4.0), (65536, 0.2, 8.0)]
+    for n, h, box in cases:
+        announce("noalloc", n, h, box)
+        pos, vel = S.generate(S.INIT_DAM_BREAK, n, n, (box,) * 3, 0.5 * h, 0.005 * h)
+        p = W.scene_params(h=h, rho0=8.0 / h ** 3, box=(box,) * 3)
+        p.prefilter_r2 = 2.0 * h * h
+        p.pressure_mult, p.near_pressure_mult = 300.0 * (h / 0.2) ** 2, 20.0 * (h / 0.2) ** 2
+        p.gravity_scale = 9.81 * h / 0.2
+        sc = W.Scene("noalloc", p, n, n, pos, vel, 1)
+        got = N._noalloc(hip, sc, _sub_dt(), wait=n % 2)
+        want = O.update(orc_params(p), _sub_dt(), pos, vel, T=n)
+        assert_bitexact(got[0][:, :3], want[0][:, :3], "positions")
+        assert_bitexact(got[1][:, :3], want[1][:, :3], "velocities")
+        assert_bitexact(got[2], want[2], "densities")
