@@ -323,11 +323,11 @@ __device__ __forceinline__ float ordered_sum(float acc, const float *plane, uint
 }
 
 // Rows of the neighbour lists: entry t of slot k at [k * cap + t], 16-bit slots
-// while every slot fits (the row then holds twice as many); one row more, spare.
+// while every slot fits (the row then holds twice as many).
 template <typename T>
 struct Rows {
-    T *rows;
-    uint32_t cap, spare;
+    T *rows, *spare;  // spare: a row that nobody reads
+    uint32_t cap;
     __device__ __forceinline__ uint32_t get(uint32_t k, uint32_t t) const { return rows[(size_t)k * cap + t]; }
 };
 
@@ -381,7 +381,8 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_density(const CoopArgs A
                     density_pair<true>(h, w2c, w3c, __uint_as_float(e.y), true, a, b);
                     t0p[r + gl] = have ? a : 0.0f;
                     t1p[r + gl] = have ? b : 0.0f;
-                    out.rows[(size_t)(cnt ? k : out.spare) * out.cap + min(total + at, out.cap - 1u)] = (T)e.x;
+                    T *const row = cnt ? out.rows + (size_t)k * out.cap : out.spare;
+                    row[min(total + at, out.cap - 1u)] = (T)e.x;
                 }
                 wave_sync();
                 acc = ordered_sum(acc, gl == 0u ? t0p : t1p, cnt > c0 ? min(kChunk, cnt - c0) : 0u);
@@ -597,7 +598,7 @@ template <typename T>
 Rows<T> coop_rows(const DevState &s)
 {
     const uint32_t cap = s.nbr_words * (uint32_t)(sizeof(uint32_t) / sizeof(T));
-    return Rows<T>{reinterpret_cast<T *>(s.nbr), cap < 128u ? cap & ~15u : 128u, s.capacity};
+    return Rows<T>{reinterpret_cast<T *>(s.nbr), reinterpret_cast<T *>(s.spare), cap < 128u ? cap & ~15u : 128u};
 }
 
 // Launches KER<G, MULTI, GRID, T> over n particle slots.

@@ -354,8 +354,9 @@ int Engine::alloc(uint32_t cap, uint32_t tcap, std::string *err)
         if (!rc) rc = dm((void **)&d_.wvals[b], u4, "work order");
     }
     if (!rc) rc = dm((void **)&d_.rank, u4, "rank");
-    if (!rc) rc = dm((void **)&d_.nbr, (u4 + sizeof(uint32_t)) * kNbrWords, "neighbour rows");  // one row spare
+    if (!rc) rc = dm((void **)&d_.nbr, u4 * kNbrWords, "neighbour rows");
     d_.nbr_words = kNbrWords;
+    d_.spare = d_.hist;  // (the radix sort's, which the forms that need a spare row do not run)
     if (!rc) rc = dm((void **)&d_.ncnt, u4, "neighbour counts");
     if (!rc) rc = dm((void **)&d_.sflags, sizeof(uint32_t) * scene_cap_, "scene flags");
     if (!rc) rc = dm((void **)&d_.fbar, sizeof(uint32_t) * kFusedBarWords, "grid barrier");

@@ -61,8 +61,9 @@ struct DevState {
     float4 *rpos;        // [capacity] render positions, particle order (null: not written)
     uint32_t *sflags;    // [scenes] grid key: 1 when a particle's cell lies outside the grid's box
                          // (copied from the count flags by the bucket sort)
-    uint32_t *nbr;       // [(capacity + 1) * nbr_words] neighbour rows by work index (nbr mode); one spare
+    uint32_t *nbr;       // [capacity * nbr_words] neighbour rows by work index (nbr mode)
     uint32_t nbr_words;  // words per particle of nbr
+    uint32_t *spare;     // at least nbr_words words that are written and never read
     uint32_t *ncnt;      // [capacity] neighbour count per row
     uint32_t *scan_err;  // [1] (host memory in an engine) raised when a bounded wait gave up (count scan, grid barrier)
     uint32_t *fbar;      // [kFusedBarWords] grid barrier of the fused update (zero between launches)

@@ -217,6 +217,7 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     s.sflags = at<uint32_t>(base, kLayout.sflags);
     s.nbr = at<uint32_t>(base, kLayout.nbr);
     s.nbr_words = kNoAllocNbrWords;
+    s.spare = at<uint32_t>(base, kLayout.pos);  // (the walking forms' only)
     s.ncnt = at<uint32_t>(base, kLayout.ncnt);
     s.scan_err = at<uint32_t>(base, kLayout.scan_err);
     s.capacity = n;
