@@ -160,7 +160,8 @@ class Engine {
     int alloc(uint32_t capacity, uint32_t table_capacity, std::string *err);
     int push_descs(std::string *err);
     int set_dt(float dt, std::string *err);
-    hipError_t enqueue_update(hipEvent_t *ev, bool rebuild_work, bool fresh, bool mark_predict = true);
+    hipError_t enqueue_update(hipEvent_t *ev, bool rebuild_work, bool fresh, bool mark_predict = true,
+                              bool shown = true);
     // Resident slots of scene s into particle order (ids[k] = p_off + k).
     hipError_t normalize_scene(uint32_t s);
     // Render positions of scene s from its current state (if they exist).

@@ -355,7 +355,7 @@ class Sim:
         _check(lib().sph_initialize(self._h, int(kind), int(seed), _ptr(b), spacing, jitter, speed))
 
     def set_colors(self, stops=None, enable=True):
-        """Render hand-off: speed colours written by every update."""
+        """Render hand-off: speed colours written by every update, and by the last one of a step."""
         st = None if stops is None else np.ascontiguousarray(stops, np.float32).reshape(16)
         _check(lib().sph_set_colors(self._h, _ptr(st), 1 if enable else 0))
 
