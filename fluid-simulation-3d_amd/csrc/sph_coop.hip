@@ -281,7 +281,7 @@ __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__re
         const uint32_t dx = o / 9u - 1u, dy = (o / 3u) % 3u - 1u, dz = o % 3u - 1u;
         uint32_t key;
         if constexpr (GRID)
-            key = S.key_off + grid_key(cx + (int)dx, cy + (int)dy, cz + (int)dz, S.cell_lo, S.gdim, S.gmod);
+            key = S.key_off + grid_key(cx + (int)dx, cy + (int)dy, cz + (int)dz, S.cell_lo, S.gdim, S.gmod, S.strip_shift);
         else
             key = S.key_off + fastmod(cell_hash(o), S.mod_m, S.table);
         m0 = bounds[key];

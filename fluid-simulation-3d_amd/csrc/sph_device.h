@@ -43,13 +43,26 @@ SPH_HD uint32_t fastmod(uint32_t a, uint64_t m, uint32_t table)
 // (u32(c) - u32(lo)) wrapping mod 2^32.  For c in [lo, lo + G) this is c - lo.
 SPH_HD uint32_t grid_wrap(uint32_t u, uint32_t g, uint64_t m) { return u < g ? u : fastmod(u, m, g); }
 
+// Bucket order of the grid key: the z cells of row (wx, wy) are consecutive
+// buckets, and the rows go through the grid in strips of 2^strip_shift rows in
+// y, by plane (wx) within a strip and by wy within a plane; the last strip takes
+// what is left of gy.  With kNoStrips, or any strip of gy rows or more, that is
+// wx * gy + wy.
+constexpr uint32_t kNoStrips = 31;
+SPH_HD uint32_t grid_row(uint32_t wx, uint32_t wy, uint32_t gx, uint32_t gy, uint32_t strip_shift)
+{
+    const uint32_t y0 = (wy >> strip_shift) << strip_shift, left = gy - y0;
+    const uint32_t rows = left < (1u << strip_shift) ? left : 1u << strip_shift;
+    return y0 * gx + (wy - y0) + wx * rows;
+}
+
 SPH_HD uint32_t grid_key(int32_t cx, int32_t cy, int32_t cz, const int32_t lo[3],
-                         const uint32_t g[3], const uint64_t m[3])
+                         const uint32_t g[3], const uint64_t m[3], uint32_t strip_shift)
 {
     const uint32_t wx = grid_wrap((uint32_t)cx - (uint32_t)lo[0], g[0], m[0]);
     const uint32_t wy = grid_wrap((uint32_t)cy - (uint32_t)lo[1], g[1], m[1]);
     const uint32_t wz = grid_wrap((uint32_t)cz - (uint32_t)lo[2], g[2], m[2]);
-    return (wx * g[1] + wy) * g[2] + wz;
+    return grid_row(wx, wy, g[0], g[1], strip_shift) * g[2] + wz;
 }
 
 // Render colour of a particle from its velocity: FluidSimCPU::updateColors

@@ -162,6 +162,8 @@ void fill_scene_desc(const sph_params &p, uint32_t n, uint32_t table, bool grid,
         d->gdim[0] = d->gdim[1] = d->gdim[2] = 1;
     }
     for (int c = 0; c < 3; ++c) d->gmod[c] = fastmod_constant(d->gdim[c]);
+    d->strip_shift = grid_strips(n, d->gdim);
+    d->pad = 0;
 }
 
 void work_key_layout(uint32_t n_scenes, EngineDesc *e)
@@ -1192,6 +1194,27 @@ int Engine::debug_spatial(uint32_t s, uint32_t *hash_id, uint32_t *key_id, uint3
        "sorted idx");
     CK(hipMemcpy(bd.data(), d_.bounds + d.key_off, sizeof(uint32_t) * ((size_t)d.table + 1),
                  hipMemcpyDeviceToHost), "bucket bounds");
+    if (d.grid && d.strip_shift != kNoStrips) {
+        // the buckets in the key's own order (sph_get_key), not in strips
+        std::vector<float4> ps0(d.n);
+        std::vector<uint32_t> si0(d.n), bd0((size_t)d.table + 1);
+        const uint64_t cells = (uint64_t)d.gdim[0] * d.gdim[1] * d.gdim[2];
+        uint32_t at = 0;
+        for (uint32_t b = 0; b <= d.table; ++b) {
+            bd0[b] = d.p_off + at;
+            if (b >= cells) continue;  // (a bucket that no cell has, or the end)
+            const uint32_t row = b / d.gdim[2];
+            const uint32_t from = grid_row(row / d.gdim[1], row % d.gdim[1], d.gdim[0], d.gdim[1], d.strip_shift) *
+                                      d.gdim[2] + b % d.gdim[2];
+            for (uint32_t k = bd[from]; k < bd[from + 1] && k - d.p_off < d.n && at < d.n; ++k, ++at) {
+                ps0[at] = ps[k - d.p_off];
+                si0[at] = si[k - d.p_off];
+            }
+        }
+        ps.swap(ps0);
+        si.swap(si0);
+        bd.swap(bd0);
+    }
     for (uint32_t b = 0; b < d.table; ++b)
         for (uint32_t k = bd[b]; k < bd[b + 1]; ++k)
             if (k - d.p_off < d.n) sk[k - d.p_off] = b;

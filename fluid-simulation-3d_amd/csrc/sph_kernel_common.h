@@ -135,7 +135,7 @@ __device__ __forceinline__ uint32_t bucket_key(const EngineDesc &E, const SceneD
                    (uint32_t)P.cy - (uint32_t)S.cell_lo[1] >= S.gdim[1] ||
                    (uint32_t)P.cz - (uint32_t)S.cell_lo[2] >= S.gdim[2]))
         count[E.table_total + S.index] = 1u;
-    return S.key_off + (S.grid ? grid_key(P.cx, P.cy, P.cz, S.cell_lo, S.gdim, S.gmod)
+    return S.key_off + (S.grid ? grid_key(P.cx, P.cy, P.cz, S.cell_lo, S.gdim, S.gmod, S.strip_shift)
                                : fastmod(P.hash, S.mod_m, S.table));
 }
 

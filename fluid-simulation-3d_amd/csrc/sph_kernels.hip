@@ -1140,7 +1140,7 @@ __device__ __forceinline__ uint32_t walk_grid(const SceneDesc &S, const float4 *
     auto fetch = [&](int r) {
         const uint32_t wx = grid_wrap(ux + (uint32_t)(r / 3 - 1), S.gdim[0], S.gmod[0]);
         const uint32_t wy = grid_wrap(uy + (uint32_t)(r % 3 - 1), gy, S.gmod[1]);
-        const uint32_t base = key_off + (wx * gy + wy) * gz;
+        const uint32_t base = key_off + grid_row(wx, wy, S.gdim[0], gy, S.strip_shift) * gz;
         if (run) {
             ns[0] = start[base + wz[0]];
             ne[2] = endt[base + wz[2]];
@@ -1404,7 +1404,7 @@ __device__ __forceinline__ void gather_bits(const SceneDesc &S, const float4 *__
     }
     uint32_t rb[9];
 #pragma unroll
-    for (int r = 0; r < 9; ++r) rb[r] = bounds[S.key_off + (wx[r / 3] * gy + wy[r % 3]) * gz + wz0];
+    for (int r = 0; r < 9; ++r) rb[r] = bounds[S.key_off + grid_row(wx[r / 3], wy[r % 3], S.gdim[0], gy, S.strip_shift) * gz + wz0];
     uint64_t rm[9];
     uint32_t off = 0;
 #pragma unroll
@@ -2125,7 +2125,7 @@ __device__ __forceinline__ void walk_prefilter(const SceneDesc &S, const float4 
             for (int dz = -1; dz <= 1; ++dz) {
                 const uint32_t hash = hash_cell(cx + dx, cy + dy, cz + dz);
                 const uint32_t key =
-                    S.key_off + (S.grid ? grid_key(cx + dx, cy + dy, cz + dz, S.cell_lo, S.gdim, S.gmod)
+                    S.key_off + (S.grid ? grid_key(cx + dx, cy + dy, cz + dz, S.cell_lo, S.gdim, S.gmod, S.strip_shift)
                                         : fastmod(hash, S.mod_m, S.table));
                 const uint32_t b = start[key], e = endt[key];
                 const float hf = (float)hash;

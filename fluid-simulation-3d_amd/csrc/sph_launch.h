@@ -176,6 +176,29 @@ inline uint32_t coop_slots(bool grid, uint32_t n, uint32_t capacity)
     return n > most ? 0u : (capacity < most ? capacity : most);
 }
 
+// Rows per strip of the grid key's bucket order, log2 (grid_row), for a scene
+// of n particles.  A gather reads three planes around its own, and an XCD works
+// on a window of some 40,000 slots (32 CUs of 16 to 24 waves).  Once planes hold
+// more than about 24,000 slots (768 KiB of positions and velocities), window
+// and neighbours no longer fit the XCD's 4 MiB L2 and every plane is fetched
+// for each of its neighbours; in strips of eight rows they fit again, for two
+// rows at a strip's edge that are fetched once more.  us of pressure + viscosity
+// per update without strips / with 16 / 8 / 4 rows:
+//   uniform 2,097,152 (21,000 slots a plane)       488 / 476 / 483 / -
+//   two blocks 3,000,000 (26,000, 34,000 inside)   612 / - / 559 / -
+//   two blocks 4,194,304 (32,000, 42,000 inside)   904 / 800 / 798 / 837
+//   uniform 4,194,304 (33,000)                     1,193 / - / 1,047 / -
+//   uniform 8,388,608 (52,000)                     2,474 / 2,277 / 2,219 / 2,490
+//   two blocks 16,777,216 (82,000, 105,000 inside) 3,574 / 3,276 / 3,223 / 3,395
+// (density gains nothing and loses up to 1%).  Scenes that the sixteen- and
+// eight-work-item gathers may take have none: their fast walk counts on rows
+// in plane order.
+constexpr uint32_t kStripPlane = 24576, kStripShift = 3;
+inline uint32_t grid_strips(uint32_t n, const uint32_t g[3])
+{
+    return n > kCoopMaxGrid && n / g[0] > kStripPlane && g[1] > (1u << kStripShift) ? kStripShift : kNoStrips;
+}
+
 // The one-launch bucket sort (k_small_sort) for one scene of n particles and
 // `table` buckets.  Every workgroup reads all keys, so above some 20,000
 // particles the three launches are faster.  us per steady update with three

@@ -54,6 +54,8 @@ struct SceneDesc {
     uint32_t grid;        // bucket key: 1 = cell-grid key, 0 = hash % table (cc:513-516)
     uint32_t gdim[3];     // grid key: period of the cell grid per axis, product <= table
     uint32_t index;       // this scene's position in the layout (per-scene flags)
+    uint32_t strip_shift; // grid key: rows per strip of the bucket order, log2 (grid_row)
+    uint32_t pad;         // (8-byte alignment)
     uint64_t gmod[3];     // grid key: remainder constants of gdim
 };
 

@@ -113,8 +113,9 @@ int sph_get_params(sph_handle h, sph_params *p);
 int sph_get_size(sph_handle h, uint32_t *n, uint32_t *table_size);
 /* Bucket key in use: *grid = 1 for the cell-grid key, with its periods
  * gdim[3] and origin cell lo[3] (key = (wx*Gy + wy)*Gz + wz, w = (u32(cell) -
- * u32(lo)) mod G per axis); *grid = 0 for hash % table_size.  Any output may
- * be NULL.  No reference counterpart (parity tests). */
+ * u32(lo)) mod G per axis; the kernels keep the buckets of large scenes in
+ * another order, which no entry point shows); *grid = 0 for hash % table_size.
+ * Any output may be NULL.  No reference counterpart (parity tests). */
 int sph_get_key(sph_handle h, int32_t *grid, uint32_t gdim[3], int32_t lo[3]);
 /* Writes the positions vector (h:79) and the velocities; either may be NULL
  * (left unchanged).  Host float4 arrays of n entries. */
