@@ -1903,12 +1903,14 @@ __device__ __forceinline__ void pressure_vblock(uint32_t vblock_, SPH_GATHER_PAR
     SPH_GATHER_EPILOGUE();
 }
 
-// The single-scene mask consumer is held to 80 VGPRs (6 waves per SIMD,
-// what the LDS mask table allows; 82 unconstrained, 5 waves): its few spills
-// lie off the take loop (-0.4% to -1.2% in A/B runs).  The multi-scene one
-// keeps its 90 (at 80 its spills cost 5%).
+// Mask consumers, pressure and viscosity: 4 waves per SIMD to the register
+// allocator.  Pressure takes 88 registers for one scene and 96 for several
+// (5 waves), without spilling; held to 80 (6 waves, 13 spilled) it takes 248 us
+// instead of 252 on 1,000,000 colliding particles, the same 103 on 1,048,576
+// uniform ones, and 1,516 instead of 1,453 on 16,777,216, where more waves in
+// flight mean more of the L2 in use.
 template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID>
-__global__ __launch_bounds__(256, (NBR && GRID && !MULTI) ? 6 : 1) void k_pressure(
+__global__ __launch_bounds__(256, NBR && GRID ? 4 : 1) void k_pressure(
     SPH_GATHER_PARAMS, const float4 *__restrict__ dens, const float4 *__restrict__ vs, float4 *__restrict__ vs2)
 {
     pressure_vblock<MULTI, WORK, LIST, NBR, GRID>(blockIdx.x, SPH_GATHER_FWD, dens, vs, vs2);
@@ -1969,10 +1971,9 @@ __device__ __forceinline__ void viscosity_vblock(uint32_t vblock_, SPH_GATHER_PA
     SPH_GATHER_EPILOGUE();
 }
 
-// (5 waves per SIMD: 96 VGPRs, which the single-scene form fits in 76 and
-// the multi-scene form in exactly 96, without spilling)
+// (walking forms: 5 waves per SIMD)
 template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID>
-__global__ __launch_bounds__(256, 5) void k_viscosity_integrate(SPH_GATHER_PARAMS,
+__global__ __launch_bounds__(256, NBR && GRID ? 4 : 5) void k_viscosity_integrate(SPH_GATHER_PARAMS,
                                                                            SPH_VISCOSITY_PARAMS)
 {
     viscosity_vblock<MULTI, WORK, LIST, NBR, GRID>(blockIdx.x, SPH_GATHER_FWD, SPH_VISCOSITY_FWD);

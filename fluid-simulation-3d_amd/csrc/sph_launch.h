@@ -122,7 +122,10 @@ inline LaunchCfg default_launch_cfg(bool grid)
         // the autotuner's usual picks: neighbour masks for all three kernels
         c.density = GatherVariant{false, false, 256, true};
         c.pressure = GatherVariant{false, false, 256, true};
-        c.viscosity = GatherVariant{false, false, 128, true};
+        // (viscosity with workgroups of 128 / 256, us: uniform 1,048,576 113 / 110,
+        // 64 scenes 349 / 333, colliding 1,000,000 164 / 159.5: a workgroup's waves
+        // share more of what the L1 holds; 512 loses on the colliding scene)
+        c.viscosity = GatherVariant{false, false, 256, true};
         c.nbr = true;
     }
     c.by_size = true;
