@@ -572,7 +572,7 @@ __device__ __forceinline__ void reorder_blocks(
     uint32_t *__restrict__ sids, const float4 *__restrict__ vel, const float4 *__restrict__ pos,
     float4 *__restrict__ xps, float4 *__restrict__ vs, float4 *__restrict__ ps,
     uint32_t *__restrict__ rank, uint32_t *__restrict__ count, uint64_t *__restrict__ chain,
-    uint32_t chain_words)
+    uint32_t chain_words, uint32_t *__restrict__ uneven)
 {
     const uint32_t n = ed->n_total, B = blockDim.x, tid = threadIdx.x;
     const Sorted out{sids, xps, vs, ps, rank};
@@ -586,6 +586,10 @@ __device__ __forceinline__ void reorder_blocks(
     const uint32_t nc = ed->table_total + ed->n_scenes;
     for (uint32_t i = b * B + tid; i < nc; i += nblk * B) count[i] = 0u;
     for (uint32_t i = b * B + tid; i < chain_words; i += nblk * B) chain[i] = 0u;
+    if (uneven && b == 0 && tid == 0) {
+        uneven[1] = uneven[0];
+        uneven[0] = 0u;
+    }
 }
 
 template <bool MULTI>
@@ -596,10 +600,10 @@ __global__ __launch_bounds__(kReorderBlock) void k_count_reorder(
     uint32_t *__restrict__ sids, const float4 *__restrict__ vel, const float4 *__restrict__ pos,
     float4 *__restrict__ xps, float4 *__restrict__ vs, float4 *__restrict__ ps,
     uint32_t *__restrict__ rank, uint32_t *__restrict__ count, uint64_t *__restrict__ chain,
-    uint32_t chain_words)
+    uint32_t chain_words, uint32_t *__restrict__ uneven)
 {
     reorder_blocks<MULTI>(blockIdx.x, gridDim.x, ed, sd, scene_of, keys, bounds, order, sids, vel, pos, xps,
-                          vs, ps, rank, count, chain, chain_words);
+                          vs, ps, rank, count, chain, chain_words, uneven);
 }
 
 // The whole bucket sort of a small scene by one launch: workgroup b owns a
@@ -1544,9 +1548,17 @@ constexpr uint32_t kListMax = 56;
 // contiguously), so every XCD gets a sample of every part of the layout --
 // scenes differ in cost per particle (a compressed pool against a falling
 // block), and one XCD per slab would leave the others idle while it ends.
+// SPREAD: one scene, uneven work: each XCD takes kPieces contiguous pieces
+//   instead of one, dealt in turn.  Set while density finds particles without a
+//   usable record (DevState::uneven): fluid compressed past 21 particles a
+//   cell costs several times as much per slot, and lies together.  us of
+//   density + pressure + viscosity with 1 / 2 / 4 / 8 / 16 pieces: colliding
+//   1,000,000 580 / 508 / 429 / 417 / 419, but uniform 1,048,576, where each
+//   piece's edges are read once more, 349 / 349.5 / 355 / 358 / 369.
 constexpr uint32_t kXcdChunk = 128;
+constexpr uint32_t kPieces = 4;
 template <bool WORK, bool GRID, bool MULTI = false>
-__device__ __forceinline__ uint32_t gather_index(uint32_t n, uint32_t b)
+__device__ __forceinline__ uint32_t gather_index(uint32_t n, uint32_t b, bool spread = false)
 {
     if (!WORK && !GRID) return b * blockDim.x + threadIdx.x;
     const uint32_t live = (n + blockDim.x - 1) / blockDim.x;
@@ -1554,10 +1566,10 @@ __device__ __forceinline__ uint32_t gather_index(uint32_t n, uint32_t b)
     uint32_t lb;
     if (j >= per) {
         lb = live + j;
-    } else if (!MULTI) {
+    } else if (!MULTI && !spread) {
         lb = x * per + j;
     } else {
-        const uint32_t C = max(1u, min(kXcdChunk, per >> 3));
+        const uint32_t C = max(1u, MULTI ? min(kXcdChunk, per >> 3) : per / kPieces);
         const uint32_t full = per / C * C;
         lb = j < full ? ((j / C) * 8u + x) * C + j % C : 8u * full + x * (per - full) + (j - full);
     }
@@ -1648,7 +1660,9 @@ __host__ __device__ constexpr uint32_t gather_wave_words(bool grid, bool nbr, bo
 
 #define SPH_GATHER_PROLOGUE()                                                       \
     extern __shared__ uint32_t lds_list[];                                          \
-    const uint32_t i = gather_index<WORK, GRID, MULTI>(ed->n_total, vblock_);      \
+    /* (density raises uneven[0] while it runs: it reads the last update's)  */  \
+    const bool spread_ = GRID && !MULTI && uneven && uneven[CONSUMER ? 0 : 1] != 0u; \
+    const uint32_t i = gather_index<WORK, GRID, MULTI>(ed->n_total, vblock_, spread_); \
     if (i >= ed->n_total) return;                                                   \
     const uint32_t g = WORK ? work[i] : svals[i];                                   \
     const uint32_t k_slot_ = WORK ? rank[g] : i;                                    \
@@ -1688,7 +1702,7 @@ __host__ __device__ constexpr uint32_t gather_wave_words(bool grid, bool nbr, bo
     ;                                                                               \
     run_scene<MULTI>(sd, scene_of, k_slot_, scene_body_)
 
-#define SPH_GATHER_FWD ed, sd, scene_of, work, rank, svals, xps, start, endt, nbr, ncnt, sflags
+#define SPH_GATHER_FWD ed, sd, scene_of, work, rank, svals, xps, start, endt, nbr, ncnt, sflags, uneven
 
 #define SPH_GATHER_PARAMS                                                                     \
     const EngineDesc *__restrict__ ed, const SceneDesc *__restrict__ sd,                      \
@@ -1696,7 +1710,7 @@ __host__ __device__ constexpr uint32_t gather_wave_words(bool grid, bool nbr, bo
         const uint32_t *__restrict__ rank, const uint32_t *__restrict__ svals,                \
         const float4 *__restrict__ xps, const uint32_t *__restrict__ start,                   \
         const uint32_t *__restrict__ endt, uint32_t *__restrict__ nbr,                        \
-        uint32_t *__restrict__ ncnt, const uint32_t *__restrict__ sflags
+        uint32_t *__restrict__ ncnt, const uint32_t *__restrict__ sflags, uint32_t *uneven
 
 // NBR (with WORK): the density pass also stores each particle's neighbours
 // with d < h (self excluded, walk order) as row i = work index of the
@@ -1796,7 +1810,10 @@ __device__ __forceinline__ void density_vblock(uint32_t vblock_, SPH_GATHER_PARA
             rho = rhon = 0.0f;
             attempt();
         }
-        if (!ok) walk<GRID, false, false, false, true>(S, xps, nullptr, start, endt, k, pi, stage, clean, body);
+        if (!ok) {
+            if (!MULTI && uneven) uneven[0] = 1u;
+            walk<GRID, false, false, false, true>(S, xps, nullptr, start, endt, k, pi, stage, clean, body);
+        }
     } else if (GRID && !LIST)
         walk<GRID, false, false, false, true>(S, xps, nullptr, start, endt, k, pi, stage, clean, body);
     else
@@ -2066,23 +2083,23 @@ __global__ __launch_bounds__(kFusedBlock) void k_fused_update(const DevState s)
                   s.order);
     grid_barrier(s.fbar, nwg, s.scan_err);
     reorder_blocks<MULTI>(b, nwg, s.ed, s.sd, s.scene_of, s.keys[0], s.bounds, s.order, s.sids, s.vel, s.pos,
-                          s.xps, s.vs, s.ps, nullptr, s.count, s.chain, s.count_blocks + 1);
+                          s.xps, s.vs, s.ps, nullptr, s.count, s.chain, s.count_blocks + 1, s.uneven);
     grid_barrier(s.fbar, nwg, s.scan_err);
     // the gathers over the virtual workgroups of the capacity's grid
     const uint32_t vblocks = (((s.capacity + kFusedBlock - 1) / kFusedBlock) + 7u) & ~7u;
     const uint32_t *const endt = s.bounds + 1;
     for (uint32_t v = b; v < vblocks; v += nwg)
         density_vblock<MULTI, false, false, true, true>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
-                                                        s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.dens);
+                                                        s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.uneven, s.dens);
     grid_barrier(s.fbar, nwg, s.scan_err);
     for (uint32_t v = b; v < vblocks; v += nwg)
         pressure_vblock<MULTI, false, false, true, true>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
-                                                         s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.dens,
+                                                         s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.uneven, s.dens,
                                                          s.vs, s.vs2);
     grid_barrier(s.fbar, nwg, s.scan_err);
     for (uint32_t v = b; v < vblocks; v += nwg)
         viscosity_vblock<MULTI, false, false, true, true>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
-                                                          s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.vs2,
+                                                          s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.uneven, s.vs2,
                                                           s.ps, s.pos, s.vel, s.ids, s.rpos, s.colors, s.keys[0],
                                                           s.keys[1], s.count, nullptr);
 }
@@ -2329,12 +2346,12 @@ hipError_t launch_bucket_sort(const DevState &s, const LaunchCfg &c, hipStream_t
         k_count_reorder<true><<<gr, kReorderBlock, 0, st>>>(s.ed, s.sd, s.scene_of, s.keys[0],
                                                              s.bounds, s.order, s.sids, s.vel,
                                                              s.pos, s.xps, s.vs, s.ps, rk,
-                                                             s.count, s.chain, nb + 1);
+                                                             s.count, s.chain, nb + 1, s.uneven);
     else
         k_count_reorder<false><<<gr, kReorderBlock, 0, st>>>(s.ed, s.sd, s.scene_of, s.keys[0],
                                                               s.bounds, s.order, s.sids, s.vel,
                                                               s.pos, s.xps, s.vs, s.ps, rk,
-                                                              s.count, s.chain, nb + 1);
+                                                              s.count, s.chain, nb + 1, s.uneven);
     SPH_LAUNCH_CHECK();
 }
 
@@ -2380,7 +2397,7 @@ inline uint32_t gather_grid(uint32_t cap, int block)
 
 #define SPH_GATHER_ARGS                                                                \
     s.ed, s.sd, s.scene_of, s.work, s.rank, s.sids, s.xps, s.bounds, s.bounds + 1, s.nbr, s.ncnt, \
-        s.sflags
+        s.sflags, s.uneven
 
 hipError_t launch_density(const DevState &s, const LaunchCfg &c, hipStream_t st)
 {

@@ -66,6 +66,8 @@ struct DevState {
     uint32_t *spare;     // at least nbr_words words that are written and never read
     uint32_t *ncnt;      // [capacity] neighbour count per row
     uint32_t *scan_err;  // [1] (host memory in an engine) raised when a bounded wait gave up (count scan, grid barrier)
+    uint32_t *uneven;    // [2] nonzero: density found particles without a usable mask record in this update,
+                         // in the last one (gather_index; null: not recorded)
     uint32_t *fbar;      // [kFusedBarWords] grid barrier of the fused update (zero between launches)
     uint32_t fused_grid; // workgroups of the fused update that the device holds resident at once
     uint32_t capacity;       // particle slots allocated

@@ -1,7 +1,7 @@
 """Fluid compressed past what a neighbour record holds, in part of a scene:
-those particles are walked 64 slots of a row at a time.  Single updates equal
-the oracle's bit for bit, updates with recorded buckets equal the reference
-key's."""
+those particles are walked 64 slots of a row at a time, and the XCDs take the
+scene in pieces.  Single updates equal the oracle's bit for bit, updates with
+recorded buckets equal the reference key's."""
 import numpy as np
 import pytest
 
@@ -45,7 +45,7 @@ def test_dense_part(per_cell, outside):
     ref = _oracle(sc, dt)
     announce("dense part", per_cell, outside)
     with S.Sim(sc.params, sc.n, S.TABLE_GRID) as sim:
-        for _ in range(2):
+        for _ in range(2):  # the second time in pieces in every pass
             sim.upload(sc.pos, sc.vel)
             sim.update(dt)
             pos_g, vel_g, dens_g = sim.download()
