@@ -233,9 +233,15 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     hipError_t e = hipSuccess;
 #define NA(x, what)                                  \
     if ((e = (x)) != hipSuccess) return hip_fail(e, what)
-    // The counts are zero when the previous call on this GPU left them so (it
-    // enqueued all its launches and none of them recorded a next update's buckets).
-    const bool clean = scratch_clean(base, false);
+    // Every call's launches leave the counts at zero, so a call clears them only
+    // when one before it on this GPU failed halfway.  Launches recorded into the
+    // caller's graph run later, after calls that this one cannot know: they always
+    // clear first, and recording them says nothing about the counts now.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) (void)hipGetLastError();
+    const bool recorded = cap != hipStreamCaptureStatusNone;
+    const bool were = scratch_clean(base, false);
+    const bool clean = were && !recorded;
     if (c.coop_n) {
         if (!clean) {
             NA(sph::launch_clear_words(s.count, kNoAllocMaxBuckets + 1, st), "clear counts");
@@ -255,7 +261,6 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
                                           reinterpret_cast<float4 *>(vel4_out),
                                           reinterpret_cast<float2 *>(dens2_out), st),
            "viscosity + integrate");
-        scratch_clean(base, true);
     } else {
         k_write_descs<<<1, 64, 0, st>>>(E, D, at<EngineDesc>(base, kLayout.ed), at<SceneDesc>(base, kLayout.sd));
         NA(hipGetLastError(), "descriptors");
@@ -269,7 +274,9 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
         NA(sph::launch_download(out, 0, n, reinterpret_cast<float4 *>(pos4_out),
                                 reinterpret_cast<float4 *>(vel4_out), reinterpret_cast<float2 *>(dens2_out), st),
            "particle order");
+        NA(sph::launch_clear_words(s.count, s.count_size, st), "clear counts");  // (the next update's buckets)
     }
+    scratch_clean(base, were || !recorded);
     if (!wait) return SPH_OK;
     NA(hipStreamSynchronize(st), "sync");
     uint32_t flag = 0;
