@@ -74,11 +74,27 @@ def sub_dt(dt=W.DT, substeps=W.SUBSTEPS):
     return float(np.float32(np.float32(dt) / np.float32(substeps)))
 
 
-def kernel_name(stage, variants, grid, multi=False):
-    """Template instantiation that runs `stage` under the gather variants `variants`
-    (kernel<MULTI, WORK, LIST, NBR, GRID>)."""
+# the default gather variants (work, list, block, rows): with them small scenes
+# run the forms with several work-items per particle
+DEFAULTS = {True: {"density": (0, 0, 256, 1), "pressure": (0, 0, 256, 1), "viscosity": (0, 0, 256, 1), "nbr": 1},
+            False: {"density": (0, 0, 64, 0), "pressure": (1, 1, 64, 0), "viscosity": (0, 0, 64, 0), "nbr": 0}}
+
+
+def is_default(variants, grid):
+    return all(DEFAULTS[grid][k] == (tuple(int(v[x]) for x in ("work", "list", "block", "rows"))
+                                     if isinstance(v, dict) else int(v))
+               for k, v in variants.items() if k in DEFAULTS[grid])
+
+
+def kernel_name(stage, variants, grid, multi=False, n=None):
+    """Template instantiation that runs `stage` for n particles under the gather
+    variants `variants` (kernel<MULTI, WORK, LIST, NBR, GRID>; several work-items
+    per particle: kernel<lanes, MULTI, GRID, list entry>)."""
     m = "true" if multi else "false"
     b = lambda x: "true" if x else "false"  # noqa: E731
+    if n is not None and n <= (1 << 17 if grid else 1 << 20) and is_default(variants, grid):
+        return (f"k_coop_{stage.split('_')[0]}<{16 if n <= 16384 else 8}u, {m}, {b(grid)}, "
+                f"unsigned {'short' if n <= 65536 else 'int'}>")
     if stage == "density" and variants["nbr"] and not grid:
         return f"k_density_rows<{m}>"
     base = {"density": "k_density", "pressure": "k_pressure",
@@ -145,7 +161,7 @@ def gather_fractions(workload, n, variants, grid, per, multi):
     instruction count."""
     out = {}
     for stage in GATHER:
-        kern = kernel_name(stage, variants, grid, multi)
+        kern = kernel_name(stage, variants, grid, multi, n)
         ms = per[stage]
         traffic = measured_traffic(workload, kern)
         valu = valu_issue(workload, kern, ms)
@@ -165,7 +181,7 @@ def roofline(workload, n, variants, grid, per, multi):
     the committed counters show bounds the kernel at its live duration: the
     larger of its VALU issue share and its measured-traffic share of HBM."""
     dom = max(GATHER, key=lambda k: per[k])
-    kern = kernel_name(dom, variants, grid, multi)
+    kern = kernel_name(dom, variants, grid, multi, n)
     ms = per[dom]
     ach = ALG_BYTES[dom] * n / (ms * 1e-3) / 1e9
     traffic = measured_traffic(workload, kern)

@@ -222,9 +222,10 @@ __device__ __forceinline__ PressureSelf pressure_self(const SceneDesc &S, const 
 // The reciprocals are 0 when unusable and >= 2^-26 else, so one minimum over
 // four values and one maximum over two decide (7 instructions, where testing
 // the six terms takes 26): with root_rn, pressure 120 -> 103 us on 1,048,576
-// uniform particles, where the L1 accesses of the neighbour gathers now take
-// the whole time (41 cycles a load, two loads a neighbour).  Pairs that fail it (weak forces, odd units) are
-// tested term by term before IEEE division is taken.
+// uniform particles, where vector issue and the neighbour gathers (two loads a
+// neighbour, 13 million L1 misses a launch) now take about as long as each
+// other.  Pairs that fail it (weak forces, odd units) are tested term by term
+// before IEEE division is taken.
 struct PressureTerms {
     float tx, ty, tz, ux, uy, uz;
 };
