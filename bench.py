@@ -92,7 +92,7 @@ def kernel_name(stage, variants, grid, multi=False, n=None):
     per particle: kernel<lanes, MULTI, GRID, list entry>)."""
     m = "true" if multi else "false"
     b = lambda x: "true" if x else "false"  # noqa: E731
-    if n is not None and n <= (1 << 17 if grid else 1 << 20) and is_default(variants, grid):
+    if n is not None and n <= (1 << 17 if grid else 1 << 24) and is_default(variants, grid):
         return (f"k_coop_{stage.split('_')[0]}<{16 if n <= 16384 else 8}u, {m}, {b(grid)}, "
                 f"unsigned {'short' if n <= 65536 else 'int'}>")
     if stage == "density" and variants["nbr"] and not grid:

@@ -163,15 +163,20 @@ inline LaunchCfg limit_launch_cfg(LaunchCfg c, bool all_fast)
 }
 
 // Largest particle count for which the gathers run with several work-items per
-// particle (sph_coop.hip); above it one work-item per particle fills the chip
-// and tests each candidate cheaper.  Measured, us per steady update (all
-// kernels) with one / several work-items per particle:
+// particle (sph_coop.hip).  Under the grid key one work-item per particle fills
+// the chip above it, and tests each candidate cheaper.  Under the reference key
+// density is cheaper so too, but only several work-items leave lists that
+// pressure and viscosity can read instead of walking, at every size measured;
+// the limit is the last of them, and where the reference's own float indices
+// end.  us per steady update (all kernels; from 1,200,000 on the three gathers)
+// with one / several work-items per particle:
 //   grid key       1,000: 64 / 27   16,384: 77 / 34   65,536: 85 / 60
 //                  131,072: 94 / 94   200,000: 115 / 127
-//   reference key  4,000: 153 / 30   50,000: 195 / 67   200,000: 318 / 184
-//                  1,000,000: 1,018 / 878
+//   reference key  4,000: 153 / 30   50,000: 195 / 64   200,000: 318 / 163
+//                  1,200,000: 1,233 / 1,017   2,000,000: 2,001 / 1,660
+//                  6,000,000: 6,662 / 5,202   16,700,000: 19,477 / 15,160
 constexpr uint32_t kCoopMaxGrid = 1u << 17;
-constexpr uint32_t kCoopMaxReference = 1u << 20;
+constexpr uint32_t kCoopMaxReference = 1u << 24;
 
 // Slots that the sixteen-work-item gathers' grid covers for n particles in a
 // layout of `capacity` slots, or 0 when the one-work-item forms run.

@@ -143,3 +143,20 @@ def test_noalloc_sizes_and_sparse_boxes_bitexact():
         assert_bitexact(got[0][:, :3], want[0][:, :3], "positions")
         assert_bitexact(got[1][:, :3], want[1][:, :3], "velocities")
         assert_bitexact(got[2], want[2], "densities")
+
+
+def test_reference_key_past_a_million():
+    """The lists' forms at a size that only the reference key takes them for, against the walking forms."""
+    n = (1 << 20) + 77
+    sc = W.uniform_lower(n=n, table=2 * n)
+    announce("reference key", n)
+    got = []
+    with S.Sim(sc.params, n, 2 * n) as sim:
+        walk = {"work": 0, "list": 0, "block": 128, "rows": False}
+        for form in (sim.variants, {"density": walk, "pressure": walk, "viscosity": walk, "nbr": 0}):
+            sim.variants = form
+            sim.upload(sc.pos, sc.vel)
+            sim.step(W.DT, 2)
+            got.append(sim.download())
+    for a, b, what in zip(*got, ("positions", "velocities", "densities")):
+        assert_bitexact(a, b, what)
