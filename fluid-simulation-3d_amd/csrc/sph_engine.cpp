@@ -361,10 +361,10 @@ int Engine::alloc(uint32_t cap, uint32_t tcap, std::string *err)
     d_.spare = d_.hist;  // (the radix sort's, which the forms that need a spare row do not run)
     if (!rc) rc = dm((void **)&d_.ncnt, u4, "neighbour counts");
     if (!rc) rc = dm((void **)&d_.sflags, sizeof(uint32_t) * scene_cap_, "scene flags");
-    if (!rc) rc = dm((void **)&d_.fbar, sizeof(uint32_t) * kFusedBarWords, "grid barrier");
-    if (!rc) rc = check(hipMemset(d_.fbar, 0, sizeof(uint32_t) * kFusedBarWords), "grid barrier", err);
-    if (!rc) rc = dm((void **)&d_.uneven, sizeof(uint32_t) * 2, "work balance");
-    if (!rc) rc = check(hipMemset(d_.uneven, 0, sizeof(uint32_t) * 2), "work balance", err);
+    // (the work-balance words lie behind the barrier's: one allocation)
+    if (!rc) rc = dm((void **)&d_.fbar, sizeof(uint32_t) * (kFusedBarWords + 2), "grid barrier");
+    if (!rc) rc = check(hipMemset(d_.fbar, 0, sizeof(uint32_t) * (kFusedBarWords + 2)), "grid barrier", err);
+    d_.uneven = d_.fbar + kFusedBarWords;
     // wrapped until a predict pass says otherwise
     if (!rc) rc = check(hipMemset(d_.sflags, 0xff, sizeof(uint32_t) * scene_cap_), "scene flags", err);
     d_.ed = d_ed_;
@@ -383,7 +383,7 @@ Engine::~Engine()
                     d_.ids,      d_.ps,       d_.order,    d_.sids,
                     d_.hist,     d_.bounds,   d_.count,    d_.chain,
                     d_.wkeys[0], d_.wkeys[1], d_.wvals[0], d_.wvals[1], d_.rank,
-                    d_.nbr,      d_.ncnt,     d_.sflags,   d_.uneven,  d_.fbar};
+                    d_.nbr,      d_.ncnt,     d_.sflags,   d_.fbar};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (tmp_pos_) (void)hipFree(tmp_pos_);
