@@ -610,6 +610,9 @@ int Engine::set_params(uint32_t s, const sph_params &p, std::string *err)
         return SPH_ERR_INVALID;
     }
     recorded_ = false;
+    if (have_tables_ && table_order_.empty())  // debug_spatial reads the tables of the last update
+        for (const SceneDesc &q : sd_h_)
+            table_order_.push_back(TableOrder{{q.gdim[0], q.gdim[1], q.gdim[2]}, q.strip_shift});
     SceneDesc &d = sd_h_[s];
     const float dt = d.dt;
     const uint32_t p_off = d.p_off, k_off = d.key_off;
@@ -791,7 +794,7 @@ int Engine::update(float dt, std::string *err)
         CK(enqueue_update(nullptr, rebuild, fresh), "launch update");
     }
     ++work_updates_;
-    have_tables_ = true;
+    tables_built();
     recorded_ = true;  // for the next update, if nothing changes and dt stays
     return SPH_OK;
 }
@@ -1075,7 +1078,7 @@ int Engine::run_steady(int n, std::string *err)
     }
     CK(hipGraphLaunch(run_exec_, stream_), "graph launch");
     work_updates_ += (uint64_t)n;
-    have_tables_ = true;
+    tables_built();
     recorded_ = true;
     return SPH_OK;
 }
@@ -1143,7 +1146,7 @@ int Engine::prime(std::string *err)
     if (rc) return rc;
     CK(e, "prime");
     if (rc2) return rc2;
-    have_tables_ = true;
+    tables_built();
     return SPH_OK;
 }
 
@@ -1196,18 +1199,20 @@ int Engine::debug_spatial(uint32_t s, uint32_t *hash_id, uint32_t *key_id, uint3
        "sorted idx");
     CK(hipMemcpy(bd.data(), d_.bounds + d.key_off, sizeof(uint32_t) * ((size_t)d.table + 1),
                  hipMemcpyDeviceToHost), "bucket bounds");
-    if (d.grid && d.strip_shift != kNoStrips) {
-        // the buckets in the key's own order (sph_get_key), not in strips
+    const TableOrder t = table_order_.empty() ? TableOrder{{d.gdim[0], d.gdim[1], d.gdim[2]}, d.strip_shift}
+                                              : table_order_[s];
+    if (d.grid && t.strip_shift != kNoStrips) {
+        // the buckets in the order of that update's key (sph_get_key), not in strips
         std::vector<float4> ps0(d.n);
         std::vector<uint32_t> si0(d.n), bd0((size_t)d.table + 1);
-        const uint64_t cells = (uint64_t)d.gdim[0] * d.gdim[1] * d.gdim[2];
+        const uint64_t cells = (uint64_t)t.gdim[0] * t.gdim[1] * t.gdim[2];
         uint32_t at = 0;
         for (uint32_t b = 0; b <= d.table; ++b) {
             bd0[b] = d.p_off + at;
             if (b >= cells) continue;  // (a bucket that no cell has, or the end)
-            const uint32_t row = b / d.gdim[2];
-            const uint32_t from = grid_row(row / d.gdim[1], row % d.gdim[1], d.gdim[0], d.gdim[1], d.strip_shift) *
-                                      d.gdim[2] + b % d.gdim[2];
+            const uint32_t row = b / t.gdim[2];
+            const uint32_t from = grid_row(row / t.gdim[1], row % t.gdim[1], t.gdim[0], t.gdim[1], t.strip_shift) *
+                                      t.gdim[2] + b % t.gdim[2];
             for (uint32_t k = bd[from]; k < bd[from + 1] && k - d.p_off < d.n && at < d.n; ++k, ++at) {
                 ps0[at] = ps[k - d.p_off];
                 si0[at] = si[k - d.p_off];

@@ -201,6 +201,17 @@ class Engine {
     uint32_t *d_scene_of_ = nullptr;
     uint32_t scene_cap_ = 1;
     bool have_tables_ = false;
+    // Per scene, the bucket order that the tables on the device were built in,
+    // where set_params has changed it since; empty while it is sd_h_'s.
+    struct TableOrder {
+        uint32_t gdim[3], strip_shift;
+    };
+    std::vector<TableOrder> table_order_;
+    void tables_built()
+    {
+        have_tables_ = true;
+        table_order_.clear();
+    }
     bool grid_ = false;  // cell-grid bucket key (else the reference's hash % table)
     bool use_graph_ = true;
     // [rebuild work order? + 2 * fresh predict? + 4 * sixteen-work-item gathers?]
