@@ -313,8 +313,9 @@ int Engine::alloc(uint32_t cap, uint32_t tcap, std::string *err)
     d_.capacity = cap;
     d_.table_capacity = tcap;
     int rc = 0;
-    // the engine descriptor's host copy, and behind it the scan error flag: host
-    // memory that the kernels write, read after a synchronisation without a copy
+    // the engine descriptor's host copy, and behind it the scan error flag and
+    // launch_download's: host memory that the kernels write, read after a
+    // synchronisation without a copy
     if (!rc) rc = check(hipHostMalloc((void **)&ed_h_, 2 * sizeof(EngineDesc)), "pinned desc", err);
     if (!rc) {
         scan_err_h_ = reinterpret_cast<uint32_t *>(ed_h_ + 1);
@@ -322,6 +323,8 @@ int Engine::alloc(uint32_t cap, uint32_t tcap, std::string *err)
         void *dev = nullptr;
         rc = check(hipHostGetDevicePointer(&dev, ed_h_, 0), "scan error flag", err);
         d_.scan_err = reinterpret_cast<uint32_t *>(static_cast<EngineDesc *>(dev) + 1);
+        corrupt_h_ = scan_err_h_ + 1;
+        d_corrupt_ = d_.scan_err + 1;
     }
     if (!rc) rc = dm((void **)&d_ed_, sizeof(EngineDesc), "engine desc");
     if (!rc) rc = dm((void **)&d_sd_, sizeof(SceneDesc) * scene_cap_, "scene table");
@@ -1164,13 +1167,21 @@ int Engine::download(uint32_t s, float *pos4, float *vel4, float *dens2, std::st
     float4 *const pos = reinterpret_cast<float4 *>(d_.nbr), *const vel = pos + d.n;
     float2 *const dens = reinterpret_cast<float2 *>(vel + d.n);
     const bool from_tables = dens2 && have_tables_;
+    corrupt_h_[0] = corrupt_h_[1] = 0;  // (no other kernel writes them)
     CK(launch_download(d_, d.p_off, d.n, pos4 ? pos : nullptr, vel4 ? vel : nullptr, from_tables ? dens : nullptr,
-                       stream_), "download order");
+                       d_corrupt_, stream_), "download order");
     CK(hipStreamSynchronize(stream_), "sync before download");
     if (int rc = device_status((int)s, err)) return rc;
+    const volatile uint32_t *const corrupt = corrupt_h_;
+    if (corrupt[0]) {
+        *err = "resident order is corrupt";
+        return SPH_ERR_STATE;
+    }
     if (pos4) CK(hipMemcpy(pos4, pos, sizeof(float4) * d.n, hipMemcpyDeviceToHost), "download positions");
     if (vel4) CK(hipMemcpy(vel4, vel, sizeof(float4) * d.n, hipMemcpyDeviceToHost), "download velocities");
-    if (from_tables) CK(hipMemcpy(dens2, dens, sizeof(float2) * d.n, hipMemcpyDeviceToHost), "download densities");
+    // (the sorted order is corrupt when the last update failed and new state was
+    // uploaded since: no densities, as before any update)
+    if (from_tables && !corrupt[1]) CK(hipMemcpy(dens2, dens, sizeof(float2) * d.n, hipMemcpyDeviceToHost), "download densities");
     else if (dens2) memset(dens2, 0, sizeof(float) * 2 * d.n);
     return SPH_OK;
 }

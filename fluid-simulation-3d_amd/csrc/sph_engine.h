@@ -187,6 +187,7 @@ class Engine {
     std::vector<sph_params> params_;
     EngineDesc *ed_h_ = nullptr;  // host copy of the engine descriptor
     uint32_t *scan_err_h_ = nullptr;  // d_.scan_err, in host memory
+    uint32_t *corrupt_h_ = nullptr, *d_corrupt_ = nullptr;  // [2] behind it: launch_download's
     // Descriptor uploads go through a ring of pinned staging slots (engine
     // descriptor, then the scene table), each reused only after the copies
     // from its previous use have run (its event), so an upload never waits

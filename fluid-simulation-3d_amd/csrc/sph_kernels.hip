@@ -2118,20 +2118,29 @@ __global__ void k_download(const float4 *__restrict__ pos, const float4 *__restr
                            const uint32_t *__restrict__ ids, const float4 *__restrict__ dens,
                            const uint32_t *__restrict__ sids, uint32_t off, uint32_t n,
                            float4 *__restrict__ out_pos, float4 *__restrict__ out_vel,
-                           float2 *__restrict__ out_dens)
+                           float2 *__restrict__ out_dens, uint32_t *__restrict__ corrupt)
 {
+    // ids and sids of the scene lie in [off, off + n); an index of ids that does
+    // not raises corrupt[0], one of sids corrupt[1]
+    bool bad_id = false, bad_sid = false;
     for (uint32_t k = off + global_id(); k < off + n; k += grid_stride()) {
-        const uint32_t q = ids[k] - off;  // ids and sids of the scene lie in [off, off + n)
-        if (q < n) {
-            if (out_pos) out_pos[q] = pos[k];
-            if (out_vel) out_vel[q] = vel[k];
+        if (out_pos || out_vel) {
+            const uint32_t q = ids[k] - off;
+            if (q < n) {
+                if (out_pos) out_pos[q] = pos[k];
+                if (out_vel) out_vel[q] = vel[k];
+            }
+            bad_id |= q >= n;
         }
         if (out_dens) {
             const uint32_t r = sids[k] - off;
             const float4 d = dens[k];
             if (r < n) out_dens[r] = make_float2(d.x, d.y);
+            bad_sid |= r >= n;
         }
     }
+    if (corrupt && bad_id) corrupt[0] = 1u;
+    if (corrupt && bad_sid) corrupt[1] = 1u;
 }
 
 // Same walk as the reference's density loop, but without the d < h cut: the
@@ -2470,9 +2479,9 @@ uint32_t fused_update_grid(bool multi, int device)
 }
 
 hipError_t launch_download(const DevState &s, uint32_t off, uint32_t n, float4 *pos, float4 *vel, float2 *dens,
-                           hipStream_t st)
+                           uint32_t *corrupt, hipStream_t st)
 {
-    k_download<<<grid_for(n, 256), 256, 0, st>>>(s.pos, s.vel, s.ids, s.dens, s.sids, off, n, pos, vel, dens);
+    k_download<<<grid_for(n, 256), 256, 0, st>>>(s.pos, s.vel, s.ids, s.dens, s.sids, off, n, pos, vel, dens, corrupt);
     SPH_LAUNCH_CHECK();
 }
 

@@ -261,9 +261,11 @@ hipError_t launch_coop_viscosity_out(const DevState &s, uint32_t n, float4 *pos,
 
 // Particles off .. off + n - 1 (one scene) into particle order: positions and
 // velocities from the resident slots [off, off + n), densities (rho, rho_near)
-// from the sorted ones; a null destination is left out.
+// from the sorted ones; a null destination is left out.  corrupt[0] / [1] (unless
+// null) are set to 1 when the particle index of a resident / sorted slot lies
+// outside the scene; such a slot is not written.
 hipError_t launch_download(const DevState &s, uint32_t off, uint32_t n, float4 *pos, float4 *vel, float2 *dens,
-                           hipStream_t st);
+                           uint32_t *corrupt, hipStream_t st);
 // Resident slots [off, off + n) of one scene (particles off .. off + n - 1)
 // into particle order: dst_pos[i] / dst_vel[i] = state of particle off + i.
 hipError_t launch_unpermute_state(const DevState &s, uint32_t off, uint32_t n, float4 *dst_pos,

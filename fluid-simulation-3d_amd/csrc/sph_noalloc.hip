@@ -272,7 +272,8 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
         NA(sph::launch_pressure(s, c, st), "pressure");
         NA(sph::launch_viscosity_integrate(out, c, st), "viscosity + integrate");
         NA(sph::launch_download(out, 0, n, reinterpret_cast<float4 *>(pos4_out),
-                                reinterpret_cast<float4 *>(vel4_out), reinterpret_cast<float2 *>(dens2_out), st),
+                                reinterpret_cast<float4 *>(vel4_out), reinterpret_cast<float2 *>(dens2_out), nullptr,
+                                st),
            "particle order");
         NA(sph::launch_clear_words(s.count, s.count_size, st), "clear counts");  // (the next update's buckets)
     }
