@@ -277,7 +277,8 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
            "particle order");
         NA(sph::launch_clear_words(s.count, s.count_size, st), "clear counts");  // (the next update's buckets)
     }
-    scratch_clean(base, were || !recorded);
+    // (the walking form clears its own buckets and chain words only)
+    scratch_clean(base, were || (c.coop_n && !recorded));
     if (!wait) return SPH_OK;
     NA(hipStreamSynchronize(st), "sync");
     uint32_t flag = 0;
