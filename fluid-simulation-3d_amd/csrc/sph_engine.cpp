@@ -261,7 +261,8 @@ int Engine::create(const std::vector<SceneSpec> &scenes, uint32_t capacity,
     e->cfg_ = default_launch_cfg(grid);
     {
         int dev = 0;
-        if (hipGetDevice(&dev) == hipSuccess) e->d_.fused_grid = fused_update_grid(e->d_.multi, dev);
+        if (hipGetDevice(&dev) == hipSuccess)
+            for (int q = 0; q < 2; ++q) e->d_.fused_grid[q] = fused_update_grid(e->d_.multi, q != 0, dev);
     }
     rc = e->check(hipMemcpy(e->d_scene_of_, scene_of.data(), sizeof(uint32_t) * capacity,
                             hipMemcpyHostToDevice),
@@ -424,10 +425,8 @@ int Engine::push_descs(std::string *err)
         *err = "scene capacity exceeded";
         return SPH_ERR_INVALID;
     }
-    bool fast = true;
-    for (const SceneDesc &d : sd_h_) fast = fast && scene_fast(d);
-    if (fast != all_fast_) invalidate_graph();
-    all_fast_ = fast;
+    all_fast_ = true;
+    for (const SceneDesc &d : sd_h_) all_fast_ = all_fast_ && scene_fast(d);
     // the next staging slot, once the copies of its previous use have run
     // (kDescRing uploads ago: normally long done)
     const int q = (int)(desc_no_++ % kDescRing);
@@ -741,7 +740,7 @@ hipError_t Engine::enqueue_update(hipEvent_t *ev, bool rebuild_work, bool fresh,
     }
     if (fused_ok(rebuild_work, fresh) && !ev) {
         // one persistent launch for the whole steady update
-        LK(launch_fused_update(st, stream_));
+        LK(launch_fused_update(st, cfg, stream_));
         return hipSuccess;
     }
     LK(launch_bucket_sort(d_, cfg, stream_));
@@ -782,7 +781,7 @@ int Engine::update(float dt, std::string *err)
         }
         stage_ms_[5] = 0.0;  // position + collision runs inside the viscosity kernel
     } else if (use_graph_) {
-        const int gi = (rebuild ? 1 : 0) + (fresh ? 2 : 0) + (coop_slots_now() ? 4 : 0);
+        const int gi = (rebuild ? 1 : 0) + (fresh ? 2 : 0) + 4 * form();
         if (!graph_exec_[gi]) {
             CK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
             hipError_t le = enqueue_update(nullptr, rebuild, fresh);
@@ -1061,8 +1060,7 @@ int Engine::step(float dt, int substeps, bool sync_after, std::string *err)
 
 int Engine::run_steady(int n, std::string *err)
 {
-    const bool coop = coop_slots_now() != 0;
-    if (!run_exec_ || run_len_ != n || run_coop_ != coop) {
+    if (!run_exec_ || run_len_ != n || run_form_ != form()) {
         if (run_exec_) (void)hipGraphExecDestroy(run_exec_);
         if (run_graph_) (void)hipGraphDestroy(run_graph_);
         run_exec_ = nullptr;
@@ -1077,7 +1075,7 @@ int Engine::run_steady(int n, std::string *err)
         CK(ce, "end capture");
         CK(hipGraphInstantiate(&run_exec_, run_graph_, nullptr, nullptr, 0), "instantiate graph");
         run_len_ = n;
-        run_coop_ = coop;
+        run_form_ = form();
     }
     CK(hipGraphLaunch(run_exec_, stream_), "graph launch");
     work_updates_ += (uint64_t)n;

@@ -130,8 +130,8 @@ class Engine {
     // three kernels, a steady update, and a launch the device holds resident
     bool fused_ok(bool rebuild_work, bool fresh) const
     {
-        return cfg_.fused && all_fast_ && grid_ && cfg_.nbr && cfg_.density.rows && cfg_.pressure.rows &&
-               cfg_.viscosity.rows && !rebuild_work && !fresh && d_.fused_grid != 0;
+        return cfg_.fused && grid_ && cfg_.nbr && cfg_.density.rows && cfg_.pressure.rows &&
+               cfg_.viscosity.rows && !rebuild_work && !fresh && d_.fused_grid[all_fast_ ? 0 : 1] != 0;
     }
     // Slots of the sixteen-work-item gathers' grid for the present layout (0:
     // the one-work-item forms run).
@@ -139,11 +139,15 @@ class Engine {
     {
         return cfg_.by_size && all_fast_ ? coop_slots(grid_, ed_h_->n_total, d_.capacity) : 0u;
     }
+    // Which kernels an update of the present layout runs, under one setting of the
+    // variants: 0 one work-item per particle, 1 several, 2 one, with IEEE operations.
+    int form() const { return !all_fast_ ? 2 : coop_slots_now() ? 1 : 0; }
     // The variants that an update of the present layout runs.
     LaunchCfg run_cfg() const
     {
-        LaunchCfg c = grid_ ? limit_launch_cfg(cfg_, all_fast_) : cfg_;
+        LaunchCfg c = cfg_;
         c.coop_n = coop_slots_now();
+        c = limit_launch_cfg(c, all_fast_);
         // (set_scan_spin is about the scan's waits, which the one-launch sort has none of)
         c.small_sort = c.coop_n && small_sort_ok(d_.multi, d_.capacity, d_.table_capacity) &&
                        ed_h_->scan_spin == kScanSpinDefault;
@@ -215,8 +219,8 @@ class Engine {
     }
     bool grid_ = false;  // cell-grid bucket key (else the reference's hash % table)
     bool use_graph_ = true;
-    // [rebuild work order? + 2 * fresh predict? + 4 * sixteen-work-item gathers?]
-    static constexpr int kGraphs = 8;
+    // [rebuild work order? + 2 * fresh predict? + 4 * form()]
+    static constexpr int kGraphs = 12;
     hipGraph_t graph_[kGraphs] = {};
     hipGraphExec_t graph_exec_[kGraphs] = {};
     // run_len_ consecutive steady updates (buckets recorded, no work-order
@@ -224,7 +228,7 @@ class Engine {
     hipGraph_t run_graph_ = nullptr;
     hipGraphExec_t run_exec_ = nullptr;
     int run_len_ = 0;
-    bool run_coop_ = false;
+    int run_form_ = 0;
     bool all_fast_ = true;  // scene_fast of every scene
     // The last update's viscosity pass recorded the next update's buckets
     // (keys, tickets, counts) and nothing has changed since: state, settings,

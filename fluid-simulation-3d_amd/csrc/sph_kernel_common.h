@@ -201,7 +201,7 @@ __device__ __forceinline__ PressureSelf pressure_self(const SceneDesc &S, const 
     p.kn = S.k_near;
     p.P = (di.x - p.rho0) * p.kp;
     p.Pn = di.y * p.kn;
-    p.near_ok = FAST && coords_clear_of_zero(pi.x, pi.y, pi.z, S.h * 0x1p-26f);
+    p.near_ok = coords_clear_of_zero(pi.x, pi.y, pi.z, FAST ? S.h * 0x1p-26f : 0x1p-60f);
     return p;
 }
 
@@ -225,7 +225,8 @@ __device__ __forceinline__ PressureSelf pressure_self(const SceneDesc &S, const 
 // uniform particles, where vector issue and the neighbour gathers (two loads a
 // neighbour, 13 million L1 misses a launch) now take about as long as each
 // other.  Pairs that fail it (weak forces, odd units) are tested term by term
-// before IEEE division is taken.
+// before IEEE division is taken.  Without FAST d's own range is tested (the
+// differences are >= 2^-84 then, and h bounds nothing) and every pair's terms.
 struct PressureTerms {
     float tx, ty, tz, ux, uy, uz;
 };
@@ -239,14 +240,14 @@ __device__ __forceinline__ PressureTerms pressure_pair(const PressureSelf &p, fl
     const float snp = (p.Pn + pnj) * 0.5f;  // cc:411
     float d = pair_root<FAST>(d2);
     float dirx, diry, dirz;
-    const bool near_fast = FAST && p.near_ok & (d2 >= 0x1p-52f);
+    const bool near_fast = p.near_ok & (FAST ? d2 >= 0x1p-52f : divisor_ok(d));
     if (near_fast) {
         const float yd = recip_rn(d);
         dirx = quotient(ox, d, yd);
         diry = quotient(oy, d, yd);
         dirz = quotient(oz, d, yd);
     } else {
-        d = sqrtf(d2);
+        if (FAST) d = sqrtf(d2);
         const bool apart = d > 0.0f;  // (0, 1, 0) at d = 0, cc:414
         dirx = apart ? ox / d : 0.0f;
         diry = apart ? oy / d : 1.0f;

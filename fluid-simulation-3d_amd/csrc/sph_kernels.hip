@@ -1302,6 +1302,17 @@ __device__ __forceinline__ uint32_t walk_grid(const SceneDesc &S, const float4 *
                         walk_run<false, false, false, true, true>(xps, 0, xps, aux, k, pi, thr, p, pe, f0, f1, f2,
                                                                   bits, none);
                     if (SKIP_SELF && k - p < 64u) bits &= ~(1ull << (k - p));
+                    if (!AUX && staged) {
+                        const float *sp = reinterpret_cast<const float *>(stage);
+#pragma unroll 1
+                        for (; bits; bits &= bits - 1) {
+                            const uint32_t m = p + (uint32_t)__builtin_ctzll(bits), o = m - lo;
+                            const float ox = sp[o] - pi.x, oy = sp[kStageBuf + o] - pi.y;
+                            const float oz = sp[2 * kStageBuf + o] - pi.z;
+                            body(m, ox, oy, oz, ox * ox + oy * oy + oz * oz, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+                        }
+                        continue;
+                    }
                     bool taken = false;
                     take_masks<KB, AUX ? 4 : 0>(xps, aux, k, pi,
                                                 [&](uint64_t &m, uint32_t &base) {
@@ -1756,8 +1767,9 @@ __device__ __forceinline__ void gather_row(const SceneDesc &S, const float4 *__r
     }
 }
 
-// Density of the slots of (virtual) workgroup vblock_ of the launch.
-template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID>
+// Density of the slots of (virtual) workgroup vblock_ of the launch.  FAST: every
+// scene is within the fast arithmetic's range (scene_fast).
+template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID, bool FAST>
 __device__ __forceinline__ void density_vblock(uint32_t vblock_, SPH_GATHER_PARAMS, float4 *__restrict__ dens)
 {
     constexpr bool CONSUMER = false;
@@ -1769,14 +1781,14 @@ __device__ __forceinline__ void density_vblock(uint32_t vblock_, SPH_GATHER_PARA
     uint32_t *row = ROWS ? nbr + (size_t)i * kNbrMax : nullptr;
     uint32_t c = 0;
     const float thr = S.thr;
-    bool wrong = false;  // MASKS: the masks hold a slot at d >= h
+    bool wrong = false;  // FAST: the masks hold a slot at d >= h
     auto body = [&](uint32_t m, float, float, float, float d2, const float4 &) {
-        const bool in = !MASKS || d2 < thr;
+        const bool in = !FAST || d2 < thr;
         float a, b;
-        density_pair<MASKS>(h, w2c, w3c, d2, in, a, b);
+        density_pair<FAST>(h, w2c, w3c, d2, in, a, b);
         rho += a;
         rhon += b;
-        if (MASKS) wrong |= !in;
+        if (FAST) wrong |= !in;
         if (ROWS && m != k) {
             if (c < kNbrMax) row[c] = m;
             ++c;
@@ -1788,27 +1800,27 @@ __device__ __forceinline__ void density_vblock(uint32_t vblock_, SPH_GATHER_PARA
     // over the wave's staging planes (free once every lane's walk is done);
     // a particle whose record is unusable walks again with the body once the
     // wave's other lanes are done with their tables, staging its rows there.
-    // The walk's test lets a slot within a rounding of h pass (walk_half); the
-    // body makes the exact one, and a wave that met such a slot (one in some
-    // hundreds) does both again with the exact test in the walk.
+    // With FAST the walk's test lets a slot within a rounding of h pass
+    // (walk_half); the body makes the exact one, so the sums are right (such a
+    // slot adds +0), and a wave that met one (one in some hundreds) walks again
+    // with the exact test for the records.
     // Grid key without masks or the LDS list: the body runs over each row's
     // mask as the walk goes (DEFER).
-    MaskOut mo{nbr, ed->n_total, mwords, 0, false};
+    MaskOut mo{nbr, ed->n_total, mwords, 0, !FAST};
     if (GRID && !LIST && MASKS) {
-        uint32_t ok = 0;
-        auto attempt = [&]() __attribute__((always_inline)) {
-            ok = walk<GRID, false, false, true, false, true>(
+        auto record = [&]() __attribute__((always_inline)) {
+            const uint32_t usable = walk<GRID, false, false, true, false, true>(
                 S, xps, nullptr, start, endt, k, pi, stage, clean,
                 [](uint32_t, float, float, float, float, const float4 &) {}, &mo);
             SPH_TABLE_DONE();
-            if (ok) gather_bits<4, false, 0>(S, xps, nullptr, start, k, pi, mo.lens, mwords, mtab, body);
-            SPH_TABLE_DONE();
+            return usable;
         };
-        attempt();
-        if (__ballot(wrong) != 0) {
+        const uint32_t ok = record();
+        if (ok) gather_bits<4, false, 0>(S, xps, nullptr, start, k, pi, mo.lens, mwords, mtab, body);
+        SPH_TABLE_DONE();
+        if (FAST && __ballot(wrong) != 0) {
             mo.exact = true;
-            rho = rhon = 0.0f;
-            attempt();
+            record();
         }
         if (!ok) {
             if (!MULTI && uneven) uneven[0] = 1u;
@@ -1827,13 +1839,14 @@ __device__ __forceinline__ void density_vblock(uint32_t vblock_, SPH_GATHER_PARA
 }
 
 // The second __launch_bounds__ argument is the minimum waves per SIMD the
-// register allocation must allow: the single-scene density pass fits 64
-// VGPRs (8 waves); the multi-scene density pass keeps the 7 it reaches
-// unconstrained.
-template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID>
-__global__ __launch_bounds__(256, 6) void k_density(SPH_GATHER_PARAMS, float4 *__restrict__ dens)
+// register allocation must allow: 6 with neighbour masks, which the mask
+// table's LDS allows too, and for several scenes; the walks of one scene fit 64
+// VGPRs (8 waves).
+template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID, bool FAST = false>
+__global__ __launch_bounds__(256, MULTI || (NBR && GRID) ? 6 : 8) void k_density(SPH_GATHER_PARAMS,
+                                                                               float4 *__restrict__ dens)
 {
-    density_vblock<MULTI, WORK, LIST, NBR, GRID>(blockIdx.x, SPH_GATHER_FWD, dens);
+    density_vblock<MULTI, WORK, LIST, NBR, GRID, FAST>(blockIdx.x, SPH_GATHER_FWD, dens);
 }
 
 // Density pass of the neighbour-row mode.  Each work-item stages its row in
@@ -1885,7 +1898,7 @@ __global__ __launch_bounds__(256) void k_density_rows(SPH_GATHER_PARAMS, float4 
     }
 }
 
-template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID>
+template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID, bool FAST>
 __device__ __forceinline__ void pressure_vblock(uint32_t vblock_, SPH_GATHER_PARAMS,
                                                 const float4 *__restrict__ dens,
                                                 const float4 *__restrict__ vs, float4 *__restrict__ vs2)
@@ -1893,10 +1906,10 @@ __device__ __forceinline__ void pressure_vblock(uint32_t vblock_, SPH_GATHER_PAR
     constexpr bool CONSUMER = NBR && GRID;  // reads the neighbour masks
     SPH_GATHER_PROLOGUE();
     const float4 di = dens[k];
-    const PressureSelf self = pressure_self<CONSUMER>(S, pi, di);
+    const PressureSelf self = pressure_self<FAST>(S, pi, di);
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     auto body = [&](uint32_t, float ox, float oy, float oz, float d2, const float4 &dj) {
-        const PressureTerms r = pressure_pair<CONSUMER>(self, ox, oy, oz, d2, dj);
+        const PressureTerms r = pressure_pair<FAST>(self, ox, oy, oz, d2, dj);
         fx += r.tx;  // cc:416
         fy += r.ty;
         fz += r.tz;
@@ -1931,11 +1944,11 @@ __device__ __forceinline__ void pressure_vblock(uint32_t vblock_, SPH_GATHER_PAR
 // instead of 252 on 1,000,000 colliding particles, the same 103 on 1,048,576
 // uniform ones, and 1,516 instead of 1,453 on 16,777,216, where more waves in
 // flight mean more of the L2 in use.
-template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID>
+template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID, bool FAST = false>
 __global__ __launch_bounds__(256, NBR && GRID ? 4 : 1) void k_pressure(
     SPH_GATHER_PARAMS, const float4 *__restrict__ dens, const float4 *__restrict__ vs, float4 *__restrict__ vs2)
 {
-    pressure_vblock<MULTI, WORK, LIST, NBR, GRID>(blockIdx.x, SPH_GATHER_FWD, dens, vs, vs2);
+    pressure_vblock<MULTI, WORK, LIST, NBR, GRID, FAST>(blockIdx.x, SPH_GATHER_FWD, dens, vs, vs2);
 }
 
 // Writes the new state at the sorted slot (pos, vel, ids: the next resident
@@ -1949,7 +1962,7 @@ __global__ __launch_bounds__(256, NBR && GRID ? 4 : 1) void k_pressure(
         uint32_t *__restrict__ count, uint32_t *__restrict__ wkeys
 #define SPH_VISCOSITY_FWD vs2, ps, pos, vel, ids, rpos, colors, keys, ticks, count, wkeys
 
-template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID>
+template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID, bool FAST>
 __device__ __forceinline__ void viscosity_vblock(uint32_t vblock_, SPH_GATHER_PARAMS, SPH_VISCOSITY_PARAMS)
 {
     constexpr bool CONSUMER = NBR && GRID;  // reads the neighbour masks
@@ -1959,7 +1972,7 @@ __device__ __forceinline__ void viscosity_vblock(uint32_t vblock_, SPH_GATHER_PA
     const float hh = S.hh, c6 = S.poly6c;
     float fx = 0.0f, fy = 0.0f, fz = 0.0f;
     auto body = [&](uint32_t, float, float, float, float d2, const float4 &vj) {
-        const float w = viscosity_weight<CONSUMER>(hh, c6, d2);
+        const float w = viscosity_weight<FAST>(hh, c6, d2);
         fx += (vj.x - vi.x) * w;             // cc:460
         fy += (vj.y - vi.y) * w;
         fz += (vj.z - vi.z) * w;
@@ -1994,17 +2007,17 @@ __device__ __forceinline__ void viscosity_vblock(uint32_t vblock_, SPH_GATHER_PA
 }
 
 // (walking forms: 5 waves per SIMD)
-template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID>
+template <bool MULTI, bool WORK, bool LIST, bool NBR, bool GRID, bool FAST = false>
 __global__ __launch_bounds__(256, NBR && GRID ? 4 : 5) void k_viscosity_integrate(SPH_GATHER_PARAMS,
                                                                            SPH_VISCOSITY_PARAMS)
 {
-    viscosity_vblock<MULTI, WORK, LIST, NBR, GRID>(blockIdx.x, SPH_GATHER_FWD, SPH_VISCOSITY_FWD);
+    viscosity_vblock<MULTI, WORK, LIST, NBR, GRID, FAST>(blockIdx.x, SPH_GATHER_FWD, SPH_VISCOSITY_FWD);
 }
 
 // ---------------------------------------------------------------------------
 // Fused steady update: one persistent launch per Update
 // ---------------------------------------------------------------------------
-// The launch holds s.fused_grid workgroups of 256 -- no more than the device
+// The launch holds s.fused_grid[] workgroups of 256 -- no more than the device
 // keeps resident at once (occupancy x compute units, a multiple of 8) -- and
 // runs the six stages of a steady update (buckets recorded by the previous
 // update's viscosity pass) in order, with a grid barrier between stages: the
@@ -2062,7 +2075,7 @@ __device__ __forceinline__ void grid_barrier(uint32_t *bar, uint32_t nwg, uint32
 }
 static_assert(64 + 16 * 63 < kFusedBarWords, "grid barrier words");
 
-template <bool MULTI>
+template <bool MULTI, bool FAST>
 __global__ __launch_bounds__(kFusedBlock) void k_fused_update(const DevState s)
 {
     __shared__ uint32_t chunk_s;
@@ -2089,16 +2102,16 @@ __global__ __launch_bounds__(kFusedBlock) void k_fused_update(const DevState s)
     const uint32_t vblocks = (((s.capacity + kFusedBlock - 1) / kFusedBlock) + 7u) & ~7u;
     const uint32_t *const endt = s.bounds + 1;
     for (uint32_t v = b; v < vblocks; v += nwg)
-        density_vblock<MULTI, false, false, true, true>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
+        density_vblock<MULTI, false, false, true, true, FAST>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
                                                         s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.uneven, s.dens);
     grid_barrier(s.fbar, nwg, s.scan_err);
     for (uint32_t v = b; v < vblocks; v += nwg)
-        pressure_vblock<MULTI, false, false, true, true>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
+        pressure_vblock<MULTI, false, false, true, true, FAST>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
                                                          s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.uneven, s.dens,
                                                          s.vs, s.vs2);
     grid_barrier(s.fbar, nwg, s.scan_err);
     for (uint32_t v = b; v < vblocks; v += nwg)
-        viscosity_vblock<MULTI, false, false, true, true>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
+        viscosity_vblock<MULTI, false, false, true, true, FAST>(v, s.ed, s.sd, s.scene_of, nullptr, nullptr, s.sids,
                                                           s.xps, s.bounds, endt, s.nbr, s.ncnt, s.sflags, s.uneven, s.vs2,
                                                           s.ps, s.pos, s.vel, s.ids, s.rpos, s.colors, s.keys[0],
                                                           s.keys[1], s.count, nullptr);
@@ -2372,7 +2385,7 @@ inline uint32_t gather_grid(uint32_t cap, int block)
     return (blocks + 7u) & ~7u;
 }
 
-// Launches kernel template KER<MULTI, WORK, LIST, NBR, GRID> chosen at run time.
+// Launches kernel template KER<MULTI, WORK, LIST, NBR, GRID, FAST> chosen at run time.
 #define SPH_GATHER_LAUNCH(KER, var, blk, st, ...)                                             \
     do {                                                                                      \
         const GatherVariant v_ = (var);                                                       \
@@ -2382,8 +2395,10 @@ inline uint32_t gather_grid(uint32_t cap, int block)
         const bool m_ = s.multi;                                                              \
         if (s.grid && c.nbr && v_.rows) {                                                     \
             const size_t ldsr_ = sizeof(uint32_t) * kMaskTabWords * (size_t)(b_ / 64);       \
-            if (m_) KER<true, false, false, true, true><<<g_, b_, ldsr_, st>>>(__VA_ARGS__);  \
-            else KER<false, false, false, true, true><<<g_, b_, ldsr_, st>>>(__VA_ARGS__);    \
+            if (m_ && c.ieee) KER<true, false, false, true, true, false><<<g_, b_, ldsr_, st>>>(__VA_ARGS__);  \
+            else if (m_) KER<true, false, false, true, true, true><<<g_, b_, ldsr_, st>>>(__VA_ARGS__);        \
+            else if (c.ieee) KER<false, false, false, true, true, false><<<g_, b_, ldsr_, st>>>(__VA_ARGS__);  \
+            else KER<false, false, false, true, true, true><<<g_, b_, ldsr_, st>>>(__VA_ARGS__);               \
         } else if (s.grid) {                                                                  \
             const size_t ldsg_ = lds_ + sizeof(uint32_t) * gather_wave_words(true, false, false) * (size_t)(b_ / 64); \
             if (m_ && v_.list) KER<true, false, true, false, true><<<g_, b_, ldsg_, st>>>(__VA_ARGS__);  \
@@ -2419,12 +2434,16 @@ hipError_t launch_density(const DevState &s, const LaunchCfg &c, hipStream_t st)
                            sizeof(uint32_t) * gather_wave_words(true, true, false) * (size_t)(b / 64);
         if (s.multi && c.density.list)
             k_density<true, false, true, true, true><<<g, b, lds, st>>>(SPH_GATHER_ARGS, s.dens);
+        else if (s.multi && c.ieee)
+            k_density<true, false, false, true, true, false><<<g, b, lds, st>>>(SPH_GATHER_ARGS, s.dens);
         else if (s.multi)
-            k_density<true, false, false, true, true><<<g, b, lds, st>>>(SPH_GATHER_ARGS, s.dens);
+            k_density<true, false, false, true, true, true><<<g, b, lds, st>>>(SPH_GATHER_ARGS, s.dens);
         else if (c.density.list)
             k_density<false, false, true, true, true><<<g, b, lds, st>>>(SPH_GATHER_ARGS, s.dens);
+        else if (c.ieee)
+            k_density<false, false, false, true, true, false><<<g, b, lds, st>>>(SPH_GATHER_ARGS, s.dens);
         else
-            k_density<false, false, false, true, true><<<g, b, lds, st>>>(SPH_GATHER_ARGS, s.dens);
+            k_density<false, false, false, true, true, true><<<g, b, lds, st>>>(SPH_GATHER_ARGS, s.dens);
         SPH_LAUNCH_CHECK();
     }
     if (c.nbr && !s.grid) {
@@ -2457,21 +2476,28 @@ hipError_t launch_viscosity_integrate(const DevState &s, const LaunchCfg &c, hip
     SPH_LAUNCH_CHECK();
 }
 
-hipError_t launch_fused_update(const DevState &s, hipStream_t st)
+namespace {
+using FusedKernel = void (*)(DevState);
+FusedKernel fused_kernel(bool multi, bool ieee)
 {
-    if (!s.grid || s.fused_grid == 0 || s.fused_grid % 8u != 0) return hipErrorInvalidConfiguration;
-    if (s.multi) k_fused_update<true><<<s.fused_grid, kFusedBlock, kFusedLds, st>>>(s);
-    else k_fused_update<false><<<s.fused_grid, kFusedBlock, kFusedLds, st>>>(s);
+    if (multi) return ieee ? k_fused_update<true, false> : k_fused_update<true, true>;
+    return ieee ? k_fused_update<false, false> : k_fused_update<false, true>;
+}
+}  // namespace
+
+hipError_t launch_fused_update(const DevState &s, const LaunchCfg &c, hipStream_t st)
+{
+    const uint32_t g = s.fused_grid[c.ieee ? 1 : 0];
+    if (!s.grid || g == 0 || g % 8u != 0) return hipErrorInvalidConfiguration;
+    fused_kernel(s.multi, c.ieee)<<<g, kFusedBlock, kFusedLds, st>>>(s);
     SPH_LAUNCH_CHECK();
 }
 
-uint32_t fused_update_grid(bool multi, int device)
+uint32_t fused_update_grid(bool multi, bool ieee, int device)
 {
     int per_cu = 0, cus = 0;
-    hipError_t e = multi ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fused_update<true>, kFusedBlock,
-                                                                         kFusedLds)
-                         : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fused_update<false>, kFusedBlock,
-                                                                         kFusedLds);
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &per_cu, reinterpret_cast<const void *>(fused_kernel(multi, ieee)), kFusedBlock, kFusedLds);
     if (e != hipSuccess || per_cu <= 0) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0)
         return 0;

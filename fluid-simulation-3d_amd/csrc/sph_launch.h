@@ -69,7 +69,7 @@ struct DevState {
     uint32_t *uneven;    // [2] nonzero: density found particles without a usable mask record in this update,
                          // in the last one (gather_index; null: not recorded)
     uint32_t *fbar;      // [kFusedBarWords] grid barrier of the fused update (zero between launches)
-    uint32_t fused_grid; // workgroups of the fused update that the device holds resident at once
+    uint32_t fused_grid[2]; // workgroups of the fused update (fast, IEEE) that the device holds resident at once
     uint32_t capacity;       // particle slots allocated
     uint32_t table_capacity; // bucket slots allocated
 };
@@ -103,6 +103,9 @@ struct LaunchCfg {
     // the bucket sort is one launch, and the density pass clears its counts
     // (with coop_n only; small_sort_ok, set per update by the engine)
     bool small_sort = false;
+    // the mask kernels use IEEE roots and divisions (a scene is outside the fast
+    // arithmetic's range; set per update by limit_launch_cfg)
+    bool ieee = false;
     int block_stream = 256;  // threads per block of streaming kernels
     bool needs_work() const { return nbr || density.work || pressure.work || viscosity.work; }
 };
@@ -144,20 +147,19 @@ inline bool same_variants(const LaunchCfg &a, const LaunchCfg &b)
            a.nbr == b.nbr && a.fused == b.fused;
 }
 
-// The kernels that read the density pass's records (neighbour masks, or lists
-// with several work-items per particle) take square roots and quotients by
-// methods that are exact for every usual radius; a scene outside that range
-// runs the walking kernels instead, with IEEE operations.
+// The mask kernels and those with several work-items per particle take square
+// roots and quotients by methods that are exact for every usual radius.  Where
+// a scene lies outside that range (scene_fast), all of its layout's scenes run
+// with IEEE operations instead: the mask kernels' own IEEE forms, or the walks,
+// which know no others.
 inline bool scene_fast(const SceneDesc &d) { return radius_fast(d.h) && d.thr >= 0x1p-60f; }
 
-// The variants that run: c, or its walking forms when a scene is not fast.
 inline LaunchCfg limit_launch_cfg(LaunchCfg c, bool all_fast)
 {
     if (!all_fast) {
         c.coop_n = 0;
         c.small_sort = false;
-        c.fused = c.nbr = false;
-        c.density.rows = c.pressure.rows = c.viscosity.rows = false;
+        c.ieee = true;
     }
     return c;
 }
@@ -228,13 +230,13 @@ hipError_t launch_predict(const DevState &s, const LaunchCfg &c, hipStream_t st)
 // descriptors written to s.ed and s.sd by the kernel.
 hipError_t launch_predict_first(const DevState &s, const EngineDesc &e, const SceneDesc &d, hipStream_t st);
 // A steady update (buckets recorded by the previous one) as one launch of
-// s.fused_grid persistent workgroups: count scan, scatter, reorder, density,
+// s.fused_grid[c.ieee] persistent workgroups: count scan, scatter, reorder, density,
 // pressure, viscosity+integrate, separated by grid barriers.  Grid key with
 // neighbour masks only (c.fused; see LaunchCfg).
-hipError_t launch_fused_update(const DevState &s, hipStream_t st);
+hipError_t launch_fused_update(const DevState &s, const LaunchCfg &c, hipStream_t st);
 // Workgroups of the fused update that fit on the device at once (its
 // occupancy x compute units, a multiple of 8), or 0 when none does.
-uint32_t fused_update_grid(bool multi, int device);
+uint32_t fused_update_grid(bool multi, bool ieee, int device);
 // Stages B2 + B3: counting sort into (bucket, particle index) order, bucket
 // bounds, gather of xp, v into sorted order; clears the counts.
 hipError_t launch_bucket_sort(const DevState &s, const LaunchCfg &c, hipStream_t st);
