@@ -427,7 +427,7 @@ int get_variants(sph::Engine *e, int32_t v[14])
         v[4 * q + 3] = g[q].rows;
     }
     v[12] = c.nbr;
-    v[13] = c.fused;
+    v[13] = c.fused ? 1 : c.pinned ? 2 : 0;
     return SPH_OK;
 }
 
@@ -448,7 +448,8 @@ int set_variants(sph::Engine *e, const int32_t v[14])
     }
     if ((c.pressure.rows || c.viscosity.rows) && !c.nbr)
         return fail(SPH_ERR_INVALID, "reading neighbour rows needs the row mode (v[12])");
-    c.fused = v[13] != 0;
+    c.fused = v[13] != 0 && v[13] != 2;
+    c.pinned = v[13] == 2;
     if (c.fused && !(c.nbr && c.density.rows && c.pressure.rows && c.viscosity.rows))
         return fail(SPH_ERR_INVALID, "the fused update (v[13]) needs the row mode in all three kernels");
     e->set_launch_cfg(c);

@@ -854,7 +854,8 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
             for (int b : {64, 128, 256}) cands.push_back({GatherVariant{w != 0, l != 0, b, false}, false});
     for (int b : {64, 128, 256}) cands.push_back({GatherVariant{!grid_, false, b, true}, true});
     // the form that the defaults take at this size, if it is another one
-    if (coop_slots(grid_, n, d_.capacity)) cands.push_back({GatherVariant{}, false, true});
+    const bool sized = all_fast_ && coop_slots(grid_, n, d_.capacity) != 0;
+    if (sized) cands.push_back({GatherVariant{}, false, true});
     double size_ms[3] = {1e30, 1e30, 1e30};
     double walk_ms[3] = {1e30, 1e30, 1e30}, row_ms[3] = {1e30, 1e30, 1e30};
     GatherVariant walk_v[3] = {keep.density, keep.pressure, keep.viscosity}, row_v[3];
@@ -868,8 +869,8 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
         c.density = c.pressure = c.viscosity = cands[ci].v;
         c.nbr = cands[ci].nbr;
         c.fused = false;
-        c.by_size = cands[ci].by_size;
-        if (c.by_size) c = default_launch_cfg(grid_);
+        c.pinned = true;
+        if (cands[ci].by_size) c = default_launch_cfg(grid_);
         cfg_ = c;
         invalidate_graph();
         work_valid_ = false;
@@ -918,14 +919,16 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
         }
     }
     LaunchCfg chosen = keep;
+    bool by_size = false;
     if (!rc) {
         chosen.density = pick[0];
         chosen.pressure = pick[1];
         chosen.viscosity = pick[2];
         chosen.nbr = use_nbr;
         chosen.fused = false;
-        chosen.by_size = false;
-        if (size_ms[0] + size_ms[1] + size_ms[2] < best[0] + best[1] + best[2]) {
+        chosen.pinned = true;
+        by_size = size_ms[0] + size_ms[1] + size_ms[2] < best[0] + best[1] + best[2];
+        if (by_size) {
             chosen = default_launch_cfg(grid_);
             for (int q = 0; q < 3; ++q) best[q] = size_ms[q];
         }
@@ -935,7 +938,7 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
     // each, timed whole, two runs of each interleaved, the faster kept.
     cfg_ = chosen;
     cfg_.fused = true;
-    const bool try_fused = !rc && !chosen.by_size && fused_ok(false, false);
+    const bool try_fused = !rc && !by_size && fused_ok(false, false);
     cfg_ = chosen;
     if (try_fused) {
         hipEvent_t t0 = nullptr, t1 = nullptr;
@@ -967,6 +970,9 @@ int Engine::autotune(float dt, int updates, double ms_out[3], std::string *err)
         if (t1) (void)hipEventDestroy(t1);
         if (!rc) chosen.fused = best_ms[1] < best_ms[0];
     }
+    // (where the pick equals the defaults, whose form was slower here; else it
+    // needs no pin)
+    if (!rc) chosen.pinned = sized && !by_size && same_variants(chosen, default_launch_cfg(grid_));
     if (!rc) rc = check(hipStreamSynchronize(stream_), "autotune sync", err);
     (void)hipFree(snap);
     timing_ = keep_timing;

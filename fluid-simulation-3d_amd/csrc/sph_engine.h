@@ -114,7 +114,6 @@ class Engine {
     void set_launch_cfg(const LaunchCfg &c)
     {
         cfg_ = sanitize_launch_cfg(c, grid_);
-        cfg_.by_size = same_variants(cfg_, default_launch_cfg(grid_));
         invalidate_graph();
     }
     bool grid() const { return grid_; }
@@ -137,7 +136,7 @@ class Engine {
     // the one-work-item forms run).
     uint32_t coop_slots_now() const
     {
-        return cfg_.by_size && all_fast_ ? coop_slots(grid_, ed_h_->n_total, d_.capacity) : 0u;
+        return all_fast_ && follows_size(cfg_, grid_) ? coop_slots(grid_, ed_h_->n_total, d_.capacity) : 0u;
     }
     // Which kernels an update of the present layout runs, under one setting of the
     // variants: 0 one work-item per particle, 1 several, 2 one, with IEEE operations.

@@ -94,11 +94,11 @@ struct LaunchCfg {
     // recorded) is one persistent launch with grid barriers between its
     // stages (launch_fused_update) instead of one launch per stage
     bool fused = false;
-    // the form of the gathers follows the scene's size (coop_slots): set in the
-    // defaults, cleared by any other choice of variants
-    bool by_size = false;
+    // one work-item per particle at every size, also where the variants are the
+    // defaults (whose form else follows the scene's size, coop_slots)
+    bool pinned = false;
     // > 0: the gathers run with sixteen work-items per particle, over a grid
-    // of this many slots (by_size, set per update by the engine)
+    // of this many slots (follows_size, set per update by the engine)
     uint32_t coop_n = 0;
     // the bucket sort is one launch, and the density pass clears its counts
     // (with coop_n only; small_sort_ok, set per update by the engine)
@@ -133,11 +133,10 @@ inline LaunchCfg default_launch_cfg(bool grid)
         c.viscosity = GatherVariant{false, false, 256, true};
         c.nbr = true;
     }
-    c.by_size = true;
     return sanitize_launch_cfg(c, grid);
 }
 
-// The same variants (whatever by_size and coop_n say).
+// The same variants (whatever pinned and coop_n say).
 inline bool same_variants(const LaunchCfg &a, const LaunchCfg &b)
 {
     auto same = [](const GatherVariant &x, const GatherVariant &y) {
@@ -145,6 +144,12 @@ inline bool same_variants(const LaunchCfg &a, const LaunchCfg &b)
     };
     return same(a.density, b.density) && same(a.pressure, b.pressure) && same(a.viscosity, b.viscosity) &&
            a.nbr == b.nbr && a.fused == b.fused;
+}
+
+// The form of the gathers follows the scene's size.
+inline bool follows_size(const LaunchCfg &c, bool grid)
+{
+    return !c.pinned && same_variants(c, default_launch_cfg(grid));
 }
 
 // The mask kernels and those with several work-items per particle take square

@@ -283,7 +283,9 @@ def _variants_dict(v):
     d = {k: {"work": bool(v[4 * q]), "list": bool(v[4 * q + 1]), "block": int(v[4 * q + 2]),
              "rows": bool(v[4 * q + 3])} for q, k in enumerate(_KERNELS)}
     d["nbr"] = bool(v[12])
-    d["fused"] = bool(v[13])
+    d["fused"] = bool(v[13] == 1)
+    if v[13] == 2:  # one work-item per particle at every size
+        d["pinned"] = True
     return d
 
 
@@ -293,7 +295,7 @@ def _variants_array(d):
         v[4 * q:4 * q + 4] = [int(d[k]["work"]), int(d[k]["list"]), int(d[k]["block"]),
                               int(d[k].get("rows", False))]
     v[12] = int(d.get("nbr", False))
-    v[13] = int(d.get("fused", False))
+    v[13] = 1 if d.get("fused", False) else 2 if d.get("pinned", False) else 0
     return v
 
 

@@ -209,8 +209,11 @@ int sph_autotune(sph_handle h, float dt, int updates, double ms[3]);
  * steady update (buckets recorded by the previous one) is one persistent
  * launch with grid barriers between its stages instead of one launch per
  * stage (profiled updates keep the separate launches; a grid barrier's
- * bounded wait that gives up is reported as SPH_ERR_DEVICE).  The array
- * has 14 entries. */
+ * bounded wait that gives up is reported as SPH_ERR_DEVICE); v[13] = 2:
+ * separate launches with one work-item per particle at every size, also
+ * where the variants are the defaults, whose form else follows the scene's
+ * size (sph_autotune picks this where it measured so).  The array has 14
+ * entries. */
 int sph_get_variants(sph_handle h, int32_t v[14]);
 int sph_set_variants(sph_handle h, const int32_t v[14]);
 /* Test support, no reference counterpart: the bound of the count scan's
