@@ -39,6 +39,11 @@ namespace {
 constexpr int kCoopBlock = 256;  // work-items per workgroup
 constexpr uint32_t kList = 96;   // list entries per particle held in LDS
 
+// Mean particles of the cells that one lane looks up (of a row's three, under
+// the grid key) from which the wave's lists are expected to overflow: a 1 / 6.4 of the
+// candidates pass, and 27 cells of 24 then give kList entries.
+constexpr uint32_t kCrowded = 24;
+
 // G lanes per particle.
 template <uint32_t G>
 struct Group {
@@ -99,6 +104,18 @@ __device__ __forceinline__ uint32_t coop_slot(uint32_t n)
     return lb * N + threadIdx.x / G;
 }
 
+// MULTI: the slot, opaque to the optimiser at each pass of run_scene's loop, so
+// that the addresses derived from it are formed where used, not hoisted out of
+// the loop and kept in registers.
+template <bool MULTI>
+__device__ __forceinline__ uint32_t opaque_slot(uint32_t k)
+{
+#if __HIP_DEVICE_COMPILE__
+    if (MULTI) asm volatile("" : "+v"(k));
+#endif
+    return k;
+}
+
 // The walk of the neighbour cells (cc:331-363) by a group: every candidate of
 // the 27 cells in the reference's order, ascending slot within a cell, tested
 // with the one-work-item walk's expressions.  put(at, m, d2): slot m goes to
@@ -112,21 +129,26 @@ __device__ __forceinline__ uint32_t coop_slot(uint32_t n)
 // the lanes that do not store around the loop by themselves, so its ballots
 // miss the others.)
 //
-// FAST: first an unrolled walk, all its loads in flight together, for the
-// common case (no float-hash test needed under the grid key, no list
-// overflow).  The general walk takes one chunk of G slots of one bucket at a
-// time, and is the whole of it where `listed` is set to the number of entries
-// that the caller already holds (nothing is walked, flush(listed) runs).
+// FAST: first an unrolled walk, its loads in flight together, for the common
+// case (no float-hash test needed under the grid key, no list overflow).  Where a
+// list overflows in it or is expected to (kCrowded), and first where !FAST,
+// batches of runs go in a loop that flushes the lists on the way: a third of the
+// general walk's time for them (131,072 particles at 24 a cell: 619 -> 282 us an
+// update; 1,000,000 under the reference key 4,739 -> 3,435, where one work-item
+// per particle takes 3,714).  The
+// general walk takes one chunk of G slots of one bucket at a time: for what is
+// left where one batch alone overflows, and under the grid key for waves that
+// need the float-hash test.
 template <uint32_t G, bool GRID, bool FAST, typename Put, typename Flush>
 __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__restrict__ xps,
                                           const uint32_t *__restrict__ bounds, uint32_t k, const float4 &pi,
-                                          bool clean, bool have_list, uint32_t listed, Put &&put_at, Flush &&flush)
+                                          bool clean, Put &&put_at, Flush &&flush)
 {
     const uint32_t lane = threadIdx.x & 63u, gl = lane & (G - 1u);
     const uint32_t below = (1u << gl) - 1u;  // the group's lanes below this one
     const float thr = S.thr;
-    uint32_t cnt = listed;  // entries of the group's list
-    bool done = have_list;
+    uint32_t cnt = 0;  // entries of the group's list
+    bool done = false;
     auto put = [&](bool pass, uint32_t p, uint32_t m, float d2) __attribute__((always_inline)) {
         put_at(pass ? min(p, kList) : kList, m, d2);
     };
@@ -208,20 +230,25 @@ __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__re
             }
         });
     };
-    if constexpr (FAST && GRID) {
-        // the particle's 27 cells lie inside the grid without wrapping and no
-        // particle's cell lies outside it: every record of a row's run belongs
-        // to the row (walk_grid)
+    // grid key, plain: the wave's particles' 27 cells lie inside the grid without
+    // wrapping and no particle's cell lies outside it, so every record of a row's
+    // run belongs to the row (walk_grid); base: the bucket of the particle's cell
+    bool plain = true;
+    uint32_t base = 0;
+    const uint32_t gy = S.gdim[1], gz = S.gdim[2];
+    if constexpr (GRID) {
         const uint32_t ux = (uint32_t)cx - (uint32_t)S.cell_lo[0];
         const uint32_t uy = (uint32_t)cy - (uint32_t)S.cell_lo[1];
         const uint32_t uz = (uint32_t)cz - (uint32_t)S.cell_lo[2];
-        const uint32_t gy = S.gdim[1], gz = S.gdim[2];
         auto inside = [](uint32_t u, uint32_t g) { return u < g && u - 1u < g && u + 1u < g; };
         const bool interior = inside(ux, S.gdim[0]) && inside(uy, gy) && inside(uz, gz);
-        if (!wave_any(!(clean && interior))) {
+        plain = !wave_any(!(clean && interior));
+        base = S.key_off + (ux * gy + uy) * gz + uz;
+    }
+    if constexpr (FAST && GRID) {
+        if (plain) {
             // the lanes fetch the bounds of the group's nine runs together
             // (G = 8: the ninth by all)
-            const uint32_t base = S.key_off + (ux * gy + uy) * gz + uz;
             const uint32_t row = min(gl, 8u);
             const uint32_t mine = base + ((row / 3u - 1u) * gy + (row % 3u - 1u)) * gz;
             const uint32_t rb = bounds[mine - 1u], re = bounds[mine + 2u];
@@ -230,23 +257,25 @@ __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__re
                 b8 = bounds[base + (gy + 1u) * gz - 1u];
                 e8 = bounds[base + (gy + 1u) * gz + 2u];
             }
-            constexpr int kRows = 3;  // runs in flight together (nine: 122 registers, 8.5 instead of 8.1 us)
-            static_for<9 / kRows>([&](auto Q) __attribute__((always_inline)) {
-                uint32_t b[kRows], e[kRows];
-                static_for<kRows>([&](auto R) __attribute__((always_inline)) {
-                    constexpr int q = decltype(R)::value, r = decltype(Q)::value * kRows + q;
-                    if constexpr (r < (int)G) {
-                        b[q] = group_bcast<G, r>(rb);
-                        e[q] = group_bcast<G, r>(re);
-                    } else {
-                        b[q] = b8;
-                        e[q] = e8;
-                    }
+            if (!wave_any(re - rb > 3u * kCrowded)) {
+                constexpr int kRows = 3;  // runs in flight together (nine: 122 registers, 8.5 instead of 8.1 us)
+                static_for<9 / kRows>([&](auto Q) __attribute__((always_inline)) {
+                    uint32_t b[kRows], e[kRows];
+                    static_for<kRows>([&](auto R) __attribute__((always_inline)) {
+                        constexpr int q = decltype(R)::value, r = decltype(Q)::value * kRows + q;
+                        if constexpr (r < (int)G) {
+                            b[q] = group_bcast<G, r>(rb);
+                            e[q] = group_bcast<G, r>(re);
+                        } else {
+                            b[q] = b8;
+                            e[q] = e8;
+                        }
+                    });
+                    runs(std::integral_constant<int, kRows>{}, std::integral_constant<int, 32>{}, std::false_type{},
+                         b, e, [](auto) { return 0.0f; });
                 });
-                runs(std::integral_constant<int, kRows>{}, std::integral_constant<int, 32>{}, std::false_type{}, b,
-                     e, [](auto) { return 0.0f; });
-            });
-            done = !wave_any(cnt > kList);
+                done = !wave_any(cnt > kList);
+            }
         }
     }
     if constexpr (FAST && !GRID) {
@@ -256,29 +285,38 @@ __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__re
         // and 75 us (one: 91).  Sixteen lanes hold nine in 80 registers: 7.8 us on
         // 3,000 particles, 8.5 with three.
         constexpr int kFetch = (27 + G - 1) / G, kCells = G == 16 ? 9 : 3;
-        uint32_t fb[kFetch], fe[kFetch];
+        uint32_t fb[kFetch], fe[kFetch], all = 0;
 #pragma unroll
         for (int c = 0; c < kFetch; ++c) {
             const uint32_t o = min(gl + G * c, 26u);
             const uint32_t key = S.key_off + fastmod(cell_hash(o), S.mod_m, S.table);
             fb[c] = bounds[key];
             fe[c] = bounds[key + 1u];
+            all += fe[c] - fb[c];
         }
-        static_for<27 / kCells>([&](auto H) __attribute__((always_inline)) {
-            uint32_t b[kCells], e[kCells];
-            static_for<kCells>([&](auto P) __attribute__((always_inline)) {
-                constexpr int q = decltype(P)::value, A = decltype(H)::value * kCells + q;
-                b[q] = group_bcast<G, A % G>(fb[A / G]);
-                e[q] = group_bcast<G, A % G>(fe[A / G]);
+        if (!wave_any(all > (uint32_t)kFetch * kCrowded)) {
+            static_for<27 / kCells>([&](auto H) __attribute__((always_inline)) {
+                uint32_t b[kCells], e[kCells];
+                static_for<kCells>([&](auto P) __attribute__((always_inline)) {
+                    constexpr int q = decltype(P)::value, A = decltype(H)::value * kCells + q;
+                    b[q] = group_bcast<G, A % G>(fb[A / G]);
+                    e[q] = group_bcast<G, A % G>(fe[A / G]);
+                });
+                runs(std::integral_constant<int, kCells>{}, std::integral_constant<int, 16>{}, std::true_type{}, b, e,
+                     [&](auto P) { return (float)cell_hash((uint32_t)(decltype(H)::value * kCells + decltype(P)::value)); });
             });
-            runs(std::integral_constant<int, kCells>{}, std::integral_constant<int, 16>{}, std::true_type{}, b, e,
-                 [&](auto P) { return (float)cell_hash((uint32_t)(decltype(H)::value * kCells + decltype(P)::value)); });
-        });
-        done = !wave_any(cnt > kList);
+            done = !wave_any(cnt > kList);
+        }
     }
     if (!done) cnt = 0;
-    // the general walk: bucket o, its slots from m0 on (each bucket by itself,
-    // so the grid's wrap seam needs no case of its own)
+    // The rest: cell o is the next one.  In batches: a row of cells at a time
+    // under the grid key, else three cells (12 to 24 registers of records; three
+    // rows leave fewer waves).  Then the general walk of bucket o, its slots from
+    // m0 on (each bucket by itself, so the grid's wrap seam needs no case of its
+    // own).
+    constexpr uint32_t kRuns = GRID ? 1 : 3, kRun = GRID ? 3 : 1;  // runs, cells of a run
+    static_assert(27 % (kRuns * kRun) == 0, "whole batches");
+    bool batches = plain;
     uint32_t o = 0, m0 = 0, e = 0;
     float f = 0.0f;
     auto bucket = [&]() {
@@ -292,14 +330,49 @@ __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__re
         e = bounds[key + 1u];
         f = (float)cell_hash(o);
     };
-    if (!done) bucket();
+    if (!done && !batches) bucket();
 #pragma unroll 1
     for (;;) {
-        if (done || wave_any(cnt + G > kList)) {
+        bool full = done;
+        if (!done && batches) {
+            uint32_t rb[kRuns], re[kRuns];
+#pragma unroll
+            for (uint32_t q = 0; q < kRuns; ++q) {
+                const uint32_t c = o + q * kRun;
+                if constexpr (GRID) {
+                    const uint32_t mid = base + ((c / 9u - 1u) * gy + ((c / 3u) % 3u - 1u)) * gz;
+                    rb[q] = bounds[mid - 1u];
+                    re[q] = bounds[mid + 2u];
+                } else {
+                    const uint32_t key = S.key_off + fastmod(cell_hash(c), S.mod_m, S.table);
+                    rb[q] = bounds[key];
+                    re[q] = bounds[key + 1u];
+                }
+            }
+            const uint32_t before = cnt;
+            runs(std::integral_constant<int, kRuns>{}, std::integral_constant<int, GRID ? 32 : 16>{},
+                 std::integral_constant<bool, !GRID>{}, rb, re,
+                 [&](auto P) { return (float)cell_hash(o + (uint32_t)decltype(P)::value); });
+            if (!wave_any(cnt > kList)) {
+                o += kRuns * kRun;
+                full = done = o == 27u;
+            } else {  // a list is full: what it held before, then this batch again
+                cnt = before;
+                full = wave_any(cnt != 0u);
+                if (!full) {  // (one batch alone fills it)
+                    batches = false;
+                    bucket();
+                }
+            }
+        } else if (!done) {
+            full = wave_any(cnt + G > kList);
+        }
+        if (full) {
             flush(cnt);
             cnt = 0;
         }
         if (done) break;
+        if (batches) continue;
         const uint32_t m = m0 + gl;
         const bool in = m < e;
         const float4 r = xps[in ? m : k];
@@ -326,13 +399,30 @@ __device__ __forceinline__ float ordered_sum(float acc, const float *plane, uint
     return acc;
 }
 
-// Rows of the neighbour lists: entry t of slot k at [k * cap + t], 16-bit slots
-// while every slot fits (the row then holds twice as many).
+// Rows of the neighbour lists: entry t of slot k at [k * cap + t].  uint16_t:
+// slots, while every slot fits.  int16_t: differences to k, under the grid key,
+// whose neighbours lie within three planes of cells: up to kCoopMaxGrid particles
+// they fit unless a plane holds more than some 30,000 (the particle then walks
+// again).  uint32_t: slots.  In 16 bits a row holds twice as many (70,000
+// colliding particles, mean of 60 steps: 128 us an update with rows of 64, 84 of
+// 128, and the walk in batches).
 template <typename T>
 struct Rows {
     T *rows, *spare;  // spare: a row that nobody reads
     uint32_t cap;
-    __device__ __forceinline__ uint32_t get(uint32_t k, uint32_t t) const { return rows[(size_t)k * cap + t]; }
+    __device__ __forceinline__ uint32_t get(uint32_t k, uint32_t t) const
+    {
+        const T e = rows[(size_t)k * cap + t];
+        return std::is_signed<T>::value ? k + (uint32_t)(int32_t)e : (uint32_t)e;
+    }
+    static __device__ __forceinline__ T entry(uint32_t k, uint32_t m)
+    {
+        return (T)(std::is_signed<T>::value ? m - k : m);
+    }
+    static __device__ __forceinline__ bool holds(uint32_t k, uint32_t m)
+    {
+        return !std::is_signed<T>::value || m - k + 32768u < 65536u;
+    }
 };
 
 struct CoopArgs {
@@ -348,27 +438,29 @@ struct CoopArgs {
 };
 
 template <uint32_t G, bool MULTI, bool GRID, typename T>
-__global__ __launch_bounds__(kCoopBlock, 4) void k_coop_density(const CoopArgs A, const Rows<T> out,
+__global__ __launch_bounds__(kCoopBlock, 5) void k_coop_density(const CoopArgs A, const Rows<T> out,
                                                                 float4 *__restrict__ dens)
 {
     constexpr uint32_t kChunk = Group<G>::kChunk;
     __shared__ uint2 lists[Group<G>::kParticles][kList + 1];                // (slot, d2)
     __shared__ __align__(16) float terms[Group<G>::kParticles][2][kChunk];  // the two sums' terms
-    const uint32_t n = A.ed->n_total, k = coop_slot<G>(n);
+    const uint32_t n = A.ed->n_total, slot = coop_slot<G>(n);
     if (A.clear) {
         const uint32_t nc = A.ed->table_total + A.ed->n_scenes;
         for (uint32_t i = blockIdx.x * kCoopBlock + threadIdx.x; i < nc; i += gridDim.x * kCoopBlock) A.clear[i] = 0u;
     }
-    if (k >= n) return;
+    if (slot >= n) return;
     const uint32_t gl = threadIdx.x & (G - 1u), gq = threadIdx.x / G;
     uint2 *const lst = lists[gq];
     float *const t0p = terms[gq][0], *const t1p = terms[gq][1];
-    const float4 pi = A.xps[k];
+    const float4 pi = A.xps[slot];
     auto scene = [&](const SceneDesc &S) __attribute__((always_inline)) {
+        const uint32_t k = opaque_slot<MULTI>(slot);
         const bool clean = GRID && A.sflags[S.index] == 0u;
         const float h = S.h, w2c = S.w2c, w3c = S.w3c;
         float acc = 0.0f;    // lane 0: rho, lane 1: near rho
         uint32_t total = 0;  // neighbours flushed so far
+        bool far = false;    // one of this lane's does not fit a row entry
         auto flush = [&](uint32_t cnt) {
             wave_sync();
             for (uint32_t c0 = 0; wave_any(c0 < cnt); c0 += kChunk) {
@@ -386,7 +478,8 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_density(const CoopArgs A
                     t0p[r + gl] = have ? a : 0.0f;
                     t1p[r + gl] = have ? b : 0.0f;
                     T *const row = cnt ? out.rows + (size_t)k * out.cap : out.spare;
-                    row[min(total + at, out.cap - 1u)] = (T)e.x;
+                    row[min(total + at, out.cap - 1u)] = Rows<T>::entry(k, e.x);
+                    far |= have & !Rows<T>::holds(k, e.x);
                 }
                 wave_sync();
                 acc = ordered_sum(acc, gl == 0u ? t0p : t1p, cnt > c0 ? min(kChunk, cnt - c0) : 0u);
@@ -395,15 +488,19 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_density(const CoopArgs A
             total += cnt;
         };
         coop_walk<G, GRID, true>(
-            S, A.xps, A.bounds, k, pi, clean, false, 0u,
+            S, A.xps, A.bounds, k, pi, clean,
             [&](uint32_t at, uint32_t m, float d2) { lst[at] = make_uint2(m, __float_as_uint(d2)); }, flush);
+        if constexpr (std::is_signed<T>::value) {
+            const uint64_t fars = __ballot(far);
+            if ((fars >> (threadIdx.x & 63u & ~(G - 1u))) & ((1ull << G) - 1ull)) total = out.cap + 1u;
+        }
         const float rho = group_bcast<G, 0>(acc), rhon = group_bcast<G, 1>(acc);
         if (gl == 0u) {
             A.ncnt[k] = total;
             dens[k] = make_float4(rho, rhon, reciprocal_or_zero(rho), reciprocal_or_zero(rhon));
         }
     };
-    run_scene<MULTI>(A.sd, A.scene_of, k, scene);
+    run_scene<MULTI>(A.sd, A.scene_of, slot, scene);
 }
 
 // The sum over a particle's neighbours of NT three-component terms each (added
@@ -421,8 +518,9 @@ __device__ __forceinline__ float coop_sum(const CoopArgs &A, const SceneDesc &S,
     const float *const mine = planes + min(gl, 2u) * kPlane;
     float acc = 0.0f;
     const uint32_t total = A.ncnt[k];
-    const bool rows = !wave_any(total > in.cap);
-    auto flush = [&](uint32_t cnt) {
+    // (the two ways share nothing: most waves take the first, which then needs
+    // neither the cell nor the registers of the walk)
+    auto take = [&](auto from_rows, uint32_t cnt) __attribute__((always_inline)) {
         wave_sync();
 #pragma unroll 1
         for (uint32_t c0 = 0; wave_any(c0 < cnt); c0 += kChunk) {
@@ -432,7 +530,7 @@ __device__ __forceinline__ float coop_sum(const CoopArgs &A, const SceneDesc &S,
 #pragma unroll
             for (uint32_t r = 0; r < R; ++r) {
                 const uint32_t t = c0 + r * G + gl, at = t < cnt ? t : 0u;
-                const uint32_t e = rows ? in.get(k, at) : lst[at];
+                const uint32_t e = decltype(from_rows)::value ? in.get(k, at) : lst[at];
                 m[r] = t < cnt ? e : k;
             }
 #pragma unroll
@@ -459,25 +557,29 @@ __device__ __forceinline__ float coop_sum(const CoopArgs &A, const SceneDesc &S,
             wave_sync();
         }
     };
-    coop_walk<G, GRID, false>(S, A.xps, A.bounds, k, pi, clean, rows, rows ? total : 0u,
-                           [&](uint32_t at, uint32_t m, float) { lst[at] = m; }, flush);
+    if (!wave_any(total > in.cap)) take(std::true_type{}, total);
+    else
+        coop_walk<G, GRID, false>(S, A.xps, A.bounds, k, pi, clean,
+                                  [&](uint32_t at, uint32_t m, float) { lst[at] = m; },
+                                  [&](uint32_t cnt) { take(std::false_type{}, cnt); });
     return acc;
 }
 
 template <uint32_t G, bool MULTI, bool GRID, typename T>
-__global__ __launch_bounds__(kCoopBlock, 4) void k_coop_pressure(const CoopArgs A, const Rows<T> in,
+__global__ __launch_bounds__(kCoopBlock, 5) void k_coop_pressure(const CoopArgs A, const Rows<T> in,
                                                                  const float4 *__restrict__ dens,
                                                                  const float4 *__restrict__ vs,
                                                                  float4 *__restrict__ vs2)
 {
     __shared__ uint32_t lists[Group<G>::kParticles][kList + 1];
     __shared__ __align__(16) float terms[Group<G>::kParticles][3][2 * Group<G>::kChunk];
-    const uint32_t n = A.ed->n_total, k = coop_slot<G>(n);
-    if (k >= n) return;
+    const uint32_t n = A.ed->n_total, slot = coop_slot<G>(n);
+    if (slot >= n) return;
     const uint32_t gl = threadIdx.x & (G - 1u), gq = threadIdx.x / G;
-    const float4 pi = A.xps[k], di = dens[k];
-    float4 v = vs[k];
+    const float4 pi = A.xps[slot], di = dens[slot];
+    float4 v = vs[slot];
     auto scene = [&](const SceneDesc &S) __attribute__((always_inline)) {
+        const uint32_t k = opaque_slot<MULTI>(slot);
         const bool clean = GRID && A.sflags[S.index] == 0u;
         const PressureSelf self = pressure_self<true>(S, pi, di);
         const float f = coop_sum<G, GRID, 2>(
@@ -498,7 +600,7 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_pressure(const CoopArgs 
         v.z = v.z + (fz / rho) * dt;
         if (gl == 0u) vs2[k] = v;
     };
-    run_scene<MULTI>(A.sd, A.scene_of, k, scene);
+    run_scene<MULTI>(A.sd, A.scene_of, slot, scene);
 }
 
 struct CoopState {  // what the viscosity stage writes (see k_viscosity_integrate)
@@ -514,16 +616,20 @@ struct CoopState {  // what the viscosity stage writes (see k_viscosity_integrat
     const float4 *dens;
 };
 
+// (waves per SIMD: what the LDS allows, 5 for density and pressure, 7 here; one
+// scene fits 72 registers, and with 75, 6 waves, the reference key's stage takes
+// 43.3 instead of 40.8 us on 200,003 particles; several scenes take 90)
 template <uint32_t G, bool MULTI, bool GRID, typename T>
-__global__ __launch_bounds__(kCoopBlock, 4) void k_coop_viscosity(const CoopArgs A, const Rows<T> in,
+__global__ __launch_bounds__(kCoopBlock, MULTI ? 5 : 7) void k_coop_viscosity(const CoopArgs A, const Rows<T> in,
                                                                   const CoopState W)
 {
     __shared__ uint32_t lists[Group<G>::kParticles][kList + 1];
     __shared__ uint32_t buckets[Group<G>::kParticles];
     __shared__ __align__(16) float terms[Group<G>::kParticles][3][Group<G>::kChunk];
-    const uint32_t n = A.ed->n_total, k = coop_slot<G>(n);
+    const uint32_t n = A.ed->n_total, slot = coop_slot<G>(n);
     const uint32_t gl = threadIdx.x & (G - 1u), gq = threadIdx.x / G;
     auto scene = [&](const SceneDesc &S) __attribute__((always_inline)) {
+        const uint32_t k = opaque_slot<MULTI>(slot);
         const float4 pi = A.xps[k], vi = W.vs2[k], x0 = W.ps[k];
         const uint32_t g = A.sids[k];
         const bool clean = GRID && A.sflags[S.index] == 0u;
@@ -562,19 +668,19 @@ __global__ __launch_bounds__(kCoopBlock, 4) void k_coop_viscosity(const CoopArgs
         buckets[gq] = bucket_key(*A.ed, S, P, W.count);
         if (W.wkeys) W.wkeys[k] = work_key(*A.ed, S, S.index, P.cx, P.cy, P.cz);
     };
-    if (k < n) run_scene<MULTI>(A.sd, A.scene_of, k, scene);
+    if (slot < n) run_scene<MULTI>(A.sd, A.scene_of, slot, scene);
     if (W.out_pos) return;
     // the tickets of the workgroup's particles, by one lane each: one atomic
     // per run of equal buckets
     __syncthreads();
     if (threadIdx.x >= Group<G>::kParticles) return;
-    const uint32_t slot = k - gq + threadIdx.x;
-    const bool valid = slot < n;
+    const uint32_t at = slot - gq + threadIdx.x;
+    const bool valid = at < n;
     const uint32_t key = valid ? buckets[threadIdx.x] : 0xffffffffu;
     const uint32_t ticket = bucket_ticket(valid, key, W.count);
     if (valid) {
-        W.keys[slot] = key;
-        W.ticks[slot] = ticket;
+        W.keys[at] = key;
+        W.ticks[at] = ticket;
     }
 }
 
@@ -606,21 +712,22 @@ Rows<T> coop_rows(const DevState &s)
 }
 
 // Launches KER<G, MULTI, GRID, T> over n particle slots.
-#define SPH_COOP_LAUNCH_T(KER, G, r_, n, st, ...)                                                  \
+#define SPH_COOP_LAUNCH_T(KER, G, GRID, T, n, st, ...)                                             \
     do {                                                                                           \
+        const Rows<T> r_ = coop_rows<T>(s);                                                        \
         const uint32_t g_ = coop_grid<G>(n);                                                       \
-        if (s.multi && s.grid) KER<G, true, true><<<g_, kCoopBlock, 0, st>>>(a, r_, __VA_ARGS__);  \
-        else if (s.multi) KER<G, true, false><<<g_, kCoopBlock, 0, st>>>(a, r_, __VA_ARGS__);      \
-        else if (s.grid) KER<G, false, true><<<g_, kCoopBlock, 0, st>>>(a, r_, __VA_ARGS__);       \
-        else KER<G, false, false><<<g_, kCoopBlock, 0, st>>>(a, r_, __VA_ARGS__);                  \
+        if (s.multi) KER<G, true, GRID><<<g_, kCoopBlock, 0, st>>>(a, r_, __VA_ARGS__);            \
+        else KER<G, false, GRID><<<g_, kCoopBlock, 0, st>>>(a, r_, __VA_ARGS__);                   \
     } while (0)
 #define SPH_COOP_LAUNCH(KER, n, st, ...)                                                           \
     do {                                                                                           \
-        const Rows<uint16_t> r16_ = coop_rows<uint16_t>(s);                                        \
-        const Rows<uint32_t> r32_ = coop_rows<uint32_t>(s);                                        \
-        if (n <= kCoopWide) SPH_COOP_LAUNCH_T(KER, 16, r16_, n, st, __VA_ARGS__);                  \
-        else if (s.capacity <= 65536u) SPH_COOP_LAUNCH_T(KER, 8, r16_, n, st, __VA_ARGS__);        \
-        else SPH_COOP_LAUNCH_T(KER, 8, r32_, n, st, __VA_ARGS__);                                  \
+        const bool wide_ = n <= kCoopWide, short_ = s.capacity <= 65536u;                          \
+        if (s.grid && wide_) SPH_COOP_LAUNCH_T(KER, 16, true, uint16_t, n, st, __VA_ARGS__);       \
+        else if (s.grid && short_) SPH_COOP_LAUNCH_T(KER, 8, true, uint16_t, n, st, __VA_ARGS__);  \
+        else if (s.grid) SPH_COOP_LAUNCH_T(KER, 8, true, int16_t, n, st, __VA_ARGS__);             \
+        else if (wide_) SPH_COOP_LAUNCH_T(KER, 16, false, uint16_t, n, st, __VA_ARGS__);           \
+        else if (short_) SPH_COOP_LAUNCH_T(KER, 8, false, uint16_t, n, st, __VA_ARGS__);           \
+        else SPH_COOP_LAUNCH_T(KER, 8, false, uint32_t, n, st, __VA_ARGS__);                       \
     } while (0)
 
 }  // namespace

@@ -261,8 +261,7 @@ int Engine::create(const std::vector<SceneSpec> &scenes, uint32_t capacity,
     e->cfg_ = default_launch_cfg(grid);
     {
         int dev = 0;
-        if (hipGetDevice(&dev) == hipSuccess)
-            for (int q = 0; q < 2; ++q) e->d_.fused_grid[q] = fused_update_grid(e->d_.multi, q != 0, dev);
+        if (hipGetDevice(&dev) == hipSuccess) e->d_.fused_grid[0] = fused_update_grid(e->d_.multi, false, dev);
     }
     rc = e->check(hipMemcpy(e->d_scene_of_, scene_of.data(), sizeof(uint32_t) * capacity,
                             hipMemcpyHostToDevice),
@@ -427,6 +426,10 @@ int Engine::push_descs(std::string *err)
     }
     all_fast_ = true;
     for (const SceneDesc &d : sd_h_) all_fast_ = all_fast_ && scene_fast(d);
+    if (!all_fast_ && d_.fused_grid[1] == 0) {
+        int dev = 0;
+        if (hipGetDevice(&dev) == hipSuccess) d_.fused_grid[1] = fused_update_grid(d_.multi, true, dev);
+    }
     // the next staging slot, once the copies of its previous use have run
     // (kDescRing uploads ago: normally long done)
     const int q = (int)(desc_no_++ % kDescRing);

@@ -182,10 +182,19 @@ inline LaunchCfg limit_launch_cfg(LaunchCfg c, bool all_fast)
 //   reference key  4,000: 153 / 30   50,000: 195 / 64   200,000: 318 / 163
 //                  1,200,000: 1,233 / 1,017   2,000,000: 2,001 / 1,660
 //                  6,000,000: 6,662 / 5,202   16,700,000: 19,477 / 15,160
-constexpr uint32_t kCoopMaxGrid = 1u << 17;
+// Compressed fluid, whose lists overflow their rows or the LDS (mean of a run of
+// 60 steps of two blocks colliding, and one state of 24 particles a cell):
+//   grid key       70,000: 216 / 84   131,072: 356 / 147; 24 a cell 662 / 282
+//   reference key  200,000: 668 / 351   1,000,000: 2,460 / 2,060; 24 a cell
+//                  3,714 / 3,435 (at 40 a cell, five times the rest density, 5,688 /
+//                  5,904)   4,000,000: 3,888 / 3,679
+// Batches under the grid key, 16 scenes: 65,536 in all 71 / 57, 119,126 110 / 90,
+// 131,072 86 / 88; a dam break of 100,000 97 / 84, of 131,072 98 / 99: the line
+// lies where calm fluid gains no more.
+constexpr uint32_t kCoopMaxGrid = 120000;
 constexpr uint32_t kCoopMaxReference = 1u << 24;
 
-// Slots that the sixteen-work-item gathers' grid covers for n particles in a
+// Slots that the several-work-item gathers' grid covers for n particles in a
 // layout of `capacity` slots, or 0 when the one-work-item forms run.
 inline uint32_t coop_slots(bool grid, uint32_t n, uint32_t capacity)
 {

@@ -18,6 +18,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "../../include/sph_amd.h"
@@ -45,6 +46,7 @@ struct Layout {
     size_t ed, sd, scan_err, sflags, chain, bounds, count;
     size_t pos, vel, xps, vs, vs2, dens, ps;
     size_t keys0, keys1, ids, sids, ncnt, order, nbr;
+    size_t rows;
     size_t total;
     size_t chain_words;
 };
@@ -68,18 +70,21 @@ constexpr Layout make_layout()
     L.chain = take(sizeof(uint64_t) * chain_words);
     L.bounds = take(sizeof(uint32_t) * (T + 1));
     L.count = take(sizeof(uint32_t) * (T + 1));  // the buckets, then one scene flag
-    L.pos = take(16 * N);
-    L.vel = take(16 * N);
     L.xps = take(16 * N);
     L.vs = take(16 * N);
     L.vs2 = take(16 * N);
     L.dens = take(16 * N);
     L.ps = take(16 * N);
+    L.sids = take(4 * N);
+    L.ncnt = take(4 * N);
+    // what the several-lanes forms need no more once the bucket sort is done (pos
+    // and vel not at all), with nbr behind it: their rows
+    L.rows = o;
+    L.pos = take(16 * N);
+    L.vel = take(16 * N);
     L.keys0 = take(4 * N);
     L.keys1 = take(4 * N);
     L.ids = take(4 * N);
-    L.sids = take(4 * N);
-    L.ncnt = take(4 * N);
     L.order = take(8 * N);
     L.nbr = take(4 * kNoAllocNbrWords * N);
     L.total = o;
@@ -217,7 +222,6 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     s.sflags = at<uint32_t>(base, kLayout.sflags);
     s.nbr = at<uint32_t>(base, kLayout.nbr);
     s.nbr_words = kNoAllocNbrWords;
-    s.spare = at<uint32_t>(base, kLayout.pos);  // (the walking forms' only)
     s.ncnt = at<uint32_t>(base, kLayout.ncnt);
     s.scan_err = at<uint32_t>(base, kLayout.scan_err);
     s.capacity = n;
@@ -233,8 +237,9 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
     hipError_t e = hipSuccess;
 #define NA(x, what)                                  \
     if ((e = (x)) != hipSuccess) return hip_fail(e, what)
-    // Every call's launches leave the counts at zero, so a call clears them only
-    // when one before it on this GPU failed halfway.  Launches recorded into the
+    // The launches of a call with several work-items per particle leave the counts
+    // at zero, so such a call clears them only when one before it on this GPU
+    // failed halfway or took the other form.  Launches recorded into the
     // caller's graph run later, after calls that this one cannot know: they always
     // clear first, and recording them says nothing about the counts now.
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -255,6 +260,12 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
         if (c.small_sort) s.ids = nullptr;  // particle order
         else NA(sph::launch_iota(s.ids, n, 0, st), "resident order");
         NA(sph::launch_bucket_sort(s, c, st), "bucket sort");
+        // 40 words a particle or more: rows of 80 to 128 neighbours, where nbr by
+        // itself holds 48, which random fluid passes (65,536 particles, 12 a cell:
+        // 184 us, now 117; 147 with one work-item per particle)
+        s.nbr = at<uint32_t>(base, kLayout.rows);
+        s.nbr_words = (uint32_t)std::min<size_t>(64, (kLayout.total - kLayout.rows) / (4 * (size_t)n));
+        s.spare = at<uint32_t>(base, kLayout.vs2);  // (pressure's, which comes later)
         NA(sph::launch_density(s, c, st), "density");
         NA(sph::launch_pressure(s, c, st), "pressure");
         NA(sph::launch_coop_viscosity_out(s, c.coop_n, reinterpret_cast<float4 *>(pos4_out),
@@ -275,10 +286,12 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
                                 reinterpret_cast<float4 *>(vel4_out), reinterpret_cast<float2 *>(dens2_out), nullptr,
                                 st),
            "particle order");
-        NA(sph::launch_clear_words(s.count, s.count_size, st), "clear counts");  // (the next update's buckets)
+        // (the next update's buckets; a call that is not recorded leaves them to the
+        // mark, below)
+        if (recorded) NA(sph::launch_clear_words(s.count, s.count_size, st), "clear counts");
     }
-    // (the walking form clears its own buckets and chain words only)
-    scratch_clean(base, were || (c.coop_n && !recorded));
+    // (the one-work-item form clears its own buckets and chain words only)
+    scratch_clean(base, c.coop_n ? were || !recorded : were && recorded);
     if (!wait) return SPH_OK;
     NA(hipStreamSynchronize(st), "sync");
     uint32_t flag = 0;
