@@ -188,10 +188,11 @@ inline LaunchCfg limit_launch_cfg(LaunchCfg c, bool all_fast)
 //   reference key  200,000: 668 / 351   1,000,000: 2,460 / 2,060; 24 a cell
 //                  3,714 / 3,435 (at 40 a cell, five times the rest density, 5,688 /
 //                  5,904)   4,000,000: 3,888 / 3,679
-// Batches under the grid key, 16 scenes: 65,536 in all 71 / 57, 119,126 110 / 90,
-// 131,072 86 / 88; a dam break of 100,000 97 / 84, of 131,072 98 / 99: the line
-// lies where calm fluid gains no more.
-constexpr uint32_t kCoopMaxGrid = 120000;
+// Calm scenes near the line, one / several: dam break of 120,000 100 / 94, 124,000
+// 145 / 99, 128,000 96 / 99, 131,072 97.5 / 100; 16 scenes 120,000 107 / 84,
+// 124,000 113 / 93, 128,000 92 / 92; 64 scenes 128,000 107 / 90, 131,072 87 / 94:
+// whole waves per scene favour one work-item, and round sizes have them.
+constexpr uint32_t kCoopMaxGrid = 127000;
 constexpr uint32_t kCoopMaxReference = 1u << 24;
 
 // Slots that the several-work-item gathers' grid covers for n particles in a

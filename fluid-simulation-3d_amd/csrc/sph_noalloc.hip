@@ -262,7 +262,7 @@ extern "C" int sph_update_noalloc(const sph_params *p, uint32_t n, float dt, con
         NA(sph::launch_bucket_sort(s, c, st), "bucket sort");
         // 40 words a particle or more: rows of 80 to 128 neighbours, where nbr by
         // itself holds 48, which random fluid passes (65,536 particles, 12 a cell:
-        // 184 us, now 117; 147 with one work-item per particle)
+        // 184 -> 89 us; 147 with one work-item per particle)
         s.nbr = at<uint32_t>(base, kLayout.rows);
         s.nbr_words = (uint32_t)std::min<size_t>(64, (kLayout.total - kLayout.rows) / (4 * (size_t)n));
         s.spare = at<uint32_t>(base, kLayout.vs2);  // (pressure's, which comes later)

@@ -61,8 +61,8 @@ CASES = {
     "differences, 24": lambda: _scene(70001, 24.0),
     "differences, 40, one outside": lambda: _scene(70001, 40.0, outside=True),
     "differences that do not fit": lambda: _scene(110000, None, box=(0.3, 23.0, 23.0)),
-    "the last size": lambda: _scene(120000, 16.0),
-    "the first size of the masks": lambda: _scene(120001, 16.0),
+    "the last size": lambda: _scene(127000, 16.0),
+    "the first size of the masks": lambda: _scene(127001, 16.0),
     "eight cells": lambda: _clump(3001, 2),
     "one cell": lambda: _clump(1500, 1),
     "64 cells, narrow lanes": lambda: _clump(17000, 4),
