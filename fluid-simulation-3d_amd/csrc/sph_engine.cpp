@@ -1139,7 +1139,9 @@ int Engine::prime(std::string *err)
         sd_h_[q].lookahead = 0.0f;
     }
     rc = push_descs(err);
-    const LaunchCfg cfg = run_cfg();
+    // (density alone: nobody reads the lists that several work-items leave)
+    LaunchCfg cfg = run_cfg();
+    if (!grid_ && ed_h_->n_total > kCoopMaxReferencePrime) cfg.coop_n = 0;
     hipError_t e = rc ? hipSuccess : launch_predict(d_, cfg, stream_);
     if (!rc && e == hipSuccess && !grid_ && !cfg.coop_n && cfg.needs_work()) {
         int wb = 0;

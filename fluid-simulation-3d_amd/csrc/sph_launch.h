@@ -194,6 +194,11 @@ inline LaunchCfg limit_launch_cfg(LaunchCfg c, bool all_fast)
 // whole waves per scene favour one work-item, and round sizes have them.
 constexpr uint32_t kCoopMaxGrid = 127000;
 constexpr uint32_t kCoopMaxReference = 1u << 24;
+// The same for the density pass of InitializeData under the reference key, which
+// no pressure follows; us of sph_initialize with one / several work-items:
+// 200,000: 198 / 165   700,000: 462 / 431   1,000,000: 684 / 729   2,500,000 (40 a
+// cell): 2,294 / 4,777.
+constexpr uint32_t kCoopMaxReferencePrime = 700000;
 
 // Slots that the several-work-item gathers' grid covers for n particles in a
 // layout of `capacity` slots, or 0 when the one-work-item forms run.
