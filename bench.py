@@ -74,41 +74,29 @@ def sub_dt(dt=W.DT, substeps=W.SUBSTEPS):
     return float(np.float32(np.float32(dt) / np.float32(substeps)))
 
 
-# the default gather variants (work, list, block, rows): with them small scenes
-# run the forms with several work-items per particle
-DEFAULTS = {True: {"density": (0, 0, 256, 1), "pressure": (0, 0, 256, 1), "viscosity": (0, 0, 256, 1), "nbr": 1},
-            False: {"density": (0, 0, 64, 0), "pressure": (1, 1, 64, 0), "viscosity": (0, 0, 64, 0), "nbr": 0}}
-
-
-def is_default(variants, grid):
-    return all(DEFAULTS[grid][k] == (tuple(int(v[x]) for x in ("work", "list", "block", "rows"))
-                                     if isinstance(v, dict) else int(v))
-               for k, v in variants.items() if k in DEFAULTS[grid])
-
-
-def kernel_name(stage, variants, grid, multi=False, n=None):
-    """Template instantiation that runs `stage` for n particles under the gather
-    variants `variants` (kernel<MULTI, WORK, LIST, NBR, GRID>; several work-items
-    per particle: kernel<lanes, MULTI, GRID, list entry>)."""
+def kernel_name(stage, variants, grid, multi=False, form=(1, 0)):
+    """Template instantiation that runs `stage` under the gather variants
+    `variants` (kernel<MULTI, WORK, LIST, NBR, GRID, FAST>; with several
+    work-items per particle, `form` of the handle: kernel<lanes, MULTI, GRID,
+    list entry>)."""
     m = "true" if multi else "false"
     b = lambda x: "true" if x else "false"  # noqa: E731
-    if n is not None and n <= (1 << 17 if grid else 1 << 24) and is_default(variants, grid):
-        return (f"k_coop_{stage.split('_')[0]}<{16 if n <= 16384 else 8}u, {m}, {b(grid)}, "
-                f"unsigned {'short' if n <= 65536 else 'int'}>")
+    if form[0] > 1:
+        entry = {16: "unsigned short", -16: "short", 32: "unsigned int"}[form[1]]
+        return f"k_coop_{stage.split('_')[0]}<{form[0]}u, {m}, {b(grid)}, {entry}>"
     if stage == "density" and variants["nbr"] and not grid:
         return f"k_density_rows<{m}>"
     base = {"density": "k_density", "pressure": "k_pressure",
             "viscosity_integrate": "k_viscosity_integrate"}[stage]
     v = variants[stage.split("_")[0]]
     if grid:
-        if stage == "density":
-            return f"{base}<{m}, false, {b(v['list'])}, {b(variants['nbr'])}, true>"
-        if variants["nbr"] and v["rows"]:
-            return f"{base}<{m}, false, false, true, true>"
-        return f"{base}<{m}, false, {b(v['list'])}, false, true>"
+        if variants["nbr"] and (stage == "density" or v["rows"]):
+            lst = stage == "density" and v["list"]
+            return f"{base}<{m}, false, {b(lst)}, true, true, {b(not lst)}>"
+        return f"{base}<{m}, false, {b(v['list'])}, false, true, false>"
     if variants["nbr"] and v["rows"]:
-        return f"{base}<{m}, true, false, true, false>"
-    return f"{base}<{m}, {b(v['work'])}, {b(v['list'])}, false, false>"
+        return f"{base}<{m}, true, false, true, false, false>"
+    return f"{base}<{m}, {b(v['work'])}, {b(v['list'])}, false, false, false>"
 
 
 # committed counter summaries are named for the workload's short name
@@ -154,14 +142,14 @@ def valu_issue(workload, kernel, ms):
                      f"{t['clock_ghz']} GHz"}
 
 
-def gather_fractions(workload, n, variants, grid, per, multi):
+def gather_fractions(workload, n, variants, grid, per, multi, form):
     """HBM and VALU fractions of each gather pass at its live duration:
     algorithmic bytes / duration / 8 TB/s, the committed measured traffic /
     duration / 8 TB/s, and the VALU issue share from the committed
     instruction count."""
     out = {}
     for stage in GATHER:
-        kern = kernel_name(stage, variants, grid, multi, n)
+        kern = kernel_name(stage, variants, grid, multi, form)
         ms = per[stage]
         traffic = measured_traffic(workload, kern)
         valu = valu_issue(workload, kern, ms)
@@ -174,14 +162,14 @@ def gather_fractions(workload, n, variants, grid, per, multi):
     return out
 
 
-def roofline(workload, n, variants, grid, per, multi):
+def roofline(workload, n, variants, grid, per, multi, form):
     """Roofline of the dominant gather kernel against HBM.  No MFMA work
     exists in this path (no dense contraction; the committed counters show
     zero MFMA instructions), so the roofline is HBM's; `limiter` names what
     the committed counters show bounds the kernel at its live duration: the
     larger of its VALU issue share and its measured-traffic share of HBM."""
     dom = max(GATHER, key=lambda k: per[k])
-    kern = kernel_name(dom, variants, grid, multi, n)
+    kern = kernel_name(dom, variants, grid, multi, form)
     ms = per[dom]
     ach = ALG_BYTES[dom] * n / (ms * 1e-3) / 1e9
     traffic = measured_traffic(workload, kern)
@@ -245,7 +233,7 @@ def bench_batch(steps, warmup, plain_steps, latency_steps, plain=True):
         t = time.perf_counter()
         b.step(bs.dt, bs.substeps)
         lat.append((time.perf_counter() - t) * 1e3)
-    variants = b.variants
+    variants, form = b.variants, b.form
     b.close()
     log(f"[bench] batched {steps} steps in {el_b:.3f} s")
 
@@ -256,8 +244,8 @@ def bench_batch(steps, warmup, plain_steps, latency_steps, plain=True):
            "step_latency_ms": {"p50": float(np.percentile(lat, 50)),
                                "p99": float(np.percentile(lat, 99)), "n": len(lat)},
            "stage_ms_per_update": per, "gather_variants": variants,
-           "roofline": roofline(bs.name, total, variants, True, per, True),
-           "gather_kernels": gather_fractions(bs.name, total, variants, True, per, True)}
+           "roofline": roofline(bs.name, total, variants, True, per, True, form),
+           "gather_kernels": gather_fractions(bs.name, total, variants, True, per, True, form)}
     if not plain:
         return out
     sims = []
@@ -330,7 +318,7 @@ def bench_scene(sc, steps, warmup, key="grid", latency_steps=20, autotune=True, 
         sim.step(sc.dt, sc.substeps)
         lat.append((time.perf_counter() - t) * 1e3)
     nonfinite = sim.count_nonfinite()
-    variants = sim.variants
+    variants, form = sim.variants, sim.form
     buckets = sim.table
     sim.close()
     per = {STAGES[i]: float(stage_ms[i]) for i in range(5)}
@@ -343,7 +331,7 @@ def bench_scene(sc, steps, warmup, key="grid", latency_steps=20, autotune=True, 
                                "p99": float(np.percentile(lat, 99)), "n": len(lat)},
            "stage_ms_per_update": per, "gather_variants": variants,
            "nonfinite_components": nonfinite}
-    out["gather_kernels"] = gather_fractions(sc.name, sc.n, variants, grid, per, False)
+    out["gather_kernels"] = gather_fractions(sc.name, sc.n, variants, grid, per, False, form)
     out["step_roofline"] = step_roofline(out["value"], sc.substeps, buckets / sc.n)
     return out
 

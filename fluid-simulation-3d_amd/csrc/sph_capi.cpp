@@ -585,6 +585,29 @@ int sph_batch_set_variants(sph_batch b, const int32_t v[14])
     return set_variants(b->eng, v);
 }
 
+namespace {
+int gather_form(const sph::Engine *e, int32_t form[2])
+{
+    if (!form) return fail(SPH_ERR_INVALID, "null output");
+    const sph::CoopForm f = e->gather_form();
+    form[0] = f.lanes;
+    form[1] = f.entry;
+    return SPH_OK;
+}
+}  // namespace
+
+int sph_debug_form(sph_handle h, int32_t form[2])
+{
+    SPH_NEED(h);
+    return gather_form(h->eng, form);
+}
+
+int sph_batch_debug_form(sph_batch b, int32_t form[2])
+{
+    SPH_NEED(b);
+    return gather_form(b->eng, form);
+}
+
 int sph_debug_set_scan_spin(sph_handle h, uint32_t sleeps)
 {
     SPH_GUARD_BEGIN

@@ -691,13 +691,6 @@ inline uint32_t coop_grid(uint32_t n)
     return ((n + N - 1) / N + 7u) & ~7u;  // XCD numbering: a multiple of 8
 }
 
-// Up to this many slots a group is 16 lanes, above it 8: twice the particles
-// per wave, fewer idle lanes in runs of 24 slots.  Measured, us per steady
-// update with 16 / 8 lanes: 1,000: 26.5 / 30.4, 8,000: 29.8 / 32.0, 16,384:
-// 33.8 / 34.2, 32,768: 46.0 / 40.5, 131,072: 113.7 / 93.7.
-constexpr uint32_t kCoopWide = 16384;
-static_assert(kCoopWide <= 65536u, "16-bit rows");
-
 CoopArgs coop_args(const DevState &s)
 {
     return CoopArgs{s.ed, s.sd, s.scene_of, s.sids, s.xps, s.bounds, s.sflags, s.ncnt, nullptr};
@@ -721,13 +714,13 @@ Rows<T> coop_rows(const DevState &s)
     } while (0)
 #define SPH_COOP_LAUNCH(KER, n, st, ...)                                                           \
     do {                                                                                           \
-        const bool wide_ = n <= kCoopWide, short_ = s.capacity <= 65536u;                          \
-        if (s.grid && wide_) SPH_COOP_LAUNCH_T(KER, 16, true, uint16_t, n, st, __VA_ARGS__);       \
-        else if (s.grid && short_) SPH_COOP_LAUNCH_T(KER, 8, true, uint16_t, n, st, __VA_ARGS__);  \
-        else if (s.grid) SPH_COOP_LAUNCH_T(KER, 8, true, int16_t, n, st, __VA_ARGS__);             \
-        else if (wide_) SPH_COOP_LAUNCH_T(KER, 16, false, uint16_t, n, st, __VA_ARGS__);           \
-        else if (short_) SPH_COOP_LAUNCH_T(KER, 8, false, uint16_t, n, st, __VA_ARGS__);           \
-        else SPH_COOP_LAUNCH_T(KER, 8, false, uint32_t, n, st, __VA_ARGS__);                       \
+        const CoopForm f_ = coop_form(s.grid, n, s.capacity);                                      \
+        if (s.grid && f_.lanes == 16) SPH_COOP_LAUNCH_T(KER, 16, true, uint16_t, n, st, __VA_ARGS__);       \
+        else if (s.grid && f_.entry == 16) SPH_COOP_LAUNCH_T(KER, 8, true, uint16_t, n, st, __VA_ARGS__);   \
+        else if (s.grid) SPH_COOP_LAUNCH_T(KER, 8, true, int16_t, n, st, __VA_ARGS__);                      \
+        else if (f_.lanes == 16) SPH_COOP_LAUNCH_T(KER, 16, false, uint16_t, n, st, __VA_ARGS__);           \
+        else if (f_.entry == 16) SPH_COOP_LAUNCH_T(KER, 8, false, uint16_t, n, st, __VA_ARGS__);            \
+        else SPH_COOP_LAUNCH_T(KER, 8, false, uint32_t, n, st, __VA_ARGS__);                                \
     } while (0)
 
 }  // namespace

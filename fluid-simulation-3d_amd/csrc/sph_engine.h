@@ -141,6 +141,12 @@ class Engine {
     // Which kernels an update of the present layout runs, under one setting of the
     // variants: 0 one work-item per particle, 1 several, 2 one, with IEEE operations.
     int form() const { return !all_fast_ ? 2 : coop_slots_now() ? 1 : 0; }
+    // Work-items per particle and list entry (coop_form; 1, 0: neither).
+    CoopForm gather_form() const
+    {
+        const uint32_t n = coop_slots_now();
+        return n ? coop_form(grid_, n, d_.capacity) : CoopForm{1, 0};
+    }
     // The variants that an update of the present layout runs.
     LaunchCfg run_cfg() const
     {

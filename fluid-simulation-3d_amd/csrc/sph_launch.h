@@ -208,6 +208,22 @@ inline uint32_t coop_slots(bool grid, uint32_t n, uint32_t capacity)
     return n > most ? 0u : (capacity < most ? capacity : most);
 }
 
+// Their form for n slots: work-items per particle, and what an entry of a
+// neighbour list is: 16 a slot in 16 bits, -16 the difference to the particle's
+// own, 32 a slot in 32 bits.  Up to kCoopWide slots a particle has 16 lanes,
+// above 8: twice the particles per wave, fewer idle lanes in runs of 24 slots.
+// us per steady update with 16 / 8 lanes: 1,000: 26.5 / 30.4, 8,000: 29.8 / 32.0,
+// 16,384: 33.8 / 34.2, 32,768: 46.0 / 40.5, 131,072: 113.7 / 93.7.
+constexpr uint32_t kCoopWide = 16384;
+struct CoopForm {
+    int lanes, entry;
+};
+inline CoopForm coop_form(bool grid, uint32_t n, uint32_t capacity)
+{
+    if (n <= kCoopWide && capacity <= 65536u) return CoopForm{16, 16};
+    return CoopForm{8, capacity <= 65536u ? 16 : grid ? -16 : 32};
+}
+
 // Rows per strip of the grid key's bucket order, log2 (grid_row), for a scene
 // of n particles.  A gather reads three planes around its own, and an XCD works
 // on a window of some 40,000 slots (32 CUs of 16 to 24 waves).  Once planes hold

@@ -155,6 +155,8 @@ def lib():
         "sph_debug_predicted": (i32, [H, p]),
         "sph_debug_velocities": (i32, [H, p, p]),
         "sph_debug_set_scan_spin": (i32, [H, u32]),
+        "sph_debug_form": (i32, [H, p]),
+        "sph_batch_debug_form": (i32, [H, p]),
         "sph_debug_neighbours": (i32, [H, p, p, u64, p]),
         "sph_generate": (i32, [i32, u64, u32, p, f, f, f, p, p]),
         "sph_server_default_config": (None, [ctypes.POINTER(ServerConfig)]),
@@ -287,6 +289,12 @@ def _variants_dict(v):
     if v[13] == 2:  # one work-item per particle at every size
         d["pinned"] = True
     return d
+
+
+def _form(fn, h):
+    f = np.zeros(2, np.int32)
+    _check(fn(h, _ptr(f)))
+    return int(f[0]), int(f[1])
 
 
 def _variants_array(d):
@@ -422,6 +430,11 @@ class Sim:
     @variants.setter
     def variants(self, d):
         _check(lib().sph_set_variants(self._h, _ptr(_variants_array(d))))
+
+    @property
+    def form(self):
+        """(work-items per particle, list entry) of the next update's gathers."""
+        return _form(lib().sph_debug_form, self._h)
 
     def debug_set_scan_spin(self, sleeps):
         """Bound of the count scan's look-back wait (64-clock sleeps); 0 makes
@@ -560,6 +573,10 @@ class Batch:
     @variants.setter
     def variants(self, d):
         _check(lib().sph_batch_set_variants(self._h, _ptr(_variants_array(d))))
+
+    @property
+    def form(self):
+        return _form(lib().sph_batch_debug_form, self._h)
 
 
 def request_bytes(params, n, table=0):

@@ -216,6 +216,11 @@ int sph_autotune(sph_handle h, float dt, int updates, double ms[3]);
  * entries. */
 int sph_get_variants(sph_handle h, int32_t v[14]);
 int sph_set_variants(sph_handle h, const int32_t v[14]);
+/* Test support, no reference counterpart: the form of the gather kernels in the
+ * next update: form[0] work-items per particle (1, 8 or 16), form[1] the entries
+ * of their neighbour lists (0 none, 16 or 32 slots in so many bits, -16
+ * differences of slots). */
+int sph_debug_form(sph_handle h, int32_t form[2]);
 /* Test support, no reference counterpart: the bound of the count scan's
  * look-back wait (the prefix sum behind the bucket table of UpdateSpatialLookup,
  * cc:486-496), in sleeps of 64 clocks; 65536 by default, about 1.7 ms.  A
@@ -337,6 +342,7 @@ int sph_batch_profile_begin(sph_batch b, uint32_t max_updates);
 int sph_batch_profile_end(sph_batch b, double mean_ms[6], uint32_t *updates);
 int sph_batch_get_variants(sph_batch b, int32_t v[14]);
 int sph_batch_set_variants(sph_batch b, const int32_t v[14]);
+int sph_batch_debug_form(sph_batch b, int32_t form[2]);
 
 /* ---- serving: continuous batching of bake requests ----
  * No reference counterpart.  A request is a scene (settings, particle count,

@@ -27,15 +27,16 @@ def test_pinned_variants_round_trip(key):
         default = a.variants
         assert "pinned" not in default and not default["fused"]
         want = _run(a, sc)
+        assert a.form == (16, 16)
         a.variants = dict(default, pinned=True)
-        assert a.variants == dict(default, pinned=True)
+        assert a.variants == dict(default, pinned=True) and a.form == (1, 0)
         b.variants = a.variants
-        assert b.variants == a.variants
+        assert b.variants == a.variants and b.form == (1, 0)
         for sim in (a, b):
             for g, w, what in zip(_run(sim, sc), want, ("positions", "velocities", "densities")):
                 assert_bitexact(g, w, what)
         a.variants = default
-        assert a.variants == default
+        assert a.variants == default and a.form == (16, 16)
 
 
 @pytest.mark.parametrize("key", [S.TABLE_GRID, S.TABLE_REFERENCE])
@@ -47,6 +48,19 @@ def test_tuned_variants_round_trip(key):
         a.autotune(W.DT / W.SUBSTEPS, 2)
         tuned = a.variants
         b.variants = tuned
-        assert b.variants == tuned
-        # a pick equal to the defaults that is not pinned is the defaults' own form
+        assert b.variants == tuned and b.form == a.form
         assert np.array_equal(_run(a, sc)[0], _run(b, sc)[0])
+
+
+@pytest.mark.parametrize("n,grid,reference", [
+    (1, (16, 16), (16, 16)), (16384, (16, 16), (16, 16)), (16385, (8, 16), (8, 16)), (65536, (8, 16), (8, 16)),
+    (65537, (8, -16), (8, 32)), (127000, (8, -16), (8, 32)), (127001, (1, 0), (8, 32)),
+])
+def test_default_form_by_size(n, grid, reference):
+    announce("form by size", n)
+    p = W.scene_params()
+    with S.Sim(p, n, S.TABLE_GRID) as a, S.Sim(p, n, S.TABLE_REFERENCE) as b:
+        assert a.form == grid and b.form == reference
+        p.prefilter_r2 = 2.0 ** -62  # outside the fast arithmetic's range
+        a.params = b.params = p
+        assert a.form == b.form == (1, 0)
