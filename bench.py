@@ -99,39 +99,39 @@ def kernel_name(stage, variants, grid, multi=False, form=(1, 0)):
     return f"{base}<{m}, {b(v['work'])}, {b(v['list'])}, false, false, false>"
 
 
-# committed counter summaries are named for the workload's short name
-PROFILE_FILES = {"batch_256": "batch_256", "uniform_1048576": "uniform_1m",
-                 "two_blocks_16777216": "two_blocks_16m"}
+# committed counter summaries, by workload: one per form that its legs run
+PROFILE_FILES = {"batch_256": ["batch_256"], "uniform_1048576": ["uniform_1m", "uniform_1m_reference"],
+                 "two_blocks_16777216": ["two_blocks_16m"], "dam_break_16384": ["dam_break_16k"]}
 
 
-def _profile(name):
-    try:
-        with open(os.path.join(PROFILES, name)) as f:
-            return json.load(f)
-    except (OSError, ValueError):
-        return None
+def _profile(workload, kind, kernel):
+    """(summary, entry) of `kernel` in profiles/<short name>_<kind>.json, or None."""
+    for name in PROFILE_FILES.get(workload, [workload]):
+        try:
+            with open(os.path.join(PROFILES, f"{name}_{kind}.json")) as f:
+                t = json.load(f)
+        except (OSError, ValueError):
+            continue
+        if t.get("workload") == workload and kernel in t.get("kernels", {}):
+            return t, t["kernels"][kernel]
+    return None
 
 
 def measured_traffic(workload, kernel):
     """HBM bytes per launch of `kernel` from the committed counter summary of
-    `workload` (profiles/<short name>_traffic.json), or None."""
-    t = _profile(f"{PROFILE_FILES.get(workload, workload)}_traffic.json")
-    if not t or t.get("workload") != workload:
-        return None
-    k = t.get("kernels", {}).get(kernel)
-    return None if k is None else float(k["traffic_bytes"])
+    `workload`, or None."""
+    found = _profile(workload, "traffic", kernel)
+    return None if found is None else float(found[1]["traffic_bytes"])
 
 
 def valu_issue(workload, kernel, ms):
     """VALU issue fraction of `kernel` at duration `ms`, from its committed
     instruction count (rocprofv3 SQ_INSTS_VALU): instructions x 2 cycles (a
     wave64 VALU instruction on a 32-lane SIMD) / (1024 SIMDs x 2.4 GHz x ms)."""
-    t = _profile(f"{PROFILE_FILES.get(workload, workload)}_valu.json")
-    if not t or t.get("workload") != workload:
+    found = _profile(workload, "valu", kernel)
+    if found is None:
         return None
-    k = t.get("kernels", {}).get(kernel)
-    if k is None:
-        return None
+    t, k = found
     instr = float(k["valu_instr_per_launch"])
     cyc = t["cycles_per_wave64_valu"]
     return {"kernel": kernel, "instr_per_launch": instr,

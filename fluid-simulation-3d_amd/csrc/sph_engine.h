@@ -132,7 +132,7 @@ class Engine {
         return cfg_.fused && grid_ && cfg_.nbr && cfg_.density.rows && cfg_.pressure.rows &&
                cfg_.viscosity.rows && !rebuild_work && !fresh && d_.fused_grid[all_fast_ ? 0 : 1] != 0;
     }
-    // Slots of the sixteen-work-item gathers' grid for the present layout (0:
+    // Slots of the several-work-item gathers' grid for the present layout (0:
     // the one-work-item forms run).
     uint32_t coop_slots_now() const
     {

@@ -1,5 +1,5 @@
 // sph_kernel_common.h -- device functions shared by the gfx950 kernels of
-// sph_kernels.hip (one work-item per particle) and sph_coop.hip (sixteen
+// sph_kernels.hip (one work-item per particle) and sph_coop.hip (16 or 8
 // work-items per particle): the scene loop, stage A, the bucket of a particle
 // and the pair terms of stages C to F.  Every floating-point expression keeps
 // the reference's operation order and rounding, so the two forms of a stage

@@ -612,12 +612,12 @@ __global__ __launch_bounds__(kReorderBlock) void k_count_reorder(
 // writes them.  What bounds a sort of this size is the chain of
 // dependent loads, each some 600 ns (the data come from other XCDs): the scan,
 // scatter and reorder launches make about twelve and start three times, this
-// one makes four (12.6 -> 10.3 us of kernel time at 16,384 particles, 9.9 ->
-// 7.1 at 1,000) -- counts and
-// keys together, then ticket, index, position and velocity of the particles found, whose ranks are taken in LDS.  Each workgroup reads all keys, so it
-// is kept to kSmallSortMax particles.  A workgroup with more than kSmallOwn particles
-// (compressed fluid, tiny tables) puts them in ticket order in `order` and
-// runs the reorder over them.  The counts stay as they are (other workgroups
+// one makes four (12.6 -> 10.3 us of kernel time at 16,384 particles, 9.9 -> 7.1
+// at 1,000): counts and keys together, then ticket, index, position and velocity
+// of the particles found, whose ranks are taken in LDS.  Each workgroup reads all
+// keys, so it is kept to kSmallSortMax particles.  A workgroup with more than
+// kSmallOwn particles (compressed fluid, tiny tables) puts them in ticket order
+// in `order` and runs the reorder over them.  The counts stay as they are (other workgroups
 // read them): the density pass that follows clears them.  ids null: the
 // resident order is particle order.
 constexpr uint32_t kFlight = 8;                                // 16-byte loads in flight per work-item

@@ -97,7 +97,7 @@ struct LaunchCfg {
     // one work-item per particle at every size, also where the variants are the
     // defaults (whose form else follows the scene's size, coop_slots)
     bool pinned = false;
-    // > 0: the gathers run with sixteen work-items per particle, over a grid
+    // > 0: the gathers run with several work-items per particle, over a grid
     // of this many slots (follows_size, set per update by the engine)
     uint32_t coop_n = 0;
     // the bucket sort is one launch, and the density pass clears its counts
@@ -238,8 +238,8 @@ inline CoopForm coop_form(bool grid, uint32_t n, uint32_t capacity)
 //   uniform 4,194,304 (33,000)                     1,193 / - / 1,047 / -
 //   uniform 8,388,608 (52,000)                     2,474 / 2,277 / 2,219 / 2,490
 //   two blocks 16,777,216 (82,000, 105,000 inside) 3,574 / 3,276 / 3,223 / 3,395
-// (density gains nothing and loses up to 1%).  Scenes that the sixteen- and
-// eight-work-item gathers may take have none: their fast walk counts on rows
+// (density gains nothing and loses up to 1%).  Scenes that the gathers with
+// several work-items per particle may take have none: their fast walk counts on rows
 // in plane order.
 constexpr uint32_t kStripPlane = 24576, kStripShift = 3;
 inline uint32_t grid_strips(uint32_t n, const uint32_t g[3])
@@ -287,7 +287,7 @@ hipError_t launch_density(const DevState &s, const LaunchCfg &c, hipStream_t st)
 hipError_t launch_pressure(const DevState &s, const LaunchCfg &c, hipStream_t st);
 hipError_t launch_viscosity_integrate(const DevState &s, const LaunchCfg &c, hipStream_t st);
 
-// The same stages with sixteen work-items per particle (sph_coop.hip), over the
+// The same stages with several work-items per particle (sph_coop.hip), over the
 // first n slots (n >= the live particles).
 hipError_t launch_coop_density(const DevState &s, uint32_t n, bool clear_counts, hipStream_t st);
 hipError_t launch_coop_pressure(const DevState &s, uint32_t n, hipStream_t st);

@@ -133,7 +133,8 @@ int sph_initialize(sph_handle h, int kind, uint64_t seed, const float box[3], fl
                    float jitter, float speed);
 /* Render hand-off (FluidSimCPU::updateColors, fluidSimCPU.cc:100-125; the
  * GLSL path's UpdateColors, compute_particle.glsl:279-304): when enabled,
- * every update also writes each particle's speed colour -- the 4-stop
+ * every sph_update, and the last update of a step, also writes each
+ * particle's speed colour -- the 4-stop
  * gradient of clamp(|v|, 0, 1.5) / 1.5 (getSpeedNormalzied,
  * physicsWorld.cc:178-182) -- fused into the integration kernel.  stops:
  * Color1..Color4 as RGBA (16 floats; NULL keeps the current ones, initially
