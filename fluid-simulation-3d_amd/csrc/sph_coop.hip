@@ -6,7 +6,7 @@
 // each a serial chain of some 240 candidate tests and 35 to 50 pair bodies: the
 // stages take that chain's latency (density 36, pressure 21, viscosity 13 us)
 // whatever the size below about 100,000 particles.  Here a group of G lanes
-// takes a particle, and at 16,384 particles they take 9.9, 7.8 and 7.8 us:
+// takes a particle, and at 16,384 particles they take 8.4, 6.1 and 7.2 us:
 //   - the candidates of a neighbour row are tested G at a time, in slot order
 //     (one coalesced load per group), and the passing ones go to a list in LDS
 //     at the place a ballot gives them, so the list has walk order;
@@ -22,7 +22,7 @@
 //
 // The density stage also writes each particle's list (its own slot among it) to
 // the neighbour-row buffer, and the pressure and viscosity stages take it from
-// there; a particle with more neighbours than a row holds walks again.
+// there; a wave with a particle of more neighbours than a row holds walks again.
 //
 // Reference: Allkams/Fluid-Simulation-3D, engine/physics/physicsWorld.cc:304-464
 // (stages C, D, E), cc:80-108 (stage F).
@@ -258,7 +258,7 @@ __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__re
                 e8 = bounds[base + (gy + 1u) * gz + 2u];
             }
             if (!wave_any(re - rb > 3u * kCrowded)) {
-                constexpr int kRows = 3;  // runs in flight together (nine: 122 registers, 8.5 instead of 8.1 us)
+                constexpr int kRows = 3;  // runs in flight together (nine: 122 registers, 0.4 us more at 16,384)
                 static_for<9 / kRows>([&](auto Q) __attribute__((always_inline)) {
                     uint32_t b[kRows], e[kRows];
                     static_for<kRows>([&](auto R) __attribute__((always_inline)) {
