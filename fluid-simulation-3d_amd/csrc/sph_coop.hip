@@ -400,30 +400,25 @@ __device__ __forceinline__ float ordered_sum(float acc, const float *plane, uint
 }
 
 // Rows of the neighbour lists: entry t of slot k at [k * cap + t].  uint16_t:
-// slots, while every slot fits.  int16_t: differences to k, under the grid key,
-// whose neighbours lie within three planes of cells: up to kCoopMaxGrid particles
-// they fit unless a plane holds more than some 30,000 (the particle then walks
-// again).  uint32_t: slots.  In 16 bits a row holds twice as many (70,000
+// slots, while every slot fits.  int16_t: the low 16 bits of slots below 131,072
+// (grid key).  The walk meets slots in ascending order, but for cells that wrap
+// around the grid, so a list's first `split` entries are those below 65,536; the
+// split lies beside the count, and a list that is not so counts as too long for
+// its row.  uint32_t: slots.  In 16 bits a row holds twice as many (70,000
 // colliding particles, mean of 60 steps: 128 us an update with rows of 64, 84 of
 // 128, and the walk in batches).
 template <typename T>
 struct Rows {
+    static constexpr bool kSplit = std::is_signed<T>::value;
     T *rows, *spare;  // spare: a row that nobody reads
     uint32_t cap;
-    __device__ __forceinline__ uint32_t get(uint32_t k, uint32_t t) const
+    __device__ __forceinline__ uint32_t get(uint32_t k, uint32_t t, uint32_t split) const
     {
         const T e = rows[(size_t)k * cap + t];
-        return std::is_signed<T>::value ? k + (uint32_t)(int32_t)e : (uint32_t)e;
-    }
-    static __device__ __forceinline__ T entry(uint32_t k, uint32_t m)
-    {
-        return (T)(std::is_signed<T>::value ? m - k : m);
-    }
-    static __device__ __forceinline__ bool holds(uint32_t k, uint32_t m)
-    {
-        return !std::is_signed<T>::value || m - k + 32768u < 65536u;
+        return kSplit ? (uint32_t)(uint16_t)e + (t < split ? 0u : 65536u) : (uint32_t)e;
     }
 };
+static_assert(kCoopMaxGrid <= 131072u, "17 bits of slots");
 
 struct CoopArgs {
     const EngineDesc *ed;
@@ -460,7 +455,8 @@ __global__ __launch_bounds__(kCoopBlock, 5) void k_coop_density(const CoopArgs A
         const float h = S.h, w2c = S.w2c, w3c = S.w3c;
         float acc = 0.0f;    // lane 0: rho, lane 1: near rho
         uint32_t total = 0;  // neighbours flushed so far
-        bool far = false;    // one of this lane's does not fit a row entry
+        uint32_t split = 0;  // neighbours below slot 65,536
+        bool mixed = false;  // one of them after a slot past it
         auto flush = [&](uint32_t cnt) {
             wave_sync();
             for (uint32_t c0 = 0; wave_any(c0 < cnt); c0 += kChunk) {
@@ -478,8 +474,15 @@ __global__ __launch_bounds__(kCoopBlock, 5) void k_coop_density(const CoopArgs A
                     t0p[r + gl] = have ? a : 0.0f;
                     t1p[r + gl] = have ? b : 0.0f;
                     T *const row = cnt ? out.rows + (size_t)k * out.cap : out.spare;
-                    row[min(total + at, out.cap - 1u)] = Rows<T>::entry(k, e.x);
-                    far |= have & !Rows<T>::holds(k, e.x);
+                    row[min(total + at, out.cap - 1u)] = (T)e.x;
+                    if constexpr (Rows<T>::kSplit) {
+                        const uint32_t lane = threadIdx.x & 63u;
+                        const uint64_t b = __ballot(have & (e.x < 65536u));
+                        const uint32_t half = (lane & 32u) ? (uint32_t)(b >> 32) : (uint32_t)b;
+                        const uint32_t low = (half >> (lane & (32u - G))) & ((1u << G) - 1u);
+                        mixed |= low != 0u && (split != total + c0 + r || (low & (low + 1u)) != 0u);
+                        split += (uint32_t)__popc(low);
+                    }
                 }
                 wave_sync();
                 acc = ordered_sum(acc, gl == 0u ? t0p : t1p, cnt > c0 ? min(kChunk, cnt - c0) : 0u);
@@ -490,10 +493,7 @@ __global__ __launch_bounds__(kCoopBlock, 5) void k_coop_density(const CoopArgs A
         coop_walk<G, GRID, true>(
             S, A.xps, A.bounds, k, pi, clean,
             [&](uint32_t at, uint32_t m, float d2) { lst[at] = make_uint2(m, __float_as_uint(d2)); }, flush);
-        if constexpr (std::is_signed<T>::value) {
-            const uint64_t fars = __ballot(far);
-            if ((fars >> (threadIdx.x & 63u & ~(G - 1u))) & ((1ull << G) - 1ull)) total = out.cap + 1u;
-        }
+        if constexpr (Rows<T>::kSplit) total = mixed || total > out.cap ? out.cap + 1u : total | split << 16;
         const float rho = group_bcast<G, 0>(acc), rhon = group_bcast<G, 1>(acc);
         if (gl == 0u) {
             A.ncnt[k] = total;
@@ -517,7 +517,7 @@ __device__ __forceinline__ float coop_sum(const CoopArgs &A, const SceneDesc &S,
     const uint32_t gl = threadIdx.x & (G - 1u);
     const float *const mine = planes + min(gl, 2u) * kPlane;
     float acc = 0.0f;
-    const uint32_t total = A.ncnt[k];
+    const uint32_t found = A.ncnt[k], split = found >> 16, total = Rows<T>::kSplit ? found & 0xffffu : found;
     // (the two ways share nothing: most waves take the first, which then needs
     // neither the cell nor the registers of the walk)
     auto take = [&](auto from_rows, uint32_t cnt) __attribute__((always_inline)) {
@@ -530,7 +530,7 @@ __device__ __forceinline__ float coop_sum(const CoopArgs &A, const SceneDesc &S,
 #pragma unroll
             for (uint32_t r = 0; r < R; ++r) {
                 const uint32_t t = c0 + r * G + gl, at = t < cnt ? t : 0u;
-                const uint32_t e = decltype(from_rows)::value ? in.get(k, at) : lst[at];
+                const uint32_t e = decltype(from_rows)::value ? in.get(k, at, split) : lst[at];
                 m[r] = t < cnt ? e : k;
             }
 #pragma unroll

@@ -209,8 +209,8 @@ inline uint32_t coop_slots(bool grid, uint32_t n, uint32_t capacity)
 }
 
 // Their form for n slots: work-items per particle, and what an entry of a
-// neighbour list is: 16 a slot in 16 bits, -16 the difference to the particle's
-// own, 32 a slot in 32 bits.  Up to kCoopWide slots a particle has 16 lanes,
+// neighbour list is: 16 a slot in 16 bits, -16 the low 16 of 17 bits, 32 a slot in
+// 32 bits.  Up to kCoopWide slots a particle has 16 lanes,
 // above 8: twice the particles per wave, fewer idle lanes in runs of 24 slots.
 // us per steady update with 16 / 8 lanes: 1,000: 26.5 / 30.4, 8,000: 29.8 / 32.0,
 // 16,384: 33.8 / 34.2, 32,768: 46.0 / 40.5, 131,072: 113.7 / 93.7.

@@ -219,8 +219,8 @@ int sph_get_variants(sph_handle h, int32_t v[14]);
 int sph_set_variants(sph_handle h, const int32_t v[14]);
 /* Test support, no reference counterpart: the form of the gather kernels in the
  * next update: form[0] work-items per particle (1, 8 or 16), form[1] the entries
- * of their neighbour lists (0 none, 16 or 32 slots in so many bits, -16
- * differences of slots). */
+ * of their neighbour lists (0 none, 16 or 32 slots in so many bits, -16 the
+ * low 16 bits of slots). */
 int sph_debug_form(sph_handle h, int32_t form[2]);
 /* Test support, no reference counterpart: the bound of the count scan's
  * look-back wait (the prefix sum behind the bucket table of UpdateSpatialLookup,

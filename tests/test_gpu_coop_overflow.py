@@ -1,7 +1,8 @@
 """Several work-items per particle where the neighbour lists end: lists longer
 than a row (48 to 128 entries by size and key) or than the LDS holds (96), one
-batch of cells alone past that, rows of slot differences that do not fit 16
-bits, and the last size that takes these forms; single scenes, batches and
+batch of cells alone past that, rows of 17-bit slots in 16 bits (thin scenes,
+whose neighbours lie far apart in slots, and a grid that wraps, which breaks the
+order that they count on), and the last size that takes these forms; single scenes, batches and
 sph_update_noalloc, bit-exact against the oracle."""
 import numpy as np
 import pytest
@@ -17,7 +18,7 @@ DT = float(np.float32(np.float32(W.DT) / np.float32(W.SUBSTEPS)))
 H = 0.2
 
 
-def _scene(n, per_cell, seed=1, box=None, outside=False):
+def _scene(n, per_cell, seed=1, box=None, outside=False, tall=None):
     """n particles, per_cell a cell on average, in the lower half of a box (or all of the one given)."""
     lower = 0.5 if box is None else 1.0
     if box is None:
@@ -29,6 +30,8 @@ def _scene(n, per_cell, seed=1, box=None, outside=False):
     pos[:, :3] = (u * box).astype(np.float32)
     if outside:
         pos[n // 2, :3] = 40.0
+    if tall is not None:  # the particles in `box`, the settings' box a cube
+        box = (tall, tall, tall)
     vel = np.zeros((n, 4), np.float32)
     vel[:, :3] = (r.random((n, 3)) - 0.5).astype(np.float32)
     return W.Scene("random", W.scene_params(h=H, rho0=8 / H**3, box=box), n, n, pos, vel, 1)
@@ -57,10 +60,15 @@ CASES = {
     "wide lanes, 40, one outside": lambda: _scene(5003, 40.0, outside=True),
     "16-bit slots, 24": lambda: _scene(40001, 24.0),
     "16-bit slots, 40": lambda: _scene(40001, 40.0),
-    "differences, 12": lambda: _scene(65537, 12.0),
-    "differences, 24": lambda: _scene(70001, 24.0),
-    "differences, 40, one outside": lambda: _scene(70001, 40.0, outside=True),
-    "differences that do not fit": lambda: _scene(110000, None, box=(0.3, 23.0, 23.0)),
+    "17-bit slots, 12": lambda: _scene(65537, 12.0),
+    "17-bit slots, 24": lambda: _scene(70001, 24.0),
+    "17-bit slots, 40, one outside": lambda: _scene(70001, 40.0, outside=True),
+    "17-bit slots, two planes": lambda: _scene(110000, None, box=(0.3, 23.0, 23.0)),
+    "17-bit slots, one plane": lambda: _scene(126001, None, box=(0.15, 25.0, 25.0)),
+    "17-bit slots, three cells in a row": lambda: _scene(90001, None, box=(23.0, 23.0, 0.3)),
+    "a grid that wraps along z": lambda: _scene(70001, None, box=(30.0, 30.0, 0.5), tall=30.0),
+    "a grid that wraps": lambda: _scene(70001, None, box=(6.0, 6.0, 6.0), tall=30.0),
+    "a grid that wraps along x": lambda: _scene(70001, None, box=(0.5, 30.0, 30.0), tall=30.0),
     "the last size": lambda: _scene(127000, 16.0),
     "the first size of the masks": lambda: _scene(127001, 16.0),
     "eight cells": lambda: _clump(3001, 2),
