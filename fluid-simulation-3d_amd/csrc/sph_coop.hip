@@ -44,6 +44,12 @@ constexpr uint32_t kList = 96;   // list entries per particle held in LDS
 // candidates pass, and 27 cells of 24 then give kList entries.
 constexpr uint32_t kCrowded = 24;
 
+// Eight lanes, grid key: where no row of the wave's particles holds more slots
+// than this, two loads of eight a row instead of four (and a third where it
+// holds more than 16).  us per update, four / two: 127,000 particles at 4 a cell
+// 88 / 82, at 1 a cell 77 / 69; 40,000 at 1 a cell 38 / 35; unchanged at 8 a cell.
+constexpr uint32_t kSparse = 22;
+
 // G lanes per particle.
 template <uint32_t G>
 struct Group {
@@ -257,7 +263,7 @@ __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__re
                 b8 = bounds[base + (gy + 1u) * gz - 1u];
                 e8 = bounds[base + (gy + 1u) * gz + 2u];
             }
-            if (!wave_any(re - rb > 3u * kCrowded)) {
+            auto rows = [&](auto cover) __attribute__((always_inline)) {
                 constexpr int kRows = 3;  // runs in flight together (nine: 122 registers, 0.4 us more at 16,384)
                 static_for<9 / kRows>([&](auto Q) __attribute__((always_inline)) {
                     uint32_t b[kRows], e[kRows];
@@ -271,11 +277,13 @@ __device__ __forceinline__ void coop_walk(const SceneDesc &S, const float4 *__re
                             e[q] = e8;
                         }
                     });
-                    runs(std::integral_constant<int, kRows>{}, std::integral_constant<int, 32>{}, std::false_type{},
-                         b, e, [](auto) { return 0.0f; });
+                    runs(std::integral_constant<int, kRows>{}, cover, std::false_type{}, b, e,
+                         [](auto) { return 0.0f; });
                 });
                 done = !wave_any(cnt > kList);
-            }
+            };
+            if (G == 8 && !wave_any(re - rb > kSparse)) rows(std::integral_constant<int, 16>{});
+            else if (!wave_any(re - rb > 3u * kCrowded)) rows(std::integral_constant<int, 32>{});
         }
     }
     if constexpr (FAST && !GRID) {

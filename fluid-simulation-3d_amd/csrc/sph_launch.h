@@ -191,7 +191,9 @@ inline LaunchCfg limit_launch_cfg(LaunchCfg c, bool all_fast)
 // Calm scenes near the line, one / several: dam break of 120,000 100 / 94, 124,000
 // 145 / 99, 128,000 96 / 99, 131,072 97.5 / 100; 16 scenes 120,000 107 / 84,
 // 124,000 113 / 93, 128,000 92 / 92; 64 scenes 128,000 107 / 90, 131,072 87 / 94:
-// whole waves per scene favour one work-item, and round sizes have them.
+// whole waves per scene favour one work-item, and round sizes have them.  Sparse
+// fluid takes fewer tests, so its line lies lower: 4 particles a cell 127,000:
+// 82 / 82, 2 a cell 100,000: 64 / 63, 1 a cell 80,000: 54 / 52, 127,000: 59 / 69.
 constexpr uint32_t kCoopMaxGrid = 127000;
 constexpr uint32_t kCoopMaxReference = 1u << 24;
 // The same for the density pass of InitializeData under the reference key, which

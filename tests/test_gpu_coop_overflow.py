@@ -2,8 +2,9 @@
 than a row (48 to 128 entries by size and key) or than the LDS holds (96), one
 batch of cells alone past that, rows of 17-bit slots in 16 bits (thin scenes,
 whose neighbours lie far apart in slots, and a grid that wraps, which breaks the
-order that they count on), and the last size that takes these forms; single scenes, batches and
-sph_update_noalloc, bit-exact against the oracle."""
+order that they count on), rows short enough for two loads, and the last size
+that takes these forms; single scenes, batches and sph_update_noalloc, bit-exact
+against the oracle."""
 import numpy as np
 import pytest
 
@@ -69,6 +70,9 @@ CASES = {
     "a grid that wraps along z": lambda: _scene(70001, None, box=(30.0, 30.0, 0.5), tall=30.0),
     "a grid that wraps": lambda: _scene(70001, None, box=(6.0, 6.0, 6.0), tall=30.0),
     "a grid that wraps along x": lambda: _scene(70001, None, box=(0.5, 30.0, 30.0), tall=30.0),
+    "sparse, 1": lambda: _scene(20001, 1.0),
+    "sparse, 4": lambda: _scene(70001, 4.0),
+    "sparse, 6": lambda: _scene(33001, 6.0),
     "the last size": lambda: _scene(127000, 16.0),
     "the first size of the masks": lambda: _scene(127001, 16.0),
     "eight cells": lambda: _clump(3001, 2),
